@@ -189,8 +189,8 @@ class Matrix:
     # kernel, merge-path, column panels (each panel on the library's choice,
     # or on a named layout: "panels_wg", "panels_wave", "panels_merge");
     # "col32" / "wg_col32": the library's choice / workgroup tiles with int32
-    # column indices kept in the SpMV (without it, banded matrices are read
-    # with int16 offsets)
+    # column indices kept in the SpMV (without it, stencils are read as row
+    # patterns and other banded matrices with int16 offsets)
     LAYOUTS = {"auto": 0, "col32": _abi.KS_MAT_COL32, "stream": _abi.KS_MAT_WG_TILES, "wg": _abi.KS_MAT_WG_TILES,
                "wg_col32": _abi.KS_MAT_WG_TILES | _abi.KS_MAT_COL32, "delta": _abi.KS_MAT_COL_DELTA,
                "wg_delta": _abi.KS_MAT_WG_TILES | _abi.KS_MAT_COL_DELTA,
@@ -233,10 +233,16 @@ class Matrix:
         return dict(n=n.value, nnz=nnz.value, spmv_kind=kind.value, lanes_per_row=lanes.value)
 
     def index_bytes(self, trans=False, precision=64):
-        """Bytes per column index that this matrix's SpMV reads (2: int16
-        offsets col - row, 4: int32 columns)."""
+        """Bytes per column index in this matrix's entry format (2: int16
+        offsets col - row or delta codes, 4: int32 columns)."""
         b = C.c_int32()
         self.ctx.check(self.ctx.lib.ks_mat_index_bytes(self.h, int(trans), precision, C.byref(b)), "index_bytes")
+        return b.value
+
+    def spmv_bytes(self, trans=False, precision=64):
+        """HBM bytes of one SpMV in the format its kernel reads."""
+        b = C.c_double()
+        self.ctx.check(self.ctx.lib.ks_mat_spmv_bytes(self.h, int(trans), precision, C.byref(b)), "spmv_bytes")
         return b.value
 
     def update_values(self, val):

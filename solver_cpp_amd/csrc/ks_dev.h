@@ -169,6 +169,8 @@ struct TileSet {
   // tile averages over 8 entries per row across more than 128 rows, none is
   // one long row), the condition of its delta-coded column format
   bool lane1 = false;
+  // workgroup tiles: some tile is one row longer than a tile
+  bool long_rows = false;
 };
 
 // SpMV plan of one CSR matrix: CSR-stream tiles (kind 0), L lanes per row
@@ -196,6 +198,10 @@ struct MatView {
   // column index that the SpMV reads
   const int16_t* col16 = nullptr;
   const uint16_t* cold = nullptr;
+  // row patterns (PatIx): one code per row and the pattern table, read
+  // instead of column indices and row pointers
+  const PatIx* pat = nullptr;
+  const int32_t* ptab = nullptr;
   int ib = 4;
   const T* val = nullptr;
   int kind = 0;
@@ -220,6 +226,12 @@ struct MatView {
     tnz = ts.tnz.p;
     carry = reinterpret_cast<T*>(pl.carry.p);
   }
+};
+
+// Row patterns (PatIx) of one side: the pattern table at p, the row codes
+// behind it (null: the side has none).
+struct PatBuf : DBuf<int32_t> {
+  const PatIx* code = nullptr;
 };
 
 // Column panels of one CSR matrix (A or A^T).  On matrices whose rows gather
@@ -252,6 +264,7 @@ struct ks_mat {
   ks::DBuf<int32_t> ptr, col;
   ks::DBuf<int16_t> col16, tcol16;  // col - row of A and A^T (banded matrices)
   ks::DBuf<uint16_t> cold, tcold;   // delta-coded columns of A and A^T
+  ks::PatBuf pat, tpat;             // row patterns of A and A^T
   ks::DBuf<double> val;
   ks::DBuf<float> val32;
   bool has_t = false;
@@ -264,13 +277,15 @@ struct ks_mat {
 
   template <class T>
   ks::MatView<T> view(bool trans) const;
-  // hands the int16 offsets to a view whose SpMV reads them
+  // hands the 16-bit indices to a view whose SpMV reads them
   template <class T>
   void set_col16(ks::MatView<T>& v, bool trans) const {
     if (v.kind != 0 || !v.wg_tiles) return;
     const int16_t* p = trans ? tcol16.p : col16.p;
     const uint16_t* q = trans ? tcold.p : cold.p;
-    if (p) { v.col16 = p; v.ib = 2; }
+    const ks::PatBuf& r = trans ? tpat : pat;
+    if (r.code) { v.pat = r.code; v.ptab = r.p; v.ib = 2; }
+    else if (p) { v.col16 = p; v.ib = 2; }
     else if (q) { v.cold = q; v.ib = 2; }
   }
 };
@@ -399,6 +414,13 @@ template <class T>
 inline double spmv_bytes(int64_t n, int64_t nnz, int ib = 4) {
   return (double)(sizeof(T) + ib) * nnz + 4.0 * (n + 1) + 2.0 * sizeof(T) * n;
 }
+// the same in a view's index format (row patterns: a 2-byte code per row
+// instead of column indices and row pointers)
+template <class T>
+inline double spmv_bytes(const MatView<T>& A) {
+  if (A.pat) return (double)sizeof(T) * A.nnz + 2.0 * A.n + 2.0 * sizeof(T) * A.n;
+  return spmv_bytes<T>(A.n, A.nnz, A.ib);
+}
 
 template <class T, int L, int NV, class Epi>
 int spmv_L(ks_ctx* c, const MatView<T>& A, const T* x, const Epi& epi, Gate g, int cls, double bytes) {
@@ -410,15 +432,19 @@ int spmv_L(ks_ctx* c, const MatView<T>& A, const T* x, const Epi& epi, Gate g, i
 }
 
 // The workgroup CSR-stream SpMV in the view's column index format, on G
-// workgroups.  G is always the int32 kernel's grid (grid_rows of that
-// instantiation): the grid, and so the reduction partials and their
-// summation order, is the same in every index format, so a solve's results
-// do not depend on the format (the 16-bit kernels, which need fewer
+// workgroups.  With reductions (NV > 0 or a projection) G is always the int32
+// kernel's grid (stream_grid): the grid, and so the reduction partials and
+// their summation order, is the same in every index format, so a solve's
+// results do not depend on the format (the 16-bit kernels, which need fewer
 // registers, may have room for more workgroups than they are given).
+// Without reductions each format fills its own residency.
 template <class T, int NX, int NV, class Epi>
 void launch_stream(ks_ctx* c, int cls, const MatView<T>& A, int G, const T* x0, const T* x1, const Epi& epi, Gate g,
                    double bytes) {
-  if (A.col16)
+  if (A.pat)
+    klaunch(c, cls, k_spmv_stream<T, NX, NV, Epi, PatIx>, G, 0, A.n, A.ntiles, A.tiles, A.tnz, A.ptab, A.pat, A.val,
+            x0, x1, epi, g, red(c), stat(c, cls, bytes));
+  else if (A.col16)
     klaunch(c, cls, k_spmv_stream<T, NX, NV, Epi, int16_t>, G, 0, A.n, A.ntiles, A.tiles, A.tnz, A.ptr, A.col16,
             A.val, x0, x1, epi, g, red(c), stat(c, cls, bytes));
   else if (A.cold)
@@ -430,11 +456,21 @@ void launch_stream(ks_ctx* c, int cls, const MatView<T>& A, int G, const T* x0, 
 }
 
 template <class T, int NX, int NV, class Epi>
+int stream_grid(ks_ctx* c, const MatView<T>& A) {
+  if constexpr (NV == 0 && !HasProj<Epi>::value) {
+    if (A.pat) return grid_rows(c, k_spmv_stream<T, NX, NV, Epi, PatIx>, A.ntiles);
+    if (A.col16) return grid_rows(c, k_spmv_stream<T, NX, NV, Epi, int16_t>, A.ntiles);
+    if (A.cold) return grid_rows(c, k_spmv_stream<T, NX, NV, Epi, uint16_t>, A.ntiles);
+  }
+  return grid_rows(c, k_spmv_stream<T, NX, NV, Epi>, A.ntiles);
+}
+
+template <class T, int NX, int NV, class Epi>
 int spmv_stream(ks_ctx* c, const MatView<T>& A, const T* x0, const T* x1, const Epi& epi, Gate g, int cls,
                 double bytes) {
   int G;
   if (A.wg_tiles) {
-    G = grid_rows(c, k_spmv_stream<T, NX, NV, Epi>, A.ntiles);
+    G = stream_grid<T, NX, NV, Epi>(c, A);
     launch_stream<T, NX, NV, Epi>(c, cls, A, G, x0, x1, epi, g, bytes);
   } else {
     G = grid_rows(c, k_spmv_wave<T, NX, NV, Epi>, (A.ntiles + kBlock / 64 - 1) / (kBlock / 64));
@@ -488,7 +524,8 @@ struct EpiPanelAcc {
   T* acc;
   int first;
   __device__ void prep() {}
-  __device__ void row(int64_t i, T s, T, double*) { acc[i] = first ? s : acc[i] + s; }
+  __device__ T pre(int64_t i) const { return first ? T(0) : acc[i]; }
+  __device__ void row(int64_t i, T s, T, double*, T a) { acc[i] = first ? s : a + s; }
   __device__ void fin(const double*) const {}
 };
 template <class T, class Epi>
@@ -496,7 +533,12 @@ struct EpiPanelLast {
   Epi e;
   const T* acc;
   __device__ void prep() { e.prep(); }
-  __device__ void row(int64_t i, T s, T s1, double* a) { e.row(i, acc[i] + s, s1, a); }
+  struct Pre {
+    T a;
+    decltype(std::declval<const Epi&>().pre(0)) p;
+  };
+  __device__ Pre pre(int64_t i) const { return Pre{acc[i], e.pre(i)}; }
+  __device__ void row(int64_t i, T s, T s1, double* a, Pre q) { e.row(i, q.a + s, s1, a, q.p); }
   __device__ void fin(const double* s) const { e.fin(s); }
 };
 
@@ -507,7 +549,7 @@ template <class T, int NV, class Epi>
 int launch_spmv(ks_ctx* c, const MatView<T>& A, const T* x, const Epi& epi, Gate g, double extra_bytes = 0,
                 bool finish = true) {
   const int cls = sizeof(T) == 8 ? KS_K_SPMV64 : KS_K_SPMV32;
-  const double bytes = spmv_bytes<T>(A.n, A.nnz, A.ib) + extra_bytes;
+  const double bytes = spmv_bytes<T>(A) + extra_bytes;
   int G;
   if (A.np > 0) {
     // the bytes of the whole SpMV are counted with the last pass
@@ -536,7 +578,7 @@ void launch_spmv2(ks_ctx* c, const MatView<T>& A, const T* x1, const T* x2, T* y
     launch_spmv<T, 0>(c, A, x2, EpiStore<T>{y2}, g);
     return;
   }
-  const double bytes = spmv_bytes<T>(A.n, A.nnz, A.ib) + 2.0 * sizeof(T) * A.n;
+  const double bytes = spmv_bytes<T>(A) + 2.0 * sizeof(T) * A.n;
   if (A.kind == 2) spmv_merge<T, 2, 0>(c, A, x1, x2, EpiStore2<T>{y1, y2}, g, KS_K_BASIS, bytes);
   else spmv_stream<T, 2, 0>(c, A, x1, x2, EpiStore2<T>{y1, y2}, g, KS_K_BASIS, bytes);
 }
@@ -598,8 +640,10 @@ inline void tile_set(ks_ctx* c, TileSet& ts, const int32_t* hp, int64_t n, int64
   // unless 2 nr <= kBlock and 8 nr < cnt; a tile over kTileNnz entries is
   // one long row
   ts.lane1 = true;
-  for (size_t i = 0; i + 1 < t.size() && ts.lane1; ++i) {
+  ts.long_rows = false;
+  for (size_t i = 0; i + 1 < t.size(); ++i) {
     const int64_t nr = t[i + 1] - t[i], cnt = (int64_t)z[i + 1] - z[i];
+    if (cnt > nnz_max) ts.long_rows = true;
     if (cnt > kTileNnz || (2 * nr <= kBlock && 8 * nr < cnt)) ts.lane1 = false;
   }
   upload_tiles(c, ts, t, z);
@@ -637,7 +681,8 @@ template <class T>
 struct EpiStore {
   T* y;
   __device__ void prep() {}
-  __device__ void row(int64_t i, T s, T, double*) { y[i] = s; }
+  __device__ NoPre pre(int64_t) const { return {}; }
+  __device__ void row(int64_t i, T s, T, double*, NoPre) { y[i] = s; }
   __device__ void fin(const double*) const {}
 };
 // y = A x streamed out with non-temporal stores: the standalone SpMV, whose
@@ -647,7 +692,8 @@ template <class T>
 struct EpiStream {
   T* y;
   __device__ void prep() {}
-  __device__ void row(int64_t i, T s, T, double*) { __builtin_nontemporal_store(s, y + i); }
+  __device__ NoPre pre(int64_t) const { return {}; }
+  __device__ void row(int64_t i, T s, T, double*, NoPre) { __builtin_nontemporal_store(s, y + i); }
   __device__ void fin(const double*) const {}
 };
 // y = (A x) * r (r: device FP64 reciprocal of the basis norm, formed by the
@@ -670,7 +716,8 @@ struct EpiDiv {
     }
   }
   __device__ T value(T s) const { return s * inv; }
-  __device__ void row(int64_t i, T s, T, double*) { y[i] = value(s); }
+  __device__ NoPre pre(int64_t) const { return {}; }
+  __device__ void row(int64_t i, T s, T, double*, NoPre) { y[i] = value(s); }
   __device__ void fin(const double*) const {}
 };
 // sqrt of the sum of the ng <= kMaxGrid partials p[] (a norm whose update
@@ -718,7 +765,8 @@ template <class T>
 struct EpiStore2 {
   T *y0, *y1;
   __device__ void prep() {}
-  __device__ void row(int64_t i, T s0, T s1, double*) { y0[i] = s0; y1[i] = s1; }
+  __device__ NoPre pre(int64_t) const { return {}; }
+  __device__ void row(int64_t i, T s0, T s1, double*, NoPre) { y0[i] = s0; y1[i] = s1; }
   __device__ void fin(const double*) const {}
 };
 
@@ -729,10 +777,11 @@ struct EpiResid {
   T* y;
   Fin f;
   __device__ void prep() {}
-  __device__ void row(int64_t i, T s, T, double* acc) {
-    const T r = (T)(b[i] - (double)s);
+  __device__ double pre(int64_t i) const { return b[i]; }
+  __device__ void row(int64_t i, T s, T, double* acc, double bi) {
+    const T r = (T)(bi - (double)s);
     y[i] = r;
-    acc[0] += (double)r * (double)r;
+    acc[0] = fma((double)r, (double)r, acc[0]);
   }
   __device__ void fin(const double* s) const { f(s); }
 };
@@ -744,9 +793,12 @@ struct EpiDot {
   T* y;
   Fin f;
   __device__ void prep() {}
-  __device__ void row(int64_t i, T s, T, double* acc) {
+  __device__ T pre(int64_t i) const { return d[i]; }
+  __device__ void row(int64_t i, T s, T, double* acc, T di) {
     y[i] = s;
-    acc[0] += (double)d[i] * (double)s;
+    // one rounding in every kernel: left to the compiler, the product and the
+    // sum are fused in some instantiations only
+    acc[0] = fma((double)di, (double)s, acc[0]);
   }
   __device__ void fin(const double* s) const { f(s); }
 };

@@ -223,7 +223,7 @@ void build_col16(ks_mat* m, DBuf<int16_t>& out, const int32_t* ptr, const int32_
 // every row encodes (sorted, first column and gaps in range: checked on the
 // device, as A^T's columns exist only there).  Returns false, with `out`
 // empty, otherwise.
-bool build_col_delta(ks_mat* m, const Plan& pl, DBuf<uint16_t>& out, const int32_t* ptr, const int32_t* col) {
+bool build_col_delta(const ks_mat* m, const Plan& pl, DBuf<uint16_t>& out, const int32_t* ptr, const int32_t* col) {
   if (pl.kind != 0 || !(pl.wg64 || pl.wg32) || !pl.wg.lane1) return false;
   ks_ctx* c = m->ctx;
   out.alloc(m->nnz);
@@ -238,20 +238,67 @@ bool build_col_delta(ks_mat* m, const Plan& pl, DBuf<uint16_t>& out, const int32
   return !hb;
 }
 
-// The SpMV's 16-bit column indices of A and A^T: int16 offsets when every
-// offset fits (off16), delta-coded columns where they apply, in the order
-// KS_MAT_COL_DELTA asks for; int32 columns otherwise, and for a side whose
-// SpMV runs on column panels (which read int32 columns).
-void build_index16(ks_mat* m, bool off16) {
+// Row patterns (PatIx) of the CSR (ptr, col) with plan pl: when its SpMV runs
+// on workgroup tiles, none of them one long row, and its rows have at most
+// kPatMax patterns whose table fits kPatTab.  `pat` holds the table, the
+// codes and (while they are built) the state in one allocation.  Returns
+// false, with nothing kept, otherwise.
+bool build_patterns(ks_mat* m, const Plan& pl, PatBuf& pat, const int32_t* ptr, const int32_t* col) {
+  if (pl.kind != 0 || !(pl.wg64 || pl.wg32) || pl.wg.long_rows) return false;
+  ks_ctx* c = m->ctx;
+  hipStream_t s = c->stream;
+  constexpr int64_t head = kPatTab + pad64(sizeof(PatState) / 4 + 1);
+  pat.alloc(head + (m->n + 1) / 2);
+  PatState* st = reinterpret_cast<PatState*>(pat.p + kPatTab);
+  k_fill<int32_t><<<1, kBlock, 0, s>>>(head, pat.p, 0);
+  k_pat_find<<<grid_map(m->n), kBlock, 0, s>>>(m->n, ptr, col, st);
+  k_pat_table<<<1, kPatSlots, 0, s>>>(st, ptr, col, pat.p);
+  k_pat_codes<<<(unsigned)pl.wg.ntiles, kBlock, 0, s>>>(st, pat.p, pl.wg.tiles.p, pl.wg.tnz.p, ptr, col,
+                                                        reinterpret_cast<PatIx*>(pat.p + head));
+  KS_HIPCK(hipGetLastError());
+  int bad = 0;
+  KS_HIPCK(hipMemcpyAsync(&bad, &st->bad, sizeof(int), hipMemcpyDeviceToHost, s));
+  KS_HIPCK(hipStreamSynchronize(s));
+  if (bad) pat.release();
+  else pat.code = reinterpret_cast<PatIx*>(pat.p + head);
+  return !bad;
+}
+
+// The SpMV's 16-bit column indices of A and A^T, unless KS_MAT_COL32: row
+// patterns where they apply (not with KS_MAT_COL_DELTA), else int16 offsets
+// when every offset fits (hp, hc: A's host row pointers and columns; A^T's
+// offsets are A's negated, so both fit), delta-coded columns where those
+// apply, in the order KS_MAT_COL_DELTA asks for; int32 columns otherwise, and
+// for a side whose SpMV runs on column panels (which read int32 columns).
+void build_index16(ks_mat* m, const int32_t* hp, const int32_t* hc) {
   const bool delta_first = (m->flags & KS_MAT_COL_DELTA) != 0;
-  auto side = [&](DBuf<int16_t>& o16, DBuf<uint16_t>& od, const Plan& pl, const PanelSet& ps, const int32_t* ptr,
-                  const int32_t* col) {
+  int off16 = -1;  // not looked at yet
+  auto side = [&](PatBuf& op, DBuf<int16_t>& o16, DBuf<uint16_t>& od, const Plan& pl,
+                  const PanelSet& ps, const int32_t* ptr, const int32_t* col) {
     if (ps.np) return;
+    if (!delta_first && build_patterns(m, pl, op, ptr, col)) return;
+    if (off16 < 0) off16 = offsets_fit16(m->n, hp, hc);
     if (off16 && !delta_first) build_col16(m, o16, ptr, col);
     else if (!build_col_delta(m, pl, od, ptr, col) && off16) build_col16(m, o16, ptr, col);
   };
-  side(m->col16, m->cold, m->plan, m->panels, m->ptr.p, m->col.p);
-  if (m->has_t) side(m->tcol16, m->tcold, m->tplan, m->tpanels, m->tptr.p, m->tcol.p);
+  side(m->pat, m->col16, m->cold, m->plan, m->panels, m->ptr.p, m->col.p);
+  if (m->has_t) side(m->tpat, m->tcol16, m->tcold, m->tplan, m->tpanels, m->tptr.p, m->tcol.p);
+}
+
+// Bytes per column index of the entry format that a side with row patterns
+// would have without them: 2 where int16 offsets or delta codes apply.
+int entry_index_bytes(const ks_mat* m, bool trans) {
+  ks_ctx* c = m->ctx;
+  const int32_t *ptr = trans ? m->tptr.p : m->ptr.p, *col = trans ? m->tcol.p : m->col.p;
+  DBuf<int> bad(1);
+  k_fill<int><<<1, kBlock, 0, c->stream>>>(1, bad.p, 0);
+  k_col_reach<<<grid_map(m->n), kBlock, 0, c->stream>>>(m->n, ptr, col, bad.p);
+  KS_HIPCK(hipGetLastError());
+  int hb = 0;
+  KS_HIPCK(hipMemcpyAsync(&hb, bad.p, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+  KS_HIPCK(hipStreamSynchronize(c->stream));
+  DBuf<uint16_t> tmp;
+  return !hb || build_col_delta(m, trans ? m->tplan : m->plan, tmp, ptr, col) ? 2 : 4;
 }
 
 // Split the CSR (hp, hc: host row pointers and columns of A or A^T) into
@@ -889,13 +936,12 @@ ks_status ks_mat_create_csr(ks_ctx* c, int64_t n, int64_t nnz, const int32_t* pt
   m->max_row = mx;
   KS_CHECK(!((flags & KS_MAT_COL32) && (flags & KS_MAT_COL_DELTA)), KS_ERR_BAD_INPUT,
            "KS_MAT_COL32 and KS_MAT_COL_DELTA exclude each other");
-  const bool off16 = !(flags & KS_MAT_COL32) && nnz > 0 && offsets_fit16(n, hp.data(), hc.data());
   make_plan(c, m->plan, hp.data(), n, nnz, (flags & KS_MAT_VECTOR) != 0, tile_choice(flags),
               merge_choice(flags, n, nnz, mx));
   if (nnz > 0 && panel_choice(flags, n, hp.data(), hc.data()))
     build_panels(m.get(), m->panels, hp.data(), hc.data(), nullptr, flags);
   if (flags & KS_MAT_TRANSPOSE) build_transpose(m.get());
-  if (!(flags & KS_MAT_COL32) && nnz > 0) build_index16(m.get(), off16);
+  if (!(flags & KS_MAT_COL32) && nnz > 0) build_index16(m.get(), hp.data(), hc.data());
   if (flags & KS_MAT_FP32_COPY) ensure_fp32(m.get());
   KS_HIPCK(hipStreamSynchronize(c->stream));
   *out = m.release();
@@ -971,7 +1017,19 @@ ks_status ks_mat_info(const ks_mat* m, int64_t* n, int64_t* nnz, int32_t* kind, 
 ks_status ks_mat_index_bytes(const ks_mat* m, int32_t trans, int32_t precision, int32_t* bytes) {
   if (!m || !bytes || (precision != KS_F64 && precision != KS_F32)) return KS_ERR_BAD_INPUT;
   if (trans && !m->has_t) return KS_ERR_BAD_INPUT;
-  *bytes = precision == KS_F64 ? m->view<double>(trans != 0).ib : m->view<float>(trans != 0).ib;
+  ks_ctx* c = m->ctx;
+  KS_API_TRY
+  set_device(c);
+  const auto v = m->view<double>(trans != 0);
+  *bytes = !v.pat ? (precision == KS_F64 ? v.ib : m->view<float>(trans != 0).ib) : entry_index_bytes(m, trans != 0);
+  return KS_OK;
+  KS_API_CATCH(c)
+}
+
+ks_status ks_mat_spmv_bytes(const ks_mat* m, int32_t trans, int32_t precision, double* bytes) {
+  if (!m || !bytes || (precision != KS_F64 && precision != KS_F32)) return KS_ERR_BAD_INPUT;
+  if (trans && !m->has_t) return KS_ERR_BAD_INPUT;
+  *bytes = precision == KS_F64 ? spmv_bytes(m->view<double>(trans != 0)) : spmv_bytes(m->view<float>(trans != 0));
   return KS_OK;
 }
 

@@ -260,7 +260,10 @@ struct RowBlocks {
 };
 
 // y = A x with L lanes per row (L | 64), RPB = kBlock/L rows per row block.
-// Epi: NV reduction values, prep(), row(row, sum, acc), fin(sums).
+// Epi: NV reduction values, prep(), pre(row) (what row() reads from memory,
+// so that a kernel can load it early; NoPre when nothing), row(row, sum,
+// second sum, acc, pre), fin(sums).
+struct NoPre {};
 template <class T, int L, int NV, class Epi>
 __global__ __launch_bounds__(kBlock) void k_spmv(int64_t n, const int32_t* __restrict__ ptr,
                                                  const int32_t* __restrict__ col,
@@ -292,7 +295,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv(int64_t n, const int32_t* __res
     for (int j = s + lane; j < e; j += L) sum += val[j] * x[col[j]];
 #pragma unroll
     for (int off = L / 2; off > 0; off >>= 1) sum += __shfl_xor(sum, off, L);
-    if (lane == 0 && row < n) epi.row(row, sum, (T)0, acc);
+    if (lane == 0 && row < n) epi.row(row, sum, (T)0, acc, epi.pre(row));
   }
   if constexpr (NV > 0) block_store<NV>(acc, ra);
 }
@@ -361,14 +364,23 @@ struct TileArr {
   U x[kN][W];
   // kFull: the whole window [a0, a0 + WIN) lies below nnz (uniform across
   // the tile), so no lane needs the entry-by-entry path; keeping that path
-  // out of the common case keeps the chunk loads back to back.
+  // out of the common case keeps the chunk loads back to back.  full(a0, nnz)
+  // is that condition.
   template <bool kFull>
   __device__ __forceinline__ void load(const U* __restrict__ p, int32_t a0, int32_t j1, int32_t nnz, int t) {
 #pragma unroll
     for (int i = 0; i < kN; ++i) {
       const int32_t e = a0 + W * t + W * NTH * i;
-      if (e < j1) {
-        if (kFull || e + W - 1 < nnz) {
+      if constexpr (kFull) {
+        // every lane loads, those past the tile its first chunk again (one
+        // more cache line): no branch, so the number of loads in flight is
+        // known and earlier ones can be waited for without these
+        const typename Chunk<U, W>::type q =
+            ld_stream(reinterpret_cast<const typename Chunk<U, W>::type*>(p + (e < j1 ? e : a0)));
+#pragma unroll
+        for (int h = 0; h < W; ++h) x[i][h] = q[h];
+      } else if (e < j1) {
+        if (e + W - 1 < nnz) {
           const typename Chunk<U, W>::type q = ld_stream(reinterpret_cast<const typename Chunk<U, W>::type*>(p + e));
 #pragma unroll
           for (int h = 0; h < W; ++h) x[i][h] = q[h];
@@ -410,19 +422,23 @@ struct QuadTile {
   TileArr<T, NTH, WIN, W> v;
   TileArr<IX, NTH, WIN, WC> c;
   int32_t pr;
+  __device__ static __forceinline__ bool full(int32_t j0, int32_t nnz) { return a0of(j0) + WIN <= nnz; }
+  // kFull: full(j0, nnz) holds; a row longer than a tile is loaded in place
+  template <bool kFull>
   __device__ __forceinline__ void load(const int32_t* __restrict__ ptr, const IX* __restrict__ col,
                                        const T* __restrict__ val, int32_t r0, int32_t r1, int32_t j0, int32_t j1,
                                        int32_t nnz, int t) {
-    if (j1 - j0 > WIN - kA + 1) return;  // long row: loaded in place
     const int32_t a0 = a0of(j0);
-    if (a0 + WIN <= nnz) {
-      v.template load<true>(val, a0, j1, nnz, t);
-      c.template load<true>(col, a0, j1, nnz, t);
-    } else {
-      v.template load<false>(val, a0, j1, nnz, t);
-      c.template load<false>(col, a0, j1, nnz, t);
-    }
-    pr = t < r1 - r0 ? ptr[r0 + t] : 0;
+    v.template load<kFull>(val, a0, j1, nnz, t);
+    c.template load<kFull>(col, a0, j1, nnz, t);
+    pr = ptr[t < r1 - r0 ? r0 + t : r1];
+  }
+  __device__ __forceinline__ void load(const int32_t* __restrict__ ptr, const IX* __restrict__ col,
+                                       const T* __restrict__ val, int32_t r0, int32_t r1, int32_t j0, int32_t j1,
+                                       int32_t nnz, int t) {
+    if (j1 - j0 > WIN - kA + 1) return;
+    if (full(j0, nnz)) load<true>(ptr, col, val, r0, r1, j0, j1, nnz, t);
+    else load<false>(ptr, col, val, r0, r1, j0, j1, nnz, t);
   }
   __device__ __forceinline__ void stage(T* sv, IX* sc, int32_t j0, int32_t j1, int t) const {
     const int32_t span = j1 - a0of(j0);
@@ -432,6 +448,67 @@ struct QuadTile {
 };
 template <class T, class IX = int32_t>
 using TileData = QuadTile<T, kBlock, kTileWin, IX>;
+
+// Lanes per row of a CSR-stream tile of nr rows and cnt entries: more than
+// one only for rows averaging over 8 entries.
+__device__ __forceinline__ int tile_lanes(int nr, int cnt) {
+  int tpr = 1;
+  while (tpr < 64 && tpr * 2 * nr <= kBlock && tpr * 8 * nr < cnt) tpr *= 2;
+  return tpr;
+}
+
+// Row-pattern column format (stencils and other matrices whose rows repeat
+// few lists of column offsets).  A pattern is one row's length and its
+// offsets col - row in CSR order; the matrix keeps a table of its at most
+// kPatMax patterns and one 16-bit code per row: the pattern's number above
+// the row's first entry's place in its tile's window (kPatShift bits).  The
+// SpMV then reads 2 bytes per row instead of 2 bytes per entry and a 4-byte
+// row pointer.  Table: [0] entries per pattern (the stride), [1 + p] the
+// length of pattern p, [1 + kPatMax + p * stride + k] its k-th offset.
+// The SpMV is bound by the bytes it streams (about 5.2 TB/s of values, codes,
+// x and y at every size from 128^3 to 192^3), so its time follows them: a
+// 7-point 160^3 product moves 302 MB in FP64 and 155 MB in FP32 instead of
+// 367 and 220 MB with int16 offsets, and takes 57 and 30 us instead of 75 and
+// 48.  32 patterns hold the 27 of a 7-point (or 27-point) box stencil and fit
+// a code beside the 11-bit place in the window.
+struct PatIx {
+  uint16_t v;
+};
+constexpr int kPatMax = 32;
+constexpr int kPatShift = 11;
+constexpr int kPatTab = 1024;  // table size limit (ints), staged in LDS
+static_assert(kTileWin <= 1 << kPatShift && kPatMax << kPatShift <= 1 << 16, "row codes fit 16 bits");
+
+// One thread's share of a tile in this format: values of the window, and the
+// code of the row it sums.
+template <class T>
+struct PatTile {
+  static constexpr int W = 16 / (int)sizeof(T);
+  __device__ static __forceinline__ int32_t a0of(int32_t j0) { return j0 & ~3; }
+  TileArr<T, kBlock, kTileWin, W> v;
+  int32_t pr;
+  __device__ static __forceinline__ bool full(int32_t j0, int32_t nnz) { return a0of(j0) + kTileWin <= nnz; }
+  template <bool kFull>
+  __device__ __forceinline__ void load(const int32_t*, const PatIx* __restrict__ code, const T* __restrict__ val,
+                                       int32_t r0, int32_t r1, int32_t j0, int32_t j1, int32_t nnz, int t) {
+    v.template load<kFull>(val, a0of(j0), j1, nnz, t);
+    const int grp = t / tile_lanes(r1 - r0, j1 - j0);
+    pr = (int32_t)code[grp < r1 - r0 ? r0 + grp : r0].v;
+  }
+  __device__ __forceinline__ void load(const int32_t* ptr, const PatIx* __restrict__ code, const T* __restrict__ val,
+                                       int32_t r0, int32_t r1, int32_t j0, int32_t j1, int32_t nnz, int t) {
+    if (full(j0, nnz)) load<true>(ptr, code, val, r0, r1, j0, j1, nnz, t);
+    else load<false>(ptr, code, val, r0, r1, j0, j1, nnz, t);
+  }
+};
+template <class T, class IX>
+struct TileOf {
+  using type = TileData<T, IX>;
+};
+template <class T>
+struct TileOf<T, PatIx> {
+  using type = PatTile<T>;
+};
 
 // Register budget of the CSR-stream kernels as waves/SIMD: FP32 64 VGPRs
 // (8 waves) for a plain SpMV and 72 (7 waves) with a fused reduction, FP64
@@ -461,9 +538,20 @@ struct HasProj<E, std::void_t<decltype(E::kProj)>> : std::true_type {};
 // kDeltaBias and every later one the gap to the previous column, decoded by
 // the one lane that sums the row (the host builds this format only when
 // every tile sums its rows one per lane and no row is a tile of its own).
+// IX = PatIx: one 16-bit code per row and a table of row patterns (above);
+// `ptr` is the table and `col` the codes.  The host builds it only when no
+// row is a tile of its own.
 // In every format the row sums are the same: entry for entry, the same x is
 // gathered in the same order.
 constexpr int32_t kDeltaBias = 49152;
+// x gathers of a row in flight before the next tile's loads: the rows of a
+// 7-point stencil whole, where the registers hold them without spilling (the
+// kernels with int32 or, in FP64, any per-entry indices keep fewer).
+template <class T, int NX, class IX>
+constexpr int kGathers = std::is_same<IX, PatIx>::value         ? 8
+                         : sizeof(IX) == 4 || (sizeof(T) == 8 && NX == 2) ? 4
+                         : sizeof(T) == 4                       ? 8
+                                                                : 6;
 template <class T, int NX, int NV, class Epi, class IX = int32_t>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kWgWaves<T, NX, NV>))) void k_spmv_stream(int64_t n, int64_t ntiles, const int32_t* __restrict__ tiles,
                                                         const int32_t* __restrict__ tnz,
@@ -476,6 +564,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kWgWaves
   st.count();
   constexpr bool kRel = std::is_same<IX, int16_t>::value;
   constexpr bool kDelta = std::is_same<IX, uint16_t>::value;
+  constexpr bool kPat = std::is_same<IX, PatIx>::value;
+  constexpr int kGB = kGathers<T, NX, IX>;
   // With the projection epilogue, the y of the workgroup's first kYT tiles
   // is kept in LDS (tile s at sy[s][row - (r0 & ~3)], 16-byte aligned row
   // chunks): the projection reads it there instead of from L2/HBM, and it
@@ -485,9 +575,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kWgWaves
   constexpr int kYT = !HasProj<Epi>::value ? 0 : sizeof(T) == 4 ? (sizeof(IX) == 2 ? 9 : 4) : (sizeof(IX) == 2 ? 4 : 2);
   constexpr int kYW = kTileRows + 4;
   __shared__ __align__(16) T sv[kTileWin];
-  __shared__ __align__(16) IX sc[kTileWin];
+  __shared__ __align__(16) IX sc[kPat ? 1 : kTileWin];
+  __shared__ int32_t stab[kPat ? kPatTab : 1];
   __shared__ __align__(16) T sy[kYT > 0 ? kYT : 1][kYT > 0 ? kYW : 1];
-  __shared__ int32_t sptr[kTileRows + 1];
+  __shared__ int32_t sptr[kPat ? 1 : kTileRows + 1];
   __shared__ double slong[NX][kBlock / 64];
   double acc[NV > 0 ? NV : 1];
 #pragma unroll
@@ -497,34 +588,42 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kWgWaves
   int64_t t, end, step;
   rbs.range(t, end, step);
   const int32_t nnz = tnz[ntiles];
-  int32_t r0 = 0, r1 = 0, j0 = 0, j1 = 0;
-  TileData<T, IX> d;
-  if (t < end) {
-    r0 = tiles[t]; r1 = tiles[t + 1]; j0 = tnz[t]; j1 = tnz[t + 1];
-    d.load(ptr, col, val, r0, r1, j0, j1, nnz, tid);
-  }
-  // meta of the next tile: loaded one tile ahead, after the data prefetch,
-  // so waiting for the prefetched columns never waits for these loads
-  int32_t nr0 = 0, nr1 = 0, nj0 = 0, nj1 = 0;
-  if (t + step < end) {
-    nr0 = tiles[t + step]; nr1 = tiles[t + step + 1]; nj0 = tnz[t + step]; nj1 = tnz[t + step + 1];
+  // bounds of the current tile and the next one: scalar loads, issued a tile
+  // before they are used
+  struct Bounds {
+    int32_t r0, r1, j0, j1;
+  };
+  auto bounds = [&](int64_t u) {
+    return u < end ? Bounds{tiles[u], tiles[u + 1], tnz[u], tnz[u + 1]} : Bounds{0, 0, 0, 0};
+  };
+  Bounds cur = bounds(t), nx = bounds(t + step);
+  typename TileOf<T, IX>::type d;
+  if (t < end) d.load(ptr, col, val, cur.r0, cur.r1, cur.j0, cur.j1, nnz, tid);
+  int pstride = 0;
+  if constexpr (kPat) {  // the pattern table (`ptr` in this format); ordered by the first tile's barrier
+    pstride = ptr[0];
+    const int m = 1 + kPatMax + kPatMax * pstride;  // the host allocates kPatTab entries
+    for (int i = tid; i < (m < kPatTab ? m : kPatTab); i += kBlock) stab[i] = ptr[i];
   }
   // the epilogue's scalars, with the first tile already in flight (an
   // epilogue may reduce partials across the workgroup here)
   epi.prep();
   int slot = 0;  // this tile's index among the workgroup's tiles
   for (; t < end; t += step, ++slot) {
+    const int32_t r0 = cur.r0, r1 = cur.r1, j0 = cur.j0, j1 = cur.j1;
+    const int32_t nr0 = nx.r0, nr1 = nx.r1, nj0 = nx.j0, nj1 = nx.j1;
     const int nr = r1 - r0, cnt = j1 - j0;
-    const int64_t tn = t + step, tnn = t + 2 * step;
-    const bool more = tn < end, more2 = tnn < end;
-    int32_t mr0 = 0, mr1 = 0, mj0 = 0, mj1 = 0;
-    if (cnt > kTileNnz) {
+    const bool more = t + step < end;
+    cur = nx;
+    if (!kPat && cnt > kTileNnz) {
       // one long row: strided partial sums, then a fixed tree
       T s0 = 0, s1 = 0;
       for (int k = tid; k < cnt; k += kBlock) {
         const T a = ld_stream(val + j0 + k);
         int c;
-        if constexpr (kDelta) {
+        if constexpr (kPat) {
+          c = 0;  // not reached
+        } else if constexpr (kDelta) {
           // not reached (no row is a tile of its own in this format); kept
           // correct: the column is the prefix sum of the row's codes
           c = r0 - kDeltaBias;
@@ -554,44 +653,85 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kWgWaves
         }
         if constexpr (kYT > 0) {
           if (slot < kYT) sy[slot][r0 & 3] = epi.value(a0);
-          else epi.row(r0, a0, a1, acc);
+          else epi.row(r0, a0, a1, acc, epi.pre(r0));
         } else {
-          epi.row(r0, a0, a1, acc);
+          epi.row(r0, a0, a1, acc, epi.pre(r0));
         }
       }
       if (more) d.load(ptr, col, val, nr0, nr1, nj0, nj1, nnz, tid);
-      if (more2) { mr0 = tiles[tnn]; mr1 = tiles[tnn + 1]; mj0 = tnz[tnn]; mj1 = tnz[tnn + 1]; }
+      nx = bounds(t + 2 * step);
       __syncthreads();
     } else {
-      if (tid < nr) sptr[tid] = d.pr - d.a0of(j0);
-      if (tid == 0) sptr[nr] = j1 - d.a0of(j0);
-      d.stage(sv, sc, j0, j1, tid);
-      __syncthreads();
-      // in flight during the sums: the next tile's data, then the meta after it
-      if (more) d.load(ptr, col, val, nr0, nr1, nj0, nj1, nnz, tid);
-      if (more2) { mr0 = tiles[tnn]; mr1 = tiles[tnn + 1]; mj0 = tnz[tnn]; mj1 = tnz[tnn + 1]; }
       // more than one thread per row only for rows averaging > 8 entries
       // (delta-coded columns: always one per row, which the host checked is
-      // the choice below for every tile)
-      int tpr = 1;
-      if constexpr (!kDelta)
-        while (tpr < 64 && tpr * 2 * nr <= kBlock && tpr * 8 * nr < cnt) tpr *= 2;
+      // the choice for every tile)
+      const int tpr = kDelta ? 1 : tile_lanes(nr, cnt);
       const int grp = tid / tpr, lane = tid % tpr;
-      if (grp < nr) {
-        const int s = sptr[grp], e = sptr[grp + 1];
-        const int cb = kRel ? r0 + grp : kDelta ? r0 + grp - kDeltaBias : 0;
-        int cd = cb;  // delta-coded: the running column
+      const bool act = grp < nr;
+      [[maybe_unused]] const int code = d.pr;  // kPat: this thread's row, taken before the next tile's load
+      if constexpr (kPat) {
+        d.v.stage(sv, j1 - d.a0of(j0), tid);
+      } else {
+        if (tid < nr) sptr[tid] = d.pr - d.a0of(j0);
+        if (tid == 0) sptr[nr] = j1 - d.a0of(j0);
+        d.stage(sv, sc, j0, j1, tid);
+      }
+      __syncthreads();
+      // the row's entries s .. e - 1 of the window (none without a row)
+      int s, e;
+      [[maybe_unused]] const int32_t* off = nullptr;  // kPat: the row's offsets, its first entry's at off[s]
+      if constexpr (kPat) {
+        const int p = code >> kPatShift;
+        s = code & ((1 << kPatShift) - 1);
+        e = act ? s + stab[1 + p] : s;
+        off = stab + (1 + kPatMax + p * pstride) - s;
+      } else {
+        s = sptr[act ? grp : nr];
+        e = sptr[act ? grp + 1 : nr];
+      }
+      const int64_t row = r0 + (act ? grp : 0);
+      const int cb = kRel || kPat ? (int)row : kDelta ? (int)row - kDeltaBias : 0;
+      int cd = cb;  // delta-coded: the running column
+      auto column = [&](int k) -> int {
+        if constexpr (kPat) return cb + off[k];
+        else if constexpr (kDelta) return cd += (int)sc[k];
+        else return cb + (int)sc[k];
+      };
+      // Vector memory answers loads in the order they were issued, so the x
+      // gathers of the row's first kGB entries and the epilogue's operand go
+      // out before the next tile's loads: the sums then wait for an L2 hit
+      // and not for HBM (160^3: FP32 34.9 -> 29.6 us with row patterns, int16
+      // offsets 47.8 -> 42.7 us in FP32 and 75.0 -> 69.4 us in FP64; a second
+      // tile in flight behind it gave nothing more).  Slots past the row's end
+      // gather x of its row.
+      auto sums = [&](auto next_tag) {
+        constexpr int kNext = decltype(next_tag)::value;  // next tile: 0 none, 1 its full window, 2 entry by entry
+        T g0[kGB], g1[kGB];
+#pragma unroll
+        for (int q = 0; q < kGB; ++q) {
+          const int k = s + lane + q * tpr;
+          const int c = k < e ? column(k) : (int)row;
+          g0[q] = x0[c];
+          if (NX == 2) g1[q] = x1[c];
+        }
+        const auto pv = epi.pre(row);
+        if constexpr (kNext == 1) d.template load<true>(ptr, col, val, nr0, nr1, nj0, nj1, nnz, tid);
+        if constexpr (kNext == 2) d.load(ptr, col, val, nr0, nr1, nj0, nj1, nnz, tid);
         T a0 = 0, a1 = 0;
-#pragma unroll 2
-        for (int k = s + lane; k < e; k += tpr) {
-          const T v = sv[k];
-          int c;
-          if constexpr (kDelta) {
-            cd += (int)sc[k];
-            c = cd;
-          } else {
-            c = cb + (int)sc[k];
+#pragma unroll
+        for (int q = 0; q < kGB; ++q) {
+          const int k = s + lane + q * tpr;
+          const T v = sv[k < e ? k : 0];
+          const T b0 = mul_add_rn(a0, v, g0[q]);
+          a0 = k < e ? b0 : a0;
+          if (NX == 2) {
+            const T b1 = mul_add_rn(a1, v, g1[q]);
+            a1 = k < e ? b1 : a1;
           }
+        }
+        for (int k = s + lane + kGB * tpr; k < e; k += tpr) {
+          const T v = sv[k];
+          const int c = column(k);
           a0 = mul_add_rn(a0, v, x0[c]);
           if (NX == 2) a1 = mul_add_rn(a1, v, x1[c]);
         }
@@ -599,19 +739,21 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kWgWaves
           a0 += __shfl_xor(a0, off, 64);
           if (NX == 2) a1 += __shfl_xor(a1, off, 64);
         }
-        if (lane == 0) {
+        if (act && lane == 0) {
           if constexpr (kYT > 0) {
             if (slot < kYT) sy[slot][(r0 & 3) + grp] = epi.value(a0);
-            else epi.row(r0 + grp, a0, a1, acc);
+            else epi.row(row, a0, a1, acc, pv);
           } else {
-            epi.row(r0 + grp, a0, a1, acc);
+            epi.row(row, a0, a1, acc, pv);
           }
         }
-      }
+      };
+      if (!more) sums(std::integral_constant<int, 0>{});
+      else if (nj1 - nj0 <= kTileNnz && d.full(nj0, nnz)) sums(std::integral_constant<int, 1>{});
+      else sums(std::integral_constant<int, 2>{});
+      nx = bounds(t + 2 * step);  // after the LDS reads, which share the scalar loads' counter
       __syncthreads();
     }
-    r0 = nr0; r1 = nr1; j0 = nj0; j1 = nj1;
-    nr0 = mr0; nr1 = mr1; nj0 = mj0; nj1 = mj1;
   }
   if constexpr (NV > 0) block_store<NV>(acc, ra);
   if constexpr (HasProj<Epi>::value) {
@@ -822,7 +964,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kStreamW
         s0 += __shfl_xor(s0, off, 64);
         if (NX == 2) s1 += __shfl_xor(s1, off, 64);
       }
-      if (lane == 0) epi.row(r0, s0, s1, acc);
+      if (lane == 0) epi.row(r0, s0, s1, acc, epi.pre(r0));
     } else {
       if (lane < nr) sptr[lane] = d.pr - (j0 & ~3);
       if (lane == 0) sptr[nr] = j1 - (j0 & ~3);
@@ -850,7 +992,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kStreamW
         a0 += __shfl_xor(a0, off, 64);
         if (NX == 2) a1 += __shfl_xor(a1, off, 64);
       }
-      if (grp < nr && sub == 0) epi.row(r0 + grp, a0, a1, acc);
+      if (grp < nr && sub == 0) epi.row(r0 + grp, a0, a1, acc, epi.pre(r0 + grp));
       wave_sync();
     }
     r0 = nr0; r1 = nr1; j0 = nj0; j1 = nj1;
@@ -1054,7 +1196,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kMergeWa
           head[s] = a0;
           if (NX == 2) head[nseg + s] = a1;
         } else {
-          epi.row(r0 + grp, a0, a1, acc);
+          epi.row(r0 + grp, a0, a1, acc, epi.pre(r0 + grp));
         }
       }
     }
@@ -1093,7 +1235,7 @@ __global__ __launch_bounds__(kBlock) void k_merge_fix(int64_t n, int64_t nseg, c
         c0 += carry[q];
         if (NX == 2) c1 += carry[nseg + q];
       }
-      epi.row(r0, c0 + head[s], NX == 2 ? c1 + head[nseg + s] : T(0), acc);
+      epi.row(r0, c0 + head[s], NX == 2 ? c1 + head[nseg + s] : T(0), acc, epi.pre(r0));
     }
   }
   if constexpr (NV > 0) block_store<NV>(acc, ra);
@@ -1732,6 +1874,16 @@ __global__ void k_col_offsets(int64_t n, const int32_t* __restrict__ ptr, const 
     for (int32_t j = ptr[r], e = ptr[r + 1]; j < e; ++j) out[j] = (int16_t)(col[j] - r);
 }
 
+// *bad is set when an entry lies over 32767 columns from its row.
+__global__ void k_col_reach(int64_t n, const int32_t* __restrict__ ptr, const int32_t* __restrict__ col, int* bad) {
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r < n; r += stride)
+    for (int32_t j = ptr[r], e = ptr[r + 1]; j < e; ++j) {
+      const int64_t d = (int64_t)col[j] - r;
+      if (d < -32767 || d > 32767) *bad = 1;
+    }
+}
+
 // Delta-coded columns (see k_spmv_stream): out[first] = col - r + kDeltaBias,
 // out[j] = col[j] - col[j - 1] after it; *bad is set when a row is not
 // sorted or a code does not fit 16 bits (the host then keeps int32 columns)
@@ -1747,6 +1899,97 @@ __global__ void k_col_delta(int64_t n, const int32_t* __restrict__ ptr, const in
       prev = col[j];
     }
   }
+}
+
+// Row patterns (PatIx), built by three kernels with no host step between
+// them.  k_pat_find enters every row's pattern hash in an open-addressing
+// table of kPatSlots slots (key 0: free; rep: a row with that key).
+// k_pat_table numbers the patterns by hash and writes the pattern table from
+// their rows.  k_pat_codes writes the row codes and compares every row with
+// its pattern entry by entry (two patterns of one hash).  Each sets `bad`
+// when the format does not apply, which ends the later ones.
+constexpr int kPatSlots = 2 * kPatMax;
+struct PatState {
+  unsigned long long key[kPatSlots];
+  int32_t rep[kPatSlots];
+  unsigned long long hash[kPatMax];  // by pattern number
+  int P, bad;
+};
+__device__ inline uint64_t pat_hash(const int32_t* __restrict__ col, int32_t a, int32_t e, int32_t r) {
+  uint64_t h = 0x9e3779b97f4a7c15ull + (uint64_t)(e - a);
+  for (int32_t j = a; j < e; ++j) {
+    h ^= (uint32_t)(col[j] - r);
+    h *= 0xff51afd7ed558ccdull;
+    h ^= h >> 32;
+  }
+  return h ? h : 1;
+}
+__global__ void k_pat_find(int64_t n, const int32_t* __restrict__ ptr, const int32_t* __restrict__ col, PatState* st) {
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r < n; r += stride) {
+    if (*(volatile int*)&st->bad) return;
+    const int32_t a = ptr[r], e = ptr[r + 1];
+    if (e - a > kPatTab - 1 - kPatMax) { st->bad = 1; return; }
+    const unsigned long long h = pat_hash(col, a, e, (int32_t)r);
+    int s = (int)(h % kPatSlots), tries = 0;
+    for (; tries < kPatSlots; ++tries, s = (s + 1) % kPatSlots) {
+      unsigned long long k = *(volatile unsigned long long*)(st->key + s);
+      if (k == 0) k = atomicCAS(st->key + s, 0ull, h);  // the key that was there
+      if (k == 0) st->rep[s] = (int32_t)r;              // this row entered it
+      if (k == 0 || k == h) break;
+    }
+    if (tries == kPatSlots) { st->bad = 1; return; }
+  }
+}
+// one workgroup of kPatSlots threads
+__global__ void k_pat_table(PatState* st, const int32_t* __restrict__ ptr, const int32_t* __restrict__ col,
+                            int32_t* tab) {
+  __shared__ int s_stride, s_P;
+  if (st->bad) return;
+  const int s = threadIdx.x;
+  if (s == 0) { s_stride = 1; s_P = 0; }
+  __syncthreads();
+  const unsigned long long k = st->key[s];
+  int32_t r = 0, a = 0, len = 0;
+  int p = 0;
+  if (k) {
+    r = st->rep[s];
+    a = ptr[r];
+    len = ptr[r + 1] - a;
+    for (int q = 0; q < kPatSlots; ++q) p += st->key[q] && st->key[q] < k;
+    atomicMax(&s_stride, len);
+    atomicAdd(&s_P, 1);
+  }
+  __syncthreads();
+  const int P = s_P, stride = s_stride;
+  if (P > kPatMax || 1 + kPatMax + P * stride > kPatTab) {
+    if (s == 0) st->bad = 1;
+    return;
+  }
+  if (s == 0) { tab[0] = stride; st->P = P; }
+  if (!k) return;
+  st->hash[p] = k;
+  tab[1 + p] = len;
+  for (int j = 0; j < len; ++j) tab[1 + kPatMax + p * stride + j] = col[a + j] - r;
+}
+// one workgroup per tile
+__global__ __launch_bounds__(kBlock) void k_pat_codes(PatState* st, const int32_t* __restrict__ tab,
+                                                      const int32_t* __restrict__ tiles,
+                                                      const int32_t* __restrict__ tnz,
+                                                      const int32_t* __restrict__ ptr,
+                                                      const int32_t* __restrict__ col, PatIx* code) {
+  if (*(volatile int*)&st->bad) return;
+  const int64_t t = blockIdx.x;
+  const int32_t r = tiles[t] + (int32_t)threadIdx.x, a0 = PatTile<double>::a0of(tnz[t]);
+  if (r >= tiles[t + 1]) return;
+  const int32_t a = ptr[r], e = ptr[r + 1], P = st->P;
+  const uint64_t h = pat_hash(col, a, e, r);
+  int p = 0;
+  while (p < P && st->hash[p] != h) ++p;
+  bool ok = p < P && tab[1 + p] == e - a;
+  for (int32_t j = a; ok && j < e; ++j) ok = tab[1 + kPatMax + p * tab[0] + (j - a)] == col[j] - r;
+  if (!ok) { st->bad = 1; return; }
+  code[r].v = (uint16_t)(p << kPatShift | (a - a0));
 }
 
 // out[0..m) = v: clears memory with a kernel (no memset node), for state

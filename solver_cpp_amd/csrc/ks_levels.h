@@ -911,14 +911,13 @@ void launch_spmv_proj(ks_ctx* c, const MatView<T>& A, const T* vk, T* w, const d
                       int nv, double* hcol, int ldh, Gate g, const double* vn, PendNorm pn = PendNorm{}) {
   if (spmv_proj_fused(A, V, ldv, nv, (const T*)w)) {
     const int cls = sizeof(T) == 8 ? KS_K_SPMV64 : KS_K_SPMV32;
-    const double bytes = spmv_bytes<T>(A.n, A.nnz, A.ib) + (double)sizeof(T) * A.n * nv;
+    const double bytes = spmv_bytes<T>(A) + (double)sizeof(T) * A.n * nv;
     EpiDivProj<T> e{};
     e.y = w; e.r = r; e.V = V; e.ldv = ldv; e.nv = nv;
     if (pn.pk >= 0) {
       e.np = c->part2.p; e.ng = pn.ng;
     }
-    // the int32 kernel's grid in every index format (see launch_stream)
-    const int G = grid_rows(c, k_spmv_stream<T, 1, 0, EpiDivProj<T>>, A.ntiles);
+    const int G = stream_grid<T, 1, 0, EpiDivProj<T>>(c, A);
     launch_stream<T, 1, 0, EpiDivProj<T>>(c, cls, A, G, vk, vk, e, g, bytes);
     if (pn.pk >= 0) launch_proj_finish(c, G, nv, FinNormProj{FinProj{hcol, ldh, nv, vn}, pn.c, pn.pk,
                                                              c->part2.p, pn.ng, 0.0}, g);
