@@ -168,6 +168,13 @@ const char* ks_status_string(int32_t status);
 ks_status ks_ctx_create(int32_t device, ks_ctx** out);
 void ks_ctx_destroy(ks_ctx* ctx);
 const char* ks_ctx_last_error(const ks_ctx* ctx);
+/* Solves of small systems run many iterations in one launch whose workgroups
+ * wait for each other (on-chip solves).  `polls` bounds each such wait
+ * (default 2^21, about a second); when one runs out, for instance because
+ * another process holds the GPU, the solve is repeated with one launch per
+ * operation.  0 makes every such solve take that way.  No reference
+ * counterpart. */
+ks_status ks_ctx_set_wait_limit(ks_ctx* ctx, int32_t polls);
 /* hipStream_t the context launches on (as void*), for callers that order
  * their own work against it. */
 void* ks_ctx_stream(ks_ctx* ctx);

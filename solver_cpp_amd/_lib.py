@@ -26,6 +26,7 @@ _SIGS = {
     "ks_ctx_create": (_i32, [_i32, _pp]),
     "ks_ctx_destroy": (None, [_vp]),
     "ks_ctx_last_error": (C.c_char_p, [_vp]),
+    "ks_ctx_set_wait_limit": (_i32, [_vp, _i32]),
     "ks_ctx_stream": (_vp, [_vp]),
     "ks_ctx_synchronize": (_i32, [_vp]),
     "ks_mat_create_csr": (_i32, [_vp, _i64, _i64, _vp, _vp, _vp, _u32, _pp]),

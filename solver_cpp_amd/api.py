@@ -99,6 +99,10 @@ class Context:
     def stream(self):
         return self.lib.ks_ctx_stream(self.h)
 
+    def set_wait_limit(self, polls):
+        """Bound on one wait inside an on-chip solve (ks_ctx_set_wait_limit)."""
+        self.check(self.lib.ks_ctx_set_wait_limit(self.h, int(polls)), "set_wait_limit")
+
     def synchronize(self):
         self.check(self.lib.ks_ctx_synchronize(self.h), "synchronize")
 

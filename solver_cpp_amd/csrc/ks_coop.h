@@ -1,0 +1,371 @@
+// ks_coop.h - Krylov iterations of a system that fits on chip, many to a launch.
+//
+// A CG step of a 256 x 256 grid moves 9 MB, a microsecond's worth, but as
+// three dependent launches it takes 14 us: each launch costs 4 to 5 us
+// whatever it does.  Here one launch runs up to kCoopIters steps.  The
+// workgroups (one per CU at most, so all are resident together) own
+// contiguous rows, one or two per thread, whose matrix entries and vector
+// elements stay in registers between the steps.  Two things cross workgroups:
+//  * vectors that other rows' products gather: written with agent-scope
+//    stores, which go through to memory, and gathered with agent-scope loads
+//    (a workgroup's own part from LDS);
+//  * reductions (Team::all_sum): every workgroup stores its sums, tagged with
+//    the number of the reduction, and polls all the others'.  One store and
+//    one load's latency, about 1.1 us for 64 workgroups, against 8 us and
+//    more for a barrier with agent-scope fences (which write back and
+//    invalidate the L2).  It is also the barrier between the steps: a
+//    workgroup's vector stores are complete before its sums are stored.
+// Sums form in a fixed order, the same in every workgroup, so solves are
+// bit-identical run to run and control flow is uniform without a broadcast.
+//
+// Every wait is bounded (CoopArgs::spin polls).  A wait that runs out (the
+// workgroups were not resident together, for instance beside another process)
+// sets *fail and ends the launch; later launches return at once and the host
+// repeats the solve with one launch per operation.
+#pragma once
+#include "ks_kernels.h"
+
+namespace ks {
+
+// Threads of a workgroup and the most rows per thread: 512 threads were the
+// fastest at most sizes (CG, 256 x 256 / 512 x 512 / 700 x 700: 6.4 / 8.6 /
+// 13.2 us a step; 256 threads 6.7 / 9.8 / 41, 1024 threads 6.6 / 8.3 / 15.0),
+// and leave the 256 registers that four rows take.
+constexpr int kCoopThreads = 512;
+constexpr int kCoopRpt = 4;
+constexpr int kCoopMaxWg = 256;
+constexpr int kCoopRow = 8;       // entries of a row held in registers
+constexpr int kCoopVals = 64;     // values of one reduction
+constexpr int kCoopIters = 1024;  // steps per launch
+constexpr int kCoopSpin = 1 << 21;
+constexpr int64_t kCoopSlots = 2 * 2 * (int64_t)kCoopVals * kCoopMaxWg;
+
+struct CoopArgs {
+  unsigned long long* slots;  // kCoopSlots words: [parity][value][workgroup][2]
+  unsigned* state;            // [0] tag of the last reduction, [1] fail
+  int spin;
+};
+
+template <class T>
+__device__ __forceinline__ T shared_load(const T* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <class T>
+__device__ __forceinline__ void shared_store(T* p, T v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// One workgroup's sum in a slot of 16 bytes: both halves carry the tag, so a
+// reader that sees the tag in both has the whole value.
+typedef unsigned slot_t __attribute__((ext_vector_type(4)));
+constexpr int kSlotScope = 16;  // buffer instructions' sc1 bit: agent scope
+struct Slots {
+  __amdgpu_buffer_rsrc_t r;
+  __device__ explicit Slots(unsigned long long* p)
+      : r(__builtin_amdgcn_make_buffer_rsrc(p, 0, (int)(kCoopSlots * 8), 0x00027000)) {}
+  __device__ void put(int slot, unsigned tag, double v) const {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const slot_t q = {(unsigned)b, tag, (unsigned)(b >> 32), tag};
+    __builtin_amdgcn_raw_buffer_store_b128(q, r, slot * 16, 0, kSlotScope);
+  }
+  __device__ slot_t get(int slot) const {
+    return __builtin_amdgcn_raw_buffer_load_b128(r, slot * 16, 0, kSlotScope);
+  }
+};
+
+// The workgroups, of NT threads, of one launch.  Every thread of every workgroup calls each
+// member together.
+template <int NT>
+struct Team {
+  static constexpr int kWaves = NT / 64;
+  CoopArgs a;
+  unsigned round;  // tag of the last reduction
+  bool good;       // no wait has run out
+
+  int* out;        // LDS: a wait of this workgroup ran out
+
+  __device__ Team(const CoopArgs& args, int* out_) : a(args), out(out_) {
+    round = a.state[0];
+    good = a.state[1] == 0;
+    if (threadIdx.x == 0) *out = 0;  // ordered by the first reduction's barrier
+  }
+  // v[i] summed over all threads of all workgroups, i < NV, in every thread.
+  template <int NV>
+  __device__ void all_sum(double (&v)[NV]) {
+    static_assert(NV <= kCoopVals, "slots");
+    __shared__ double red[NV][kWaves];
+    __shared__ double tot[NV];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, W = gridDim.x;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const double s = wave_sum(v[i]);
+      if (lane == 0) red[i][w] = s;
+    }
+    // this thread's vector stores are complete
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    ++round;
+    const Slots slots(a.slots);
+    const int base = (round & 1) * kCoopVals * kCoopMaxWg;
+    if ((int)threadIdx.x < NV) {
+      double s = 0.0;
+#pragma unroll
+      for (int k = 0; k < kWaves; ++k) s += red[threadIdx.x][k];
+      slots.put(base + (int)threadIdx.x * kCoopMaxWg + blockIdx.x, round, s);
+    }
+    // value i is collected by wavefront i % kWaves: lane u polls workgroups u,
+    // u + 64, .. together
+    for (int i = w; i < NV; i += kWaves) {
+      constexpr int kQ = kCoopMaxWg / 64;
+      const int q = base + i * kCoopMaxWg + lane;
+      slot_t t[kQ];
+      for (int k = 0;; ++k) {
+        bool all = true;
+#pragma unroll
+        for (int u = 0; u < kQ; ++u)
+          if (64 * u < W) t[u] = slots.get(q + (lane + 64 * u < W ? 64 * u : 0));
+#pragma unroll
+        for (int u = 0; u < kQ; ++u)
+          if (64 * u < W) all &= lane + 64 * u >= W || (t[u][1] == round && t[u][3] == round);
+        if (all) break;
+        if (k >= a.spin) { *out = 1; break; }
+        asm volatile("" ::: "memory");  // load again
+      }
+      double s = 0.0;
+#pragma unroll
+      for (int u = 0; u < kQ; ++u)
+        if (lane + 64 * u < W) s += __builtin_bit_cast(double, ((uint64_t)t[u][2] << 32) | t[u][0]);
+      s = wave_sum(s);
+      if (lane == 0) tot[i] = s;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NV; ++i) v[i] = tot[i];
+    if (*out) good = false;
+  }
+  // at the end of the launch: the next launch's first tag, or the failure
+  __device__ void close() {
+    if (threadIdx.x != 0) return;
+    if (!good) a.state[1] = 1;
+    else if (blockIdx.x == 0) a.state[0] = round;
+  }
+};
+
+// The rows of one thread: their entries in registers, and the products with a
+// vector whose own part lies in LDS.  Row j of the thread is row0 + NT j +
+// threadIdx.x; workgroup b owns rows [b * per, (b + 1) * per).
+template <class T, int NT, int RPT>
+struct CoopRows {
+  T a[RPT][kCoopRow];
+  int32_t c[RPT][kCoopRow];
+  int len[RPT];
+  int32_t row0, own;  // the workgroup's first row and number of rows
+  __device__ void load(int64_t n, const int32_t* __restrict__ ptr, const int32_t* __restrict__ col,
+                       const T* __restrict__ val) {
+    const int64_t per = (int64_t)RPT * NT, r0 = (int64_t)blockIdx.x * per;
+    row0 = (int32_t)r0;
+    own = (int32_t)(n - r0 < per ? n - r0 : per);
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) {
+      const int i = at(j);
+      const int32_t s = i < own ? ptr[row0 + i] : 0, e = i < own ? ptr[row0 + i + 1] : 0;
+      len[j] = e - s;
+#pragma unroll
+      for (int k = 0; k < kCoopRow; ++k) {
+        a[j][k] = k < len[j] ? val[s + k] : T(0);
+        c[j][k] = k < len[j] ? col[s + k] : 0;
+      }
+    }
+  }
+  __device__ static int at(int j) { return j * NT + (int)threadIdx.x; }
+  __device__ bool has(int j) const { return at(j) < own; }
+  __device__ bool local(int32_t i) const { return (unsigned)(i - row0) < (unsigned)own; }
+  // Row sums in CSR order, products rounded before the add, as the SpMV
+  // kernels form them.  far(c) loads what x of another workgroup's row c is
+  // formed from, near(that) forms it: the loads of two rows go out together
+  // before the first is used (waited for one by one they cost 0.7 us each).
+  template <class Far, class Near>
+  __device__ __forceinline__ void mul(const T* xl, Far far, Near near, T (&y)[RPT]) const {
+    constexpr int J = RPT < 2 ? RPT : 2;
+#pragma unroll
+    for (int j0 = 0; j0 < RPT; j0 += J) {
+      decltype(far(0)) f[J][kCoopRow];
+#pragma unroll
+      for (int j = 0; j < J; ++j)
+#pragma unroll
+        for (int k = 0; k < kCoopRow; ++k)
+          if (k < len[j0 + j] && !local(c[j0 + j][k])) f[j][k] = far(c[j0 + j][k]);
+#pragma unroll
+      for (int j = 0; j < J; ++j) {
+        T s = T(0);
+#pragma unroll
+        for (int k = 0; k < kCoopRow; ++k)
+          if (k < len[j0 + j]) {
+            const int32_t i = c[j0 + j][k];
+            s = mul_add_rn(s, a[j0 + j][k], local(i) ? xl[i - row0] : near(f[j][k]));
+          }
+        y[j0 + j] = s;
+      }
+    }
+  }
+};
+
+// Whether a CG-family solve ends at count with (r, r) = rr; -1 goes on, else
+// its status (cg_check's rule).
+__device__ inline int cg_stop(long long count, long long maxloop, double rr, double bnorm, double eps) {
+  if (count > maxloop) return 2;
+  const double num = sqrt(rr), err = (bnorm == 0.0 && num == 0.0) ? 0.0 : num / bnorm;
+  return err <= eps ? 0 : !finite(err) ? 3 : -1;
+}
+
+// The residual history as one thread writes it, its length in a register
+// (cg_check's entries).
+struct CoopHist {
+  double* h;
+  long long n, cap;
+  __device__ void add(long long count, long long maxloop, double rr, double bnorm) {
+    if (count > maxloop) return;
+    const double num = sqrt(rr);
+    if (h && n < cap) {
+      h[2 * n] = (double)count;
+      h[2 * n + 1] = (bnorm == 0.0 && num == 0.0) ? 0.0 : num / bnorm;
+    }
+    ++n;
+  }
+};
+
+// CG (cg.cpp:148-272), up to `iters` steps.  mode 0 goes on from the last
+// launch (x in xs, r and p in vec, the scalars in c), 1 starts from
+// r = (T)src and x = 0, 2 from the r (in vec), x and scalars that other kernels
+// left.  A step:
+//   p = beta p + r, q = A p
+//   alpha = rr / (p, q)              first reduction
+//   x += alpha p, r -= alpha q
+//   beta = rr' / rr, stop test       second reduction
+// A gathered p_j of another workgroup is formed from its r_j and the step
+// before's p_j, as that workgroup forms it, so no third reduction has to wait
+// for the new p.  vec holds r (written between the reductions, read after the
+// second) and two p, by parity of the step: a workgroup that is a step ahead
+// of another does not write what that one still reads.
+// last: no launch follows; xout (FP32 solves) receives x when the solve ends.
+// Measured (5-point grids, FP64, per step against three launches): see
+// coop_fits.
+template <class T, int NT, int RPT>
+__global__ __launch_bounds__(NT) void k_cg_coop(int64_t n, const int32_t* __restrict__ ptr,
+                                                const int32_t* __restrict__ col, const T* __restrict__ val,
+                                                const double* __restrict__ src, T* xs, T* vec, int64_t ld,
+                                                double* xout, Ctl* c, CoopArgs ca, int mode, int last, int iters,
+                                                Gate g, StatArgs st) {
+  if (g.off()) return;
+  __shared__ int s_out;
+  Team<NT> team(ca, &s_out);
+  if (!team.good) return;
+  __shared__ T pl[RPT * NT];
+  CoopRows<T, NT, RPT> A;
+  A.load(n, ptr, col, val);
+  T x[RPT], r[RPT], p[RPT], q[RPT];
+  const double eps = c->eps;
+  const long long maxloop = c->maxloop;
+  long long count = mode ? 1 : c->count;
+  double bnorm = c->bnorm, rr = c->rr, alpha = 0.0, beta = mode ? 0.0 : c->beta;
+  CoopHist hist{c->hist, mode == 1 ? 0 : c->nhist, c->hist_cap};
+  int stop = -1;
+  const bool boss = blockIdx.x == 0 && threadIdx.x == 0;
+  bool fresh = mode != 0;  // p is r
+  T* now = vec + (count & 1 ? 2 * ld : ld);  // this step's p
+  T* old = vec + (count & 1 ? ld : 2 * ld);  // the last one's
+#pragma unroll
+  for (int j = 0; j < RPT; ++j) {
+    x[j] = r[j] = p[j] = T(0);
+    if (A.has(j)) {
+      const int32_t i = A.row0 + A.at(j);
+      if (mode == 1) r[j] = (T)src[i];
+      else { x[j] = xs[i]; r[j] = vec[i]; }
+      if (mode == 0) p[j] = old[i];
+    }
+  }
+  if (mode == 1) {
+    double s[1] = {0.0};
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) {
+      if (A.has(j)) shared_store(vec + A.row0 + A.at(j), r[j]);
+      s[0] += (double)r[j] * (double)r[j];
+    }
+    team.all_sum(s);
+    rr = s[0];
+    bnorm = sqrt(rr);
+    stop = team.good ? cg_stop(count, maxloop, rr, bnorm, eps) : 3;
+    if (boss) hist.add(count, maxloop, rr, bnorm);
+  }
+  int done = 0;
+  while (stop < 0 && done < iters) {
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) {
+      p[j] = fresh ? r[j] : (T)(beta * (double)p[j] + (double)r[j]);
+      pl[A.at(j)] = p[j];
+      if (A.has(j)) shared_store(now + A.row0 + A.at(j), p[j]);
+    }
+    __syncthreads();
+    struct Raw {
+      T r, p;
+    };
+    if (fresh)
+      A.mul(pl, [&](int32_t i) { return shared_load(vec + i); }, [](T ri) { return ri; }, q);
+    else
+      A.mul(pl, [&](int32_t i) { return Raw{shared_load(vec + i), shared_load(old + i)}; },
+            [&](Raw f) { return (T)(beta * (double)f.p + (double)f.r); }, q);
+    double s[1] = {0.0};
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) s[0] = fma((double)p[j], (double)q[j], s[0]);
+    team.all_sum(s);
+    alpha = rr / s[0];
+    s[0] = 0.0;
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) {
+      x[j] = (T)(alpha * (double)p[j] + (double)x[j]);
+      r[j] = (T)((-alpha) * (double)q[j] + (double)r[j]);
+      if (A.has(j)) shared_store(vec + A.row0 + A.at(j), r[j]);
+      s[0] = fma((double)r[j], (double)r[j], s[0]);
+    }
+    team.all_sum(s);
+    if (!team.good) break;
+    beta = s[0] / rr;
+    rr = s[0];
+    ++count;
+    ++done;
+    fresh = false;
+    T* t = now;
+    now = old;
+    old = t;
+    stop = cg_stop(count, maxloop, rr, bnorm, eps);
+    if (boss) hist.add(count, maxloop, rr, bnorm);
+  }
+  if (team.good) {
+#pragma unroll
+    for (int j = 0; j < RPT; ++j)
+      if (A.has(j)) {
+        const int32_t i = A.row0 + A.at(j);
+        xs[i] = x[j];
+        if (xout && (stop >= 0 || last)) xout[i] = (double)x[j];
+      }
+    if (boss) {
+      if (mode == 1) { c->done = 0; c->ksz = 0; c->steps = 0; c->bnorm = bnorm; }
+      c->count = count;
+      c->nhist = hist.n;
+      const double num = sqrt(rr);
+      c->err = (bnorm == 0.0 && num == 0.0) ? 0.0 : num / bnorm;
+      c->rr = rr;
+      c->alpha = alpha;
+      c->beta = beta;
+      c->steps += done;
+      c->tsteps += done;
+      c->stop = 0;
+      c->status = 2;
+      if (stop >= 0) ctl_stop(c, stop);
+      st.count_many(done);
+    }
+  }
+  team.close();
+}
+
+}  // namespace ks

@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "../../include/ksolve.h"
+#include "ks_coop.h"
 #include "ks_kernels.h"
 
 namespace ks {
@@ -145,7 +146,10 @@ struct ks_ctx {
   std::string err;
   ks::DBuf<double> part;                 // kMaxGrid * kMaxNV reduction partials
   ks::DBuf<double> part2;                // kMaxGrid partials of a norm whose finisher is deferred
-  ks::DBuf<unsigned long long> stats;    // launches[8], bytes[8]
+  ks::DBuf<unsigned long long> stats;    // launches[8], bytes[8], on-chip solves' state (tag, fail)
+  ks::DBuf<unsigned long long> coop;     // on-chip solves' reduction slots (kCoopSlots)
+  bool coop_off = false;                 // solve with one launch per operation
+  int coop_spin = ks::kCoopSpin;         // polls of one bounded wait
   ks::DBuf<double> scal;                 // scalar outputs of the BLAS entry points
   int* hflags = nullptr;                 // host-mapped flags (host view)
   int* hflags_dev = nullptr;             // same memory, device view
@@ -207,6 +211,7 @@ struct MatView {
   int kind = 0;
   bool wg_tiles = false;
   int L = 8;
+  int64_t max_row = 0;
   int64_t ntiles = 0;
   const int32_t* tiles = nullptr;
   const int32_t* tnz = nullptr;
@@ -295,6 +300,7 @@ inline ks::MatView<double> ks_mat::view<double>(bool trans) const {
   ks::MatView<double> v;
   v.n = n; v.nnz = nnz;
   const ks::Plan& pl = trans ? tplan : plan;
+  v.max_row = trans ? max_trow : max_row;
   if (trans) { v.ptr = tptr.p; v.col = tcol.p; v.val = tval.p; }
   else { v.ptr = ptr.p; v.col = col.p; v.val = val.p; }
   v.set_plan(pl);
@@ -308,6 +314,7 @@ inline ks::MatView<float> ks_mat::view<float>(bool trans) const {
   ks::MatView<float> v;
   v.n = n; v.nnz = nnz;
   const ks::Plan& pl = trans ? tplan : plan;
+  v.max_row = trans ? max_trow : max_row;
   if (trans) { v.ptr = tptr.p; v.col = tcol.p; v.val = tval32.p; }
   else { v.ptr = ptr.p; v.col = col.p; v.val = val32.p; }
   v.set_plan(pl);
@@ -378,6 +385,32 @@ void klaunch(ks_ctx* c, int cls, void (*kernel)(P...), int G, size_t shmem, A&&.
   else
     kernel<<<G, kBlock, shmem, c->stream>>>(P(args)...);
   KS_HIPCK(hipGetLastError());
+}
+
+// Whether a solve with A runs on chip (ks_coop.h): rows of at most kCoopRow
+// entries, at most kCoopRpt per thread of one workgroup per CU.  The line is
+// what the registers hold; up to it a step is the faster one on chip (CG, us a
+// step, on chip against three launches: 32 x 32 3.8 / 13.5, 256 x 256 6.4 /
+// 13.3, 512 x 512 8.6 / 16.4, 724 x 724 13.7 / 23.0, 32^3 6.4 / 14.7, 64^3
+// 9.3 / 16.8, 80^3 23.0 / 25.0; VPCG with ten FP32 CG steps, 300 x 300 102 /
+// 173).
+template <class T>
+bool coop_fits(const ks_ctx* c, const MatView<T>& A) {
+  return !c->coop_off && A.kind == 0 && A.max_row <= kCoopRow &&
+         A.n <= (int64_t)kCoopRpt * kCoopThreads * std::min(c->num_cus, kCoopMaxWg);
+}
+inline CoopArgs coop_args(ks_ctx* c) {
+  return CoopArgs{c->coop.p, reinterpret_cast<unsigned*>(c->stats.p + 2 * KS_K_NCLASS), c->coop_spin};
+}
+// rows per thread: as few as the CUs allow
+inline int coop_rows(const ks_ctx* c, int64_t n) {
+  int r = 1;
+  while (n > (int64_t)r * kCoopThreads * std::min(c->num_cus, kCoopMaxWg)) r *= 2;
+  return r;
+}
+inline int coop_grid(const ks_ctx* c, int64_t n) {
+  const int64_t per = (int64_t)coop_rows(c, n) * kCoopThreads;
+  return (int)((n + per - 1) / per);
 }
 
 // Finisher of a reduction whose producer ran on G workgroups.

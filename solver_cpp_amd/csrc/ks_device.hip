@@ -700,14 +700,31 @@ int64_t total_inner_steps(Level& L) {
   return h.tsteps;
 }
 
-// Run a constructed solve level and fill the result.  prof_mask selects the
+// On-chip solves' slots and state as at the start: no tag given, no failure.
+void coop_reset(ks_ctx* c) {
+  k_fill<unsigned long long><<<grid_map(kCoopSlots), kBlock, 0, c->stream>>>(kCoopSlots, c->coop.p, 0ull);
+  k_fill<unsigned long long><<<1, kBlock, 0, c->stream>>>(1, c->stats.p + 2 * KS_K_NCLASS, 0ull);
+  KS_HIPCK(hipGetLastError());
+}
+
+// One on-chip solve at a time per device: its workgroups wait for each other,
+// so two of them that share the CUs could each hold what the other needs.
+std::mutex& coop_mutex(int device) {
+  static std::mutex m[64];
+  return m[device & 63];
+}
+
+// Run a constructed solve level and fill the result.  Returns false when an
+// on-chip launch gave up waiting (x and res are then undefined).  prof_mask selects the
 // kernel classes timed with events; rbuf (optional, n doubles of device
 // memory the solve no longer needs at the end) holds the residuals of the
 // true-residual checks.
-void run_level(ks_ctx* c, ks_mat* m, Level& Lv, const ks_params* p, unsigned prof_mask, bool trans,
+bool run_level(ks_ctx* c, ks_mat* m, Level& Lv, const ks_params* p, unsigned prof_mask, bool trans,
                const double* b, double* x, double* hist, int64_t hist_cap, ks_result* res, double* x0norm_out,
                double* rbuf) {
   Level* L = &Lv;
+  std::unique_lock<std::mutex> lk;
+  if (L->on_chip()) lk = std::unique_lock<std::mutex>(coop_mutex(c->device));
   L->x0given = (p->flags & KS_X0_GIVEN) != 0;
   double r0 = 0;
   if (L->x0given) r0 = resid_norm(c, m, trans, b, x, rbuf);
@@ -720,8 +737,14 @@ void run_level(ks_ctx* c, ks_mat* m, Level& Lv, const ks_params* p, unsigned pro
   const auto t1 = std::chrono::steady_clock::now();
   Ctl h;
   KS_HIPCK(hipMemcpy(&h, L->dctl.p, sizeof(Ctl), hipMemcpyDeviceToHost));
-  unsigned long long st[2 * KS_K_NCLASS];
+  unsigned long long st[2 * KS_K_NCLASS + 1];
   KS_HIPCK(hipMemcpy(st, c->stats.p, sizeof(st), hipMemcpyDeviceToHost));
+  if (L->on_chip() && (st[2 * KS_K_NCLASS] >> 32)) {
+    coop_reset(c);
+    return false;
+  }
+  // tags are 32 bits: start again long before they could meet an old one
+  if (L->on_chip() && (uint32_t)st[2 * KS_K_NCLASS] > (1u << 31)) coop_reset(c);
   double ms[KS_K_NCLASS] = {0};
   c->prof.collect(ms);
   c->prof.mask = 0;
@@ -754,13 +777,26 @@ void run_level(ks_ctx* c, ks_mat* m, Level& Lv, const ks_params* p, unsigned pro
     }
   }
   if (x0norm_out) *x0norm_out = r0;
+  return true;
 }
 
 void solve_impl(ks_ctx* c, ks_mat* m, const ks_params* p, bool trans, const double* b, double* x, double* hist,
                 int64_t hist_cap, ks_result* res, double* x0norm_out) {
-  auto L = make_solver(c, m, p, trans, hist ? hist_cap : 0);
-  run_level(c, m, *L, p, p->profile > 0 ? (unsigned)p->profile : 0u, trans, b, x, hist, hist_cap, res, x0norm_out,
-            nullptr);
+  // per-class times need the operations' own launches
+  c->coop_off = p->profile > 0;
+  DBuf<double> x0;  // the initial guess, should an on-chip solve have to be repeated
+  for (;;) {
+    auto L = make_solver(c, m, p, trans, hist ? hist_cap : 0);
+    if (L->on_chip() && (p->flags & KS_X0_GIVEN)) {
+      x0.alloc(m->n);
+      KS_HIPCK(hipMemcpyAsync(x0.p, x, sizeof(double) * m->n, hipMemcpyDeviceToDevice, c->stream));
+    }
+    if (run_level(c, m, *L, p, p->profile > 0 ? (unsigned)p->profile : 0u, trans, b, x, hist, hist_cap, res,
+                  x0norm_out, nullptr))
+      return;
+    c->coop_off = true;
+    if (x0.p) KS_HIPCK(hipMemcpyAsync(x, x0.p, sizeof(double) * m->n, hipMemcpyDeviceToDevice, c->stream));
+  }
 }
 
 // ------------------------------------------------ no-allocation CG solve ---
@@ -834,7 +870,9 @@ ks_status ks_ctx_create(int32_t device, ks_ctx** out) {
     c->part.alloc((size_t)kMaxGrid * kMaxNV);
     c->part2.alloc((size_t)kMaxGrid);
     KS_HIPCK(hipMemsetAsync(c->part2.p, 0, sizeof(double) * kMaxGrid, c->stream));
-    c->stats.alloc(2 * KS_K_NCLASS);
+    c->stats.alloc(2 * KS_K_NCLASS + 1);
+    c->coop.alloc(kCoopSlots);
+    coop_reset(c);
     c->scal.alloc(1024);
     KS_HIPCK(hipHostMalloc((void**)&c->hflags, 64 * sizeof(int), hipHostMallocMapped));
     std::memset(c->hflags, 0, 64 * sizeof(int));
@@ -869,6 +907,7 @@ void ks_ctx_destroy(ks_ctx* c) {
   for (auto e : c->evpool) (void)hipEventDestroy(e);
   c->part.release();
   c->stats.release();
+  c->coop.release();
   c->scal.release();
   if (c->hflags) (void)hipHostFree(c->hflags);
   if (c->stream && c->own_stream) (void)hipStreamDestroy(c->stream);
@@ -876,6 +915,11 @@ void ks_ctx_destroy(ks_ctx* c) {
 }
 
 const char* ks_ctx_last_error(const ks_ctx* c) { return c ? c->err.c_str() : "null context"; }
+ks_status ks_ctx_set_wait_limit(ks_ctx* c, int32_t polls) {
+  if (!c || polls < 0) return KS_ERR_BAD_INPUT;
+  c->coop_spin = polls;
+  return KS_OK;
+}
 void* ks_ctx_stream(ks_ctx* c) { return c ? (void*)c->stream : nullptr; }
 ks_status ks_ctx_synchronize(ks_ctx* c) {
   if (!c) return KS_ERR_BAD_INPUT;
@@ -1316,10 +1360,15 @@ ks_status ks_solve_noalloc(ks_ctx* c, ks_mat* m, const ks_params* p, const doubl
   static_assert(CgLevel<double>::scratch_doubles(kNoAllocMaxRows) <= 3 * kNoAllocMaxRows + 1024,
                 "scratch holds three padded vectors and the control state at the maximum size");
   std::lock_guard<std::mutex> lk(scratch_table().call[c->device]);
-  CgLevel<double> L;
-  L.setup(c, m->view<double>(false), outer_cfg(p, 0), c->scratch);
-  // q is free once the solve has ended: it holds the final residual check
-  run_level(c, m, L, p, 0u, false, b, x, nullptr, 0, res, nullptr, L.q.p);
+  // an on-chip solve that has to be repeated would need a copy of the guess
+  c->coop_off = (p->flags & KS_X0_GIVEN) != 0;
+  for (;;) {
+    CgLevel<double> L;
+    L.setup(c, m->view<double>(false), outer_cfg(p, 0), c->scratch);
+    // q is free once the solve has ended: it holds the final residual check
+    if (run_level(c, m, L, p, 0u, false, b, x, nullptr, 0, res, nullptr, L.q.p)) break;
+    c->coop_off = true;
+  }
   KS_HIPCK(hipStreamSynchronize(c->stream));
   return KS_OK;
   KS_API_CATCH(c)

@@ -101,12 +101,51 @@ struct StatArgs {
       atomicAdd(bytes + cls, nbytes);
     }
   }
+  // by one thread, for a launch that did the work of m
+  __device__ void count_many(int m) const {
+    if (!launches) return;
+    atomicAdd(launches + cls, (unsigned long long)m);
+    atomicAdd(bytes + cls, nbytes * (unsigned long long)m);
+  }
 };
 
 // ----------------------------------------------------------- reductions --
+// v of lane ^ 32, ^ 16 (permlane swaps) and of the lane CTRL names (DPP), on
+// both halves of a double: register moves, where a shuffle goes through LDS.
+template <int CTRL>
+__device__ __forceinline__ double dpp(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, 0xf, 0xf, false);
+  const uint32_t hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, 0xf, 0xf, false);
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+template <int OFF>
+__device__ __forceinline__ uint32_t swap_lanes(uint32_t x) {
+  const int lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0));
+  if constexpr (OFF == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    return lane & 32 ? r[0] : r[1];
+  } else {
+    const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    return lane & 16 ? r[0] : r[1];
+  }
+}
+template <int OFF>
+__device__ __forceinline__ double swap_lanes(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  return __builtin_bit_cast(double, ((uint64_t)swap_lanes<OFF>((uint32_t)(b >> 32)) << 32) |
+                                        swap_lanes<OFF>((uint32_t)b));
+}
+// The sum over the wavefront, in every lane: the pairs lane ^ 32, ^ 16, ^ 8,
+// ^ 4, ^ 2, ^ 1 in this order (row_ror:8 is ^ 8 in a row of 16; row_ror:4 is
+// ^ 4 once the values repeat every 8 lanes).
 __device__ inline double wave_sum(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  v += swap_lanes<32>(v);
+  v += swap_lanes<16>(v);
+  v += dpp<0x128>(v);  // row_ror:8
+  v += dpp<0x124>(v);  // row_ror:4
+  v += dpp<0x4e>(v);   // quad_perm:[2,3,0,1]
+  v += dpp<0xb1>(v);   // quad_perm:[1,0,3,2]
   return v;
 }
 

@@ -605,6 +605,8 @@ struct Level {
   virtual void enqueue_finish() {}
   virtual int64_t reported_iters(const Ctl& h) const { return h.count; }
   virtual double unit_seconds_estimate() const = 0;
+  // some of this solve's launches run on chip (ks_coop.h)
+  virtual bool on_chip() const { return false; }
 };
 
 // ------------------------------------------------------------- CG ------
@@ -612,8 +614,11 @@ template <class T>
 struct CgLevel : Level {
   MatView<T> A;
   DBuf<T> r, p, q, xown;
+  DBuf<T> vec;  // on chip: r, p and q above, in one allocation
   T* x = nullptr;
   double* xout = nullptr;
+  bool coop = false;            // on chip: a unit is kCoopIters steps in one launch (k_cg_coop)
+  const double* src = nullptr;  // on chip: the right-hand side
   // Doubles of device memory setup(..., mem) takes: r, p and q (each padded
   // to 64 elements), then the small arrays and the control block.
   static constexpr int64_t scratch_doubles(int64_t n) { return 3 * pad64(n) + ctl_doubles(0, 0); }
@@ -621,23 +626,30 @@ struct CgLevel : Level {
   // that holds every vector and the control state instead of allocations
   void setup(ks_ctx* cx, const MatView<T>& a, const LevelCfg& cf, double* mem = nullptr) {
     c = cx; A = a; n = a.n; cfg = cf;
+    coop = coop_fits(c, A) && cfg.maxloop > 0;
+    const int64_t ld = pad64(n);
     if (mem) {
       KS_CHECK(sizeof(T) == 8, KS_ERR_UNSUPPORTED, "borrowed CG state is FP64 only");
-      const int64_t ld = pad64(n);
       r.borrow((T*)mem, n);
       p.borrow((T*)(mem + ld), n);
       q.borrow((T*)(mem + 2 * ld), n);
       setup_ctl(0, 0, mem + 3 * ld);
       return;
     }
-    r.alloc(n); p.alloc(n); q.alloc(n);
+    if (coop) {
+      vec.alloc(3 * ld);
+      r.borrow(vec.p, n); p.borrow(vec.p + ld, n); q.borrow(vec.p + 2 * ld, n);
+    } else {
+      r.alloc(n); p.alloc(n); q.alloc(n);
+    }
     if (sizeof(T) != 8) xown.alloc(n);
     setup_ctl(0, 0);
   }
   void enqueue_init(const double* b, double* x_out) override {
     xout = x_out;
     x = sizeof(T) == 8 ? (T*)x_out : xown.p;
-    const double* src = b;
+    src = b;
+    if (coop && !x0given) return;  // the first launch starts the solve
     if (x0given) {  // outer FP64 only: bnorm, then r = b - A x0
       launch_map<1>(c, n, OpSetBnorm{b, ctl()}, gouter(), KS_K_REDUCE, 8.0 * n);
       launch_spmv<T, 1>(c, A, x, EpiResid<T, FinNone>{b, r.p, FinNone{}}, gouter(), 8.0 * n);
@@ -650,6 +662,25 @@ struct CgLevel : Level {
   // take the totals themselves (OpCgUpdateF, OpXpbyF): three launches per
   // iteration, no finisher
   void enqueue_unit(int64_t u) override {
+    if (coop) {
+      const int mode = u > 0 ? 0 : x0given ? 2 : 1;
+      const int64_t ld = pad64(n);
+      const int iters = (int)std::min<int64_t>(kCoopIters, cfg.maxloop - u * kCoopIters);
+      const StatArgs st = stat(c, sizeof(T) == 8 ? KS_K_SPMV64 : KS_K_SPMV32, spmv_bytes<T>(A) + 10.0 * sizeof(T) * n);
+      auto go = [&](auto kernel) {
+        kernel<<<coop_grid(c, n), kCoopThreads, 0, c->stream>>>(n, A.ptr, A.col, A.val, src, x, r.p, ld,
+                                                             sizeof(T) == 8 ? nullptr : xout, ctl(), coop_args(c), mode,
+                                                             u + 1 == max_units(), iters,
+                                                             mode == 1 ? gouter() : gstep(), st);
+      };
+      switch (coop_rows(c, n)) {
+        case 1: go(k_cg_coop<T, kCoopThreads, 1>); break;
+        case 2: go(k_cg_coop<T, kCoopThreads, 2>); break;
+        default: go(k_cg_coop<T, kCoopThreads, 4>); break;
+      }
+      KS_HIPCK(hipGetLastError());
+      return;
+    }
     const int slot = (int)(u & 1);
     const int gd = launch_spmv<T, 1>(c, A, p.p, EpiDot<T, FinAlpha>{p.p, q.p, FinAlpha{ctl()}}, gstep(),
                                      sizeof(T) * (double)n, false);
@@ -658,14 +689,19 @@ struct CgLevel : Level {
     launch_map<0>(c, n, OpXpbyF<T>{p.p, r.p, ctl(), c->part2.p, gu, slot, 0.0}, gstep(), KS_K_AXPY,
                   3.0 * sizeof(T) * n);
   }
-  int64_t max_units() const override { return cfg.maxloop > 0 ? cfg.maxloop : 0; }
+  int64_t max_units() const override {
+    if (coop) return (cfg.maxloop + (int64_t)kCoopIters - 1) / kCoopIters;
+    return cfg.maxloop > 0 ? cfg.maxloop : 0;
+  }
+  bool on_chip() const override { return coop; }
   void enqueue_finish() override {
-    if (sizeof(T) != 8) {
+    if (sizeof(T) != 8 && !coop) {
       k_convert<T, double><<<grid_map(n), kBlock, 0, c->stream>>>(n, x, xout, gouter());
       KS_HIPCK(hipGetLastError());
     }
   }
   double unit_seconds_estimate() const override {
+    if (coop) return 4e-6 * std::min(cfg.maxloop, kCoopIters);
     return std::max(3 * 4e-6, (spmv_bytes<T>(n, A.nnz) + 10.0 * sizeof(T) * n) / 4e12);
   }
 };
@@ -1102,6 +1138,7 @@ struct GmresLevel : Level {
     cycle_end();  // no-op unless the solve stopped in a cycle not yet assembled
   }
   int64_t reported_iters(const Ctl& hc) const override { return hc.count + 1; }
+  bool on_chip() const override { return inner && inner->on_chip(); }
   double unit_seconds_estimate() const override {
     double s = (spmv_bytes<T>(n, A.nnz) + (double)sizeof(T) * n * (R + 8)) / 4e12 + 5 * 4e-6;
     if (inner) s += inner->max_units() * inner->unit_seconds_estimate();
@@ -1266,6 +1303,7 @@ struct GcrLevel : Level {
       KS_HIPCK(hipGetLastError());
     }
   }
+  bool on_chip() const override { return inner && inner->on_chip(); }
   double unit_seconds_estimate() const override {
     double s = (spmv_bytes<T>(n, A.nnz) + (double)sizeof(T) * n * (2 * R + 8)) / 4e12 + 7 * 4e-6;
     if (inner) s += inner->max_units() * inner->unit_seconds_estimate();
@@ -1409,6 +1447,7 @@ struct VpcgLevel : Level {
     launch_map<0>(c, n, OpXpby<double>{p.p, z.p, nullptr, nullptr, ctl(), 0.0}, gstep(), KS_K_AXPY, 24.0 * n);
   }
   int64_t max_units() const override { return cfg.maxloop > 0 ? cfg.maxloop : 0; }
+  bool on_chip() const override { return inner->on_chip(); }
   double unit_seconds_estimate() const override {
     return (spmv_bytes<double>(n, A.nnz) + 150.0 * n) / 4e12 + 5 * 4e-6 +
            inner->max_units() * inner->unit_seconds_estimate();
