@@ -74,7 +74,11 @@ typedef enum ks_status {
                                  XCD's L2 (chosen automatically, with no layout
                                  flag, for n >= 2^21 rows when over half the
                                  entries lie more than n/8 columns from their
-                                 row) */
+                                 row, unless column blocks apply: then, with
+                                 heavy-tailed row lengths as for KS_MAT_MERGE,
+                                 at least 393216 rows and 10M entries, the SpMV
+                                 gathers x from slices of 16384 columns in LDS
+                                 in a pass of its own) */
 #define KS_MAT_COL32    2048u /* keep int32 column indices in the SpMV.  Without
                                  it, a matrix whose rows repeat at most 32
                                  lists of column offsets col - row (stencils)
@@ -199,7 +203,8 @@ ks_status ks_mat_get_transpose(ks_mat* m, int32_t* tptr, int32_t* tcol,
 /* Destroy every matrix of a context before the context itself. */
 void ks_mat_destroy(ks_mat* m);
 /* n, nnz and the SpMV variant chosen: spmv_kind 0 CSR-stream tiles (workgroup
- * or wavefront), 1 lanes-per-row vector kernel, 2 merge path, 3 column panels;
+ * or wavefront), 1 lanes-per-row vector kernel, 2 merge path, 3 column panels or
+ * blocks;
  * lanes_per_row is the vector kernel's lanes per row (the smallest power of
  * two >= the mean row length, in [2, 64]), reported for every kind. */
 ks_status ks_mat_info(const ks_mat* m, int64_t* n, int64_t* nnz,

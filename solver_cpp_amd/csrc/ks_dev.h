@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "../../include/ksolve.h"
+#include "ks_bins.h"
 #include "ks_coop.h"
 #include "ks_kernels.h"
 
@@ -221,6 +222,7 @@ struct MatView {
   int np = 0;
   const MatView* panel = nullptr;
   T* pacc = nullptr;
+  BinView bins;  // column blocks (kind 3, bins.nblk > 0): two passes (ks_bins.h)
   void set_plan(const Plan& pl) {
     kind = pl.kind;
     L = pl.L;
@@ -237,6 +239,14 @@ struct MatView {
 // behind it (null: the side has none).
 struct PatBuf : DBuf<int32_t> {
   const PatIx* code = nullptr;
+};
+
+// Column blocks and segments of one side (ks_bins.h).
+struct BinSet {
+  DBuf<int32_t> seg, snz, unit, shift;
+  DBuf<uint16_t> lcol, place, before;
+  DBuf<uint64_t> mask;
+  BinView v;  // nblk 0: the side has none
 };
 
 // Column panels of one CSR matrix (A or A^T).  On matrices whose rows gather
@@ -278,6 +288,8 @@ struct ks_mat {
   ks::DBuf<float> tval32;
   ks::Plan plan, tplan;
   ks::PanelSet panels, tpanels;
+  ks::BinSet bins, tbins;
+  ks::DBuf<double> xg;  // their x by entry, used by one product at a time
   int64_t max_row = 0, max_trow = 0;
 
   template <class T>
@@ -306,6 +318,8 @@ inline ks::MatView<double> ks_mat::view<double>(bool trans) const {
   v.set_plan(pl);
   const ks::PanelSet& ps = trans ? tpanels : panels;
   if (ps.np) { v.np = ps.np; v.panel = ps.v64.data(); v.pacc = ps.acc64.p; v.kind = 3; }
+  v.bins = trans ? tbins.v : bins.v;
+  if (v.bins.nblk) v.kind = 3;
   set_col16(v, trans);
   return v;
 }
@@ -320,6 +334,8 @@ inline ks::MatView<float> ks_mat::view<float>(bool trans) const {
   v.set_plan(pl);
   const ks::PanelSet& ps = trans ? tpanels : panels;
   if (ps.np && ps.val32.p) { v.np = ps.np; v.panel = ps.v32.data(); v.pacc = ps.acc32.p; v.kind = 3; }
+  v.bins = trans ? tbins.v : bins.v;
+  if (v.bins.nblk) v.kind = 3;
   set_col16(v, trans);
   return v;
 }
@@ -351,12 +367,12 @@ inline int grid_rows(int64_t nrb) {
 // larger than one resident wave leaves a second, partly filled wave of
 // workgroups (a tail) that runs after the rest.
 template <class K>
-int resident(ks_ctx* c, K kernel, size_t dyn_lds = 0) {
+int resident(ks_ctx* c, K kernel, size_t dyn_lds = 0, int threads = kBlock) {
   const auto key = std::make_pair(reinterpret_cast<const void*>(kernel), dyn_lds);
   auto it = c->occ.find(key);
   if (it != c->occ.end()) return it->second;
   int per_cu = 0;
-  KS_HIPCK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kernel), kBlock,
+  KS_HIPCK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kernel), threads,
                                                          dyn_lds));
   const int r = std::max(1, per_cu) * std::max(1, c->num_cus);
   c->occ.emplace(key, r);
@@ -377,14 +393,23 @@ int grid_rows(ks_ctx* c, K kernel, int64_t nrb, size_t dyn_lds = 0) {
 // that the runtime sets to the kernel's own execution interval (the
 // dispatch's begin and end timestamps, as in a profiler's kernel trace), so
 // the per-class times exclude the gaps between kernels.
-template <class... P, class... A>
-void klaunch(ks_ctx* c, int cls, void (*kernel)(P...), int G, size_t shmem, A&&... args) {
+template <int NT, class... P, class... A>
+void klaunch_t(ks_ctx* c, int cls, void (*kernel)(P...), int G, size_t shmem, A&&... args) {
   hipEvent_t e0 = nullptr, e1 = nullptr;
   if (c->prof.pair(cls, e0, e1))
-    hipExtLaunchKernelGGL(kernel, dim3(G), dim3(kBlock), (uint32_t)shmem, c->stream, e0, e1, 0u, P(args)...);
+    hipExtLaunchKernelGGL(kernel, dim3(G), dim3(NT), (uint32_t)shmem, c->stream, e0, e1, 0u, P(args)...);
   else
-    kernel<<<G, kBlock, shmem, c->stream>>>(P(args)...);
+    kernel<<<G, NT, shmem, c->stream>>>(P(args)...);
   KS_HIPCK(hipGetLastError());
+}
+template <class... P, class... A>
+void klaunch(ks_ctx* c, int cls, void (*kernel)(P...), int G, size_t shmem, A&&... args) {
+  klaunch_t<kBlock>(c, cls, kernel, G, shmem, std::forward<A>(args)...);
+}
+// workgroups of NT threads
+template <int NT, class... P, class... A>
+void klaunch_n(ks_ctx* c, int cls, void (*kernel)(P...), int G, A&&... args) {
+  klaunch_t<NT>(c, cls, kernel, G, 0, std::forward<A>(args)...);
 }
 
 // Whether a solve with A runs on chip (ks_coop.h): rows of at most kCoopRow
@@ -452,6 +477,7 @@ inline double spmv_bytes(int64_t n, int64_t nnz, int ib = 4) {
 template <class T>
 inline double spmv_bytes(const MatView<T>& A) {
   if (A.pat) return (double)sizeof(T) * A.nnz + 2.0 * A.n + 2.0 * sizeof(T) * A.n;
+  if (A.bins.nblk) return (3.0 * sizeof(T) + 4) * A.nnz + 4.0 * (A.n + 1) + 2.0 * sizeof(T) * A.n;
   return spmv_bytes<T>(A.n, A.nnz, A.ib);
 }
 
@@ -575,6 +601,21 @@ struct EpiPanelLast {
   __device__ void fin(const double* s) const { e.fin(s); }
 };
 
+// First pass of a product over column blocks: x by entry into bins.xg.
+template <class T>
+void launch_bin_gather(ks_ctx* c, const BinView& B, int64_t n, const T* x, Gate g, int cls) {
+  klaunch_n<kBinGather>(c, cls, k_bin_gather<T>, (int)B.nunit, n, B.unit, B.lcol, x, (T*)B.xg, g);
+}
+// Both passes; returns the second's grid (one resident wave of its workgroups).
+template <class T, int NV, class Epi>
+int spmv_bins(ks_ctx* c, const MatView<T>& A, const T* x, const Epi& epi, Gate g, int cls, double bytes) {
+  launch_bin_gather<T>(c, A.bins, A.n, x, g, cls);
+  const int G = grid_rows(std::min<int64_t>(A.bins.nseg, resident(c, k_bin_sum<T, NV, Epi>, 0, kBinSum)));
+  klaunch_n<kBinSum>(c, cls, k_bin_sum<T, NV, Epi>, G, A.bins, A.ptr, A.val, (const T*)A.bins.xg, epi, g, red(c),
+                     stat(c, cls, bytes));
+  return G;
+}
+
 // y-side epilogue of SpMV plus NV reduction values (finished by k_finish).
 // With finish false no finisher is launched (a later kernel forms the
 // totals of the G partials, G returned).
@@ -584,7 +625,9 @@ int launch_spmv(ks_ctx* c, const MatView<T>& A, const T* x, const Epi& epi, Gate
   const int cls = sizeof(T) == 8 ? KS_K_SPMV64 : KS_K_SPMV32;
   const double bytes = spmv_bytes<T>(A) + extra_bytes;
   int G;
-  if (A.np > 0) {
+  if (A.bins.nblk) {
+    G = spmv_bins<T, NV>(c, A, x, epi, g, cls, bytes);
+  } else if (A.np > 0) {
     // the bytes of the whole SpMV are counted with the last pass
     for (int p = 0; p + 1 < A.np; ++p)
       spmv_dispatch<T, 0>(c, A.panel[p], x, EpiPanelAcc<T>{A.pacc, p == 0}, g, cls, 0.0);
@@ -606,7 +649,7 @@ struct EpiStore2;
 // with the plan's tiles).
 template <class T>
 void launch_spmv2(ks_ctx* c, const MatView<T>& A, const T* x1, const T* x2, T* y1, T* y2, Gate g) {
-  if (A.np > 0) {  // column panels: two single-vector SpMVs
+  if (A.np > 0 || A.bins.nblk) {  // column panels or blocks: two single-vector SpMVs
     launch_spmv<T, 0>(c, A, x1, EpiStore<T>{y1}, g);
     launch_spmv<T, 0>(c, A, x2, EpiStore<T>{y2}, g);
     return;

@@ -136,10 +136,22 @@ bool merge_choice(uint32_t flags, int64_t n, int64_t nnz, int64_t max_row) {
 // with 6 / 8 / 12 / 16 panels): fewer passes miss L2 more on the gathers,
 // more passes re-read every row's pointer and partial sum more often.
 constexpr int kPanels = 10;
-bool panel_choice(uint32_t flags, int64_t n, const int32_t* hp, const int32_t* hc) {
-  if (flags & KS_MAT_PANELS) return true;
-  if (flags & (KS_MAT_VECTOR | KS_MAT_WG_TILES | KS_MAT_WAVE_TILES | KS_MAT_MERGE)) return false;
-  if (n < (int64_t(1) << 21)) return false;
+// The line: two streaming passes beat one gathering pass once x outgrows what
+// the L2s serve (n) and there are entries enough for two launches that fill
+// the GPU.  Measured, FP64 / FP32 / SDDMM in us, column blocks against the
+// layout before them (merge path, column panels from 2^21 rows): rows of up
+// to 4096 entries, n = 250000 115 / 80 / 139 against 103 / 93 / 166, 400000
+// 155 / 104 / 183 against 163 / 147 / 320, 10^6 405 / 208 / 421 against 530 /
+// 368 / 789, 4 10^6 1596 / 965 / 1645 against 1884 / 1604 / 3511; rows of up
+// to 300 entries, n = 500000 (6.6M entries) 97 / 61 / 109 against 67 / 58 /
+// 127, 10^6 (13M) 129 / 85 / 148 against 155 / 112 / 236, 4 10^6 488 / 254 /
+// 478 against 1275 / 748 / 998.  Sides of even row lengths (a random
+// matrix's A^T) keep tiles and panels, which are as fast in FP64 (4 10^6:
+// 1527 against 1418) and fuse the GMRES projection.
+constexpr int64_t kBinMinRows = 3 << 17, kBinMinEntries = 10 << 20;
+constexpr uint32_t kLayouts = KS_MAT_PANELS | KS_MAT_VECTOR | KS_MAT_WG_TILES | KS_MAT_WAVE_TILES | KS_MAT_MERGE;
+// over half of the entries of sampled rows lie more than n/8 columns away
+bool gathers_far(int64_t n, const int32_t* hp, const int32_t* hc) {
   int64_t far = 0, all = 0;
   for (int64_t r = 0; r < n; r += 61)
     for (int32_t j = hp[r]; j < hp[r + 1]; ++j) {
@@ -147,6 +159,79 @@ bool panel_choice(uint32_t flags, int64_t n, const int32_t* hp, const int32_t* h
       ++all;
     }
   return all > 0 && 2 * far > all;
+}
+bool panel_choice(uint32_t flags, int64_t n, const int32_t* hp, const int32_t* hc) {
+  if (flags & kLayouts) return (flags & KS_MAT_PANELS) != 0;
+  return n >= (int64_t(1) << 21) && gathers_far(n, hp, hc);
+}
+bool bin_shape(int64_t n, int64_t nnz, int64_t max_row) {
+  return n >= kBinMinRows && n <= (int64_t)kBinBlocks * kBinCols && nnz >= kBinMinEntries && max_row <= kBinEntries;
+}
+// Column blocks (ks_bins.h), by default (no layout flag), for a matrix whose
+// gathers are mostly far and whose row lengths are heavy-tailed, where its
+// shape allows it.
+bool bin_choice(uint32_t flags, int64_t n, int64_t nnz, int64_t max_row, const int32_t* hp, const int32_t* hc) {
+  return !(flags & kLayouts) && merge_choice(flags, n, nnz, max_row) && bin_shape(n, nnz, max_row) &&
+         gathers_far(n, hp, hc);
+}
+
+// Column blocks of the CSR (ptr, col; hp: host row pointers).
+void build_bins(ks_mat* m, BinSet& bs, const int32_t* hp, const int32_t* ptr, const int32_t* col) {
+  ks_ctx* c = m->ctx;
+  hipStream_t s = c->stream;
+  const int64_t n = m->n, nnz = m->nnz;
+  TileSet ts;
+  std::vector<int32_t> t = build_tiles(hp, n, kBinRows, kBinEntries), z(t.size());
+  for (size_t i = 0; i < t.size(); ++i) z[i] = hp[t[i]];
+  upload_tiles(c, ts, t, z);
+  const int64_t nseg = ts.ntiles;
+  const int nblk = (int)((n + kBinCols - 1) / kBinCols);
+  const int64_t runs = nseg * nblk;
+  DBuf<int32_t> run(runs + 1);  // start in xg of the run of (block, segment), block-major
+  k_bin_count<<<(unsigned)nseg, kBlock, 0, s>>>(nblk, nseg, ts.tnz.p, col, run.p);
+  const int64_t nb = (runs + 1023) / 1024;
+  DBuf<int64_t> bsum(nb + 1);
+  k_scan_blocks<<<nb, kBlock, 0, s>>>(runs, run.p, bsum.p);
+  k_scan_serial<<<1, 1, 0, s>>>(nb, bsum.p);
+  k_scan_apply<<<nb, kBlock, 0, s>>>(runs, run.p, bsum.p, run.p);
+  KS_HIPCK(hipGetLastError());
+  bs.lcol.alloc(nnz + 4);  // read four at a time
+  bs.place.alloc(nnz);
+  bs.mask.alloc(nseg * kBinWords);
+  bs.before.alloc(nseg * kBinWords);
+  bs.shift.alloc(runs);
+  k_bin_fill<<<(unsigned)nseg, kBlock, 0, s>>>(nblk, nseg, ts.tnz.p, col, run.p, bs.lcol.p, bs.place.p, bs.mask.p,
+                                               bs.before.p, bs.shift.p);
+  KS_HIPCK(hipGetLastError());
+  // the first pass's units: at most kBinUnit entries of one block
+  std::vector<int32_t> start(nblk + 1, (int32_t)nnz), unit;
+  DBuf<int32_t> dstart(nblk);
+  k_bin_starts<<<grid_map(nblk), kBlock, 0, s>>>(nblk, nseg, run.p, dstart.p);
+  KS_HIPCK(hipGetLastError());
+  KS_HIPCK(hipMemcpyAsync(start.data(), dstart.p, sizeof(int32_t) * nblk, hipMemcpyDeviceToHost, s));
+  KS_HIPCK(hipStreamSynchronize(s));
+  for (int b = 0; b < nblk; ++b) {
+    const int64_t k = std::max<int64_t>(1, (start[b + 1] - start[b] + kBinUnit - 1) / kBinUnit);
+    const int64_t a = start[b], len = start[b + 1] - a;
+    for (int64_t i = 0; i < k; ++i)
+      if (len > 0) {
+        unit.push_back(b);
+        unit.push_back((int32_t)(a + len * i / k));
+        unit.push_back((int32_t)(a + len * (i + 1) / k));
+      }
+  }
+  bs.unit.alloc(unit.size());
+  KS_HIPCK(hipMemcpyAsync(bs.unit.p, unit.data(), sizeof(int32_t) * unit.size(), hipMemcpyHostToDevice, s));
+  if (!m->xg.p) m->xg.alloc(nnz + 4);
+  KS_HIPCK(hipStreamSynchronize(s));
+  bs.seg = std::move(ts.tiles);
+  bs.snz = std::move(ts.tnz);
+  bs.v.nseg = nseg;
+  bs.v.nunit = (int64_t)unit.size() / 3;
+  bs.v.nblk = nblk;
+  bs.v.seg = bs.seg.p; bs.v.snz = bs.snz.p; bs.v.unit = bs.unit.p;
+  bs.v.mask = bs.mask.p; bs.v.before = bs.before.p; bs.v.shift = bs.shift.p;
+  bs.v.lcol = bs.lcol.p; bs.v.place = bs.place.p; bs.v.xg = m->xg.p;
 }
 
 // Panel values from A's values (and their FP32 copy when there is one).
@@ -275,7 +360,7 @@ void build_index16(ks_mat* m, const int32_t* hp, const int32_t* hc) {
   int off16 = -1;  // not looked at yet
   auto side = [&](PatBuf& op, DBuf<int16_t>& o16, DBuf<uint16_t>& od, const Plan& pl,
                   const PanelSet& ps, const int32_t* ptr, const int32_t* col) {
-    if (ps.np) return;
+    if (ps.np || pl.kind != 0) return;
     if (!delta_first && build_patterns(m, pl, op, ptr, col)) return;
     if (off16 < 0) off16 = offsets_fit16(m->n, hp, hc);
     if (off16 && !delta_first) build_col16(m, o16, ptr, col);
@@ -490,10 +575,18 @@ void build_transpose(ks_mat* m) {
     k_gather<double, double><<<grid_map(nnz), kBlock, 0, s>>>(nnz, m->tperm.p, m->val.p, m->tval.p);
     KS_HIPCK(hipGetLastError());
   }
+  m->has_t = true;
+  // A^T gathers as randomly as A
+  const bool far = m->bins.v.nblk || m->panels.np;
+  if (far && !(m->flags & kLayouts) && merge_choice(m->flags, n, nnz, mx) && bin_shape(n, nnz, mx)) {
+    m->tplan.L = choose_lanes(n, nnz);
+    m->tplan.kind = 2;
+    build_bins(m, m->tbins, htp.data(), m->tptr.p, m->tcol.p);
+    return;
+  }
   make_plan(c, m->tplan, htp.data(), n, nnz, (m->flags & KS_MAT_VECTOR) != 0, tile_choice(m->flags),
             merge_choice(m->flags, n, nnz, mx));
-  m->has_t = true;
-  if (m->panels.np && nnz > 0) {  // A^T gathers as randomly as A
+  if (nnz > 0 && (m->panels.np || (far && n >= (int64_t(1) << 21)))) {
     std::vector<int32_t> htc(nnz);
     KS_HIPCK(hipMemcpyAsync(htc.data(), m->tcol.p, sizeof(int32_t) * nnz, hipMemcpyDeviceToHost, s));
     KS_HIPCK(hipStreamSynchronize(s));
@@ -980,10 +1073,16 @@ ks_status ks_mat_create_csr(ks_ctx* c, int64_t n, int64_t nnz, const int32_t* pt
   m->max_row = mx;
   KS_CHECK(!((flags & KS_MAT_COL32) && (flags & KS_MAT_COL_DELTA)), KS_ERR_BAD_INPUT,
            "KS_MAT_COL32 and KS_MAT_COL_DELTA exclude each other");
-  make_plan(c, m->plan, hp.data(), n, nnz, (flags & KS_MAT_VECTOR) != 0, tile_choice(flags),
+  if (bin_choice(flags, n, nnz, mx, hp.data(), hc.data())) {
+    m->plan.L = choose_lanes(n, nnz);
+    m->plan.kind = 2;  // no tiles: the bins are the plan
+    build_bins(m.get(), m->bins, hp.data(), m->ptr.p, m->col.p);
+  } else {
+    make_plan(c, m->plan, hp.data(), n, nnz, (flags & KS_MAT_VECTOR) != 0, tile_choice(flags),
               merge_choice(flags, n, nnz, mx));
-  if (nnz > 0 && panel_choice(flags, n, hp.data(), hc.data()))
-    build_panels(m.get(), m->panels, hp.data(), hc.data(), nullptr, flags);
+    if (nnz > 0 && panel_choice(flags, n, hp.data(), hc.data()))
+      build_panels(m.get(), m->panels, hp.data(), hc.data(), nullptr, flags);
+  }
   if (flags & KS_MAT_TRANSPOSE) build_transpose(m.get());
   if (!(flags & KS_MAT_COL32) && nnz > 0) build_index16(m.get(), hp.data(), hc.data());
   if (flags & KS_MAT_FP32_COPY) ensure_fp32(m.get());
@@ -1053,7 +1152,7 @@ ks_status ks_mat_info(const ks_mat* m, int64_t* n, int64_t* nnz, int32_t* kind, 
   if (!m) return KS_ERR_BAD_INPUT;
   if (n) *n = m->n;
   if (nnz) *nnz = m->nnz;
-  if (kind) *kind = m->panels.np ? 3 : m->plan.kind;
+  if (kind) *kind = m->panels.np || m->bins.v.nblk ? 3 : m->plan.kind;
   if (lanes) *lanes = m->plan.L;
   return KS_OK;
 }
@@ -1313,7 +1412,13 @@ ks_status ks_sddmm(ks_mat* m, double alpha, const double* u, const double* v, do
   const int64_t nrb = (n + kBlock / L - 1) / (kBlock / L);
   const double bytes = 12.0 * m->nnz + 4.0 * (n + 1) + 16.0 * n;
   const int G = grid_rows(nrb);
-  switch (L) {
+  const BinView& B = m->bins.v;
+  if (B.nblk) {
+    launch_bin_gather<double>(c, B, n, vi.p, Gate{}, KS_K_OTHER);
+    const int Gb = grid_rows(std::min<int64_t>(B.nseg, resident(c, k_bin_sddmm, 0, kBinSum)));
+    klaunch_n<kBinSum>(c, KS_K_OTHER, k_bin_sddmm, Gb, B, m->ptr.p, alpha, ui.p, (const double*)B.xg, o.p,
+                       stat(c, KS_K_OTHER, 28.0 * m->nnz + 4.0 * (n + 1) + 16.0 * n));
+  } else switch (L) {
     case 2: k_sddmm<2><<<G, kBlock, 0, c->stream>>>(n, m->ptr.p, m->col.p, alpha, ui.p, vi.p, o.p, stat(c, KS_K_OTHER, bytes)); break;
     case 4: k_sddmm<4><<<G, kBlock, 0, c->stream>>>(n, m->ptr.p, m->col.p, alpha, ui.p, vi.p, o.p, stat(c, KS_K_OTHER, bytes)); break;
     case 8: k_sddmm<8><<<G, kBlock, 0, c->stream>>>(n, m->ptr.p, m->col.p, alpha, ui.p, vi.p, o.p, stat(c, KS_K_OTHER, bytes)); break;

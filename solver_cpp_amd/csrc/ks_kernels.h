@@ -153,11 +153,12 @@ __device__ inline double wave_sum(double v) {
 // are formed by k_finish, launched right after the producing kernel: the
 // kernel boundary orders the partials before their use, so no device-scope
 // fence (which on gfx950 writes back and invalidates the XCD's L2) is needed.
-template <int NV>
+// NT: the workgroup's threads.
+template <int NV, int NT = kBlock>
 __device__ void block_store(double (&acc)[NV], RedArgs ra) {
-  __shared__ double sw[NV][kBlock / 64];
+  __shared__ double sw[NV][NT / 64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  constexpr int nw = kBlock / 64;
+  constexpr int nw = NT / 64;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     double v = wave_sum(acc[i]);
