@@ -164,7 +164,8 @@ struct BinLoad {
   T x[U];
   int p[U];
   __device__ __forceinline__ static int at(int u, int cnt) { return min((int)threadIdx.x + u * kBinSum, cnt - 1); }
-  // run numbers first, then their shifts, then every entry
+  // run numbers first, then their shifts, then every entry.  Not for a
+  // segment without entries: it has no run, and no last place.
   __device__ __forceinline__ void load(const BinView& B, int64_t s, int32_t j0, int cnt, const T* __restrict__ xg) {
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint64_t* mask = B.mask + s * kBinWords + w;
@@ -258,10 +259,12 @@ __global__ __launch_bounds__(kBinSum) __attribute__((amdgpu_waves_per_eu(4))) vo
   for (; s < end; s += step) {
     const int32_t r0 = B.seg[s], r1 = B.seg[s + 1], j0 = B.snz[s], cnt = B.snz[s + 1] - j0;
     BinLoad<T> x;
-    x.load(B, s, j0, cnt, xg);
     T v[U];
+    if (cnt > 0) {
+      x.load(B, s, j0, cnt, xg);
 #pragma unroll
-    for (int u = 0; u < U; ++u) v[u] = ld_stream(val + j0 + BinLoad<T>::at(u, cnt));
+      for (int u = 0; u < U; ++u) v[u] = ld_stream(val + j0 + BinLoad<T>::at(u, cnt));
+    }
     x.stage(cnt, sp);
     __syncthreads();
 #pragma unroll
@@ -300,7 +303,7 @@ __global__ __launch_bounds__(kBinSum) __attribute__((amdgpu_waves_per_eu(4))) vo
   for (; s < end; s += step) {
     const int32_t r0 = B.seg[s], r1 = B.seg[s + 1], j0 = B.snz[s], cnt = B.snz[s + 1] - j0;
     BinLoad<double> x;
-    x.load(B, s, j0, cnt, xg);
+    if (cnt > 0) x.load(B, s, j0, cnt, xg);
     x.stage(cnt, sp);
     __syncthreads();
     for (int32_t rb = r0 + w; rb < r1; rb += kBinSum)

@@ -123,3 +123,18 @@ def test_solves(ctx, outer, inner, kw):
     (x, r, h), (y, s, g) = out
     assert r["status"] == s["status"] == 0 and abs(r["iters"] - s["iters"]) <= 1
     assert np.linalg.norm(x - y) <= 1e-10 * np.linalg.norm(y)
+
+
+@pytest.mark.parametrize("where", ["first", "middle", "last"])
+def test_segments_without_entries(ctx, where):
+    # two whole segments (4096 rows) of empty rows: they have no column block's run
+    n = 393216 + 5000
+    cnt = np.full(n, 28)
+    cnt[50000:52000] = np.random.default_rng(19).integers(0, 300, 2000)
+    cnt[60000] = 8000
+    at = dict(first=0, middle=200000, last=n - 9000)[where]
+    cnt[at:at + 9000] = 0
+    ptr = np.zeros(n + 1, np.int32)
+    ptr[1:] = np.cumsum(cnt)
+    rng = np.random.default_rng(20)
+    _check(ctx, ptr, rng.integers(0, n, ptr[-1]).astype(np.int32), rng.standard_normal(ptr[-1]), 3)
