@@ -18,6 +18,7 @@
 #include "../../include/ksolve.h"
 #include "ks_bins.h"
 #include "ks_coop.h"
+#include "ks_rows.h"
 #include "ks_kernels.h"
 
 namespace ks {
@@ -207,6 +208,10 @@ struct MatView {
   // instead of column indices and row pointers
   const PatIx* pat = nullptr;
   const int32_t* ptab = nullptr;
+  // row classes (RowIx): a byte per row, and the table with its values
+  const RowIx* row = nullptr;
+  const int32_t* rtab = nullptr;
+  const T* rval = nullptr;
   int ib = 4;
   const T* val = nullptr;
   int kind = 0;
@@ -239,6 +244,17 @@ struct MatView {
 // behind it (null: the side has none).
 struct PatBuf : DBuf<int32_t> {
   const PatIx* code = nullptr;
+};
+
+// Row classes (RowIx) of one side: the table at p, then its values in FP64 and
+// FP32, the state and the codes (null: the side has none).
+struct RowBuf : DBuf<int32_t> {
+  static constexpr int64_t kV64 = kRowTab, kV32 = kV64 + 2 * kRowMax * kRowLen, kState = kV32 + kRowMax * kRowLen;
+  static constexpr int64_t kHead = kState + (sizeof(PatState<kRowMax>) / 4 + 64) / 64 * 64;
+  RowIx* code = nullptr;
+  double* v64() const { return reinterpret_cast<double*>(p + kV64); }
+  float* v32() const { return reinterpret_cast<float*>(p + kV32); }
+  PatState<kRowMax>* state() const { return reinterpret_cast<PatState<kRowMax>*>(p + kState); }
 };
 
 // Column blocks and segments of one side (ks_bins.h).
@@ -280,6 +296,7 @@ struct ks_mat {
   ks::DBuf<int16_t> col16, tcol16;  // col - row of A and A^T (banded matrices)
   ks::DBuf<uint16_t> cold, tcold;   // delta-coded columns of A and A^T
   ks::PatBuf pat, tpat;             // row patterns of A and A^T
+  ks::RowBuf rows, trows;           // row classes of A and A^T
   ks::DBuf<double> val;
   ks::DBuf<float> val32;
   bool has_t = false;
@@ -301,6 +318,13 @@ struct ks_mat {
     const int16_t* p = trans ? tcol16.p : col16.p;
     const uint16_t* q = trans ? tcold.p : cold.p;
     const ks::PatBuf& r = trans ? tpat : pat;
+    const ks::RowBuf& w = trans ? trows : rows;
+    if (w.code) {
+      v.row = w.code;
+      v.rtab = w.p;
+      if constexpr (sizeof(T) == 8) v.rval = w.v64();
+      else v.rval = w.v32();
+    }
     if (r.code) { v.pat = r.code; v.ptab = r.p; v.ib = 2; }
     else if (p) { v.col16 = p; v.ib = 2; }
     else if (q) { v.cold = q; v.ib = 2; }
@@ -473,9 +497,11 @@ inline double spmv_bytes(int64_t n, int64_t nnz, int ib = 4) {
   return (double)(sizeof(T) + ib) * nnz + 4.0 * (n + 1) + 2.0 * sizeof(T) * n;
 }
 // the same in a view's index format (row patterns: a 2-byte code per row
-// instead of column indices and row pointers)
+// instead of column indices and row pointers; row classes: a byte per row
+// instead of the values as well)
 template <class T>
 inline double spmv_bytes(const MatView<T>& A) {
+  if (A.row) return 1.0 * A.n + 2.0 * sizeof(T) * A.n;
   if (A.pat) return (double)sizeof(T) * A.nnz + 2.0 * A.n + 2.0 * sizeof(T) * A.n;
   if (A.bins.nblk) return (3.0 * sizeof(T) + 4) * A.nnz + 4.0 * (A.n + 1) + 2.0 * sizeof(T) * A.n;
   return spmv_bytes<T>(A.n, A.nnz, A.ib);
@@ -500,7 +526,10 @@ int spmv_L(ks_ctx* c, const MatView<T>& A, const T* x, const Epi& epi, Gate g, i
 template <class T, int NX, int NV, class Epi>
 void launch_stream(ks_ctx* c, int cls, const MatView<T>& A, int G, const T* x0, const T* x1, const Epi& epi, Gate g,
                    double bytes) {
-  if (A.pat)
+  if (A.row)
+    klaunch(c, cls, k_spmv_rows<T, NX, NV, Epi>, G, 0, A.n, A.ntiles, A.tiles, A.rtab, A.row, A.rval, x0, x1, epi,
+             g, red(c), stat(c, cls, bytes));
+  else if (A.pat)
     klaunch(c, cls, k_spmv_stream<T, NX, NV, Epi, PatIx>, G, 0, A.n, A.ntiles, A.tiles, A.tnz, A.ptab, A.pat, A.val,
             x0, x1, epi, g, red(c), stat(c, cls, bytes));
   else if (A.col16)
@@ -517,6 +546,7 @@ void launch_stream(ks_ctx* c, int cls, const MatView<T>& A, int G, const T* x0, 
 template <class T, int NX, int NV, class Epi>
 int stream_grid(ks_ctx* c, const MatView<T>& A) {
   if constexpr (NV == 0 && !HasProj<Epi>::value) {
+    if (A.row) return grid_rows(c, k_spmv_rows<T, NX, NV, Epi>, A.ntiles);
     if (A.pat) return grid_rows(c, k_spmv_stream<T, NX, NV, Epi, PatIx>, A.ntiles);
     if (A.col16) return grid_rows(c, k_spmv_stream<T, NX, NV, Epi, int16_t>, A.ntiles);
     if (A.cold) return grid_rows(c, k_spmv_stream<T, NX, NV, Epi, uint16_t>, A.ntiles);

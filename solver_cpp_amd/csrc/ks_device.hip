@@ -332,12 +332,12 @@ bool build_patterns(ks_mat* m, const Plan& pl, PatBuf& pat, const int32_t* ptr, 
   if (pl.kind != 0 || !(pl.wg64 || pl.wg32) || pl.wg.long_rows) return false;
   ks_ctx* c = m->ctx;
   hipStream_t s = c->stream;
-  constexpr int64_t head = kPatTab + pad64(sizeof(PatState) / 4 + 1);
+  constexpr int64_t head = kPatTab + pad64(sizeof(PatState<kPatMax>) / 4 + 1);
   pat.alloc(head + (m->n + 1) / 2);
-  PatState* st = reinterpret_cast<PatState*>(pat.p + kPatTab);
+  auto* st = reinterpret_cast<PatState<kPatMax>*>(pat.p + kPatTab);
   k_fill<int32_t><<<1, kBlock, 0, s>>>(head, pat.p, 0);
-  k_pat_find<<<grid_map(m->n), kBlock, 0, s>>>(m->n, ptr, col, st);
-  k_pat_table<<<1, kPatSlots, 0, s>>>(st, ptr, col, pat.p);
+  k_pat_find<kPatMax><<<grid_map(m->n), kBlock, 0, s>>>(m->n, ptr, col, nullptr, st);
+  k_pat_table<kPatMax><<<1, 2 * kPatMax, 0, s>>>(st, ptr, col, pat.p);
   k_pat_codes<<<(unsigned)pl.wg.ntiles, kBlock, 0, s>>>(st, pat.p, pl.wg.tiles.p, pl.wg.tnz.p, ptr, col,
                                                         reinterpret_cast<PatIx*>(pat.p + head));
   KS_HIPCK(hipGetLastError());
@@ -349,25 +349,69 @@ bool build_patterns(ks_mat* m, const Plan& pl, PatBuf& pat, const int32_t* ptr, 
   return !bad;
 }
 
+// Row classes (RowIx) of the CSR (ptr, col, val) with plan pl, under
+// build_patterns' conditions, for matrices of kRowMinNnz entries or more.  Not
+// for a borrowed matrix, whose values the caller may change in place.
+void build_rows(ks_mat* m, const Plan& pl, RowBuf& rows, const int32_t* ptr, const int32_t* col, const double* val) {
+  if (pl.kind != 0 || !(pl.wg64 || pl.wg32) || pl.wg.long_rows || m->nnz < kRowMinNnz || m->n > kRowMaxN ||
+      (m->flags & KS_MAT_BORROW))
+    return;
+  ks_ctx* c = m->ctx;
+  hipStream_t s = c->stream;
+  rows.alloc(RowBuf::kHead + (m->n + 3) / 4);
+  PatState<kRowMax>* st = rows.state();
+  RowIx* code = reinterpret_cast<RowIx*>(rows.p + RowBuf::kHead);
+  k_fill<int32_t><<<1, kBlock, 0, s>>>(RowBuf::kHead, rows.p, 0);
+  k_pat_find<kRowMax><<<grid_map(m->n), kBlock, 0, s>>>(m->n, ptr, col, val, st);
+  k_pat_table<kRowMax><<<1, 2 * kRowMax, 0, s>>>(st, ptr, col, rows.p);
+  k_row_codes<<<grid_map(m->n), kBlock, 0, s>>>(m->n, st, ptr, col, val, code);
+  k_row_vals<<<1, kRowMax, 0, s>>>(st, rows.p, ptr, val, rows.v64(), rows.v32());
+  KS_HIPCK(hipGetLastError());
+  int bad = 0;
+  KS_HIPCK(hipMemcpyAsync(&bad, &st->bad, sizeof(int), hipMemcpyDeviceToHost, s));
+  KS_HIPCK(hipStreamSynchronize(s));
+  if (bad) rows.release();
+  else rows.code = code;
+}
+
+// New values: refreshes a side's classes; *bad (after the stream's next
+// synchronisation) tells whether its rows no longer agree (drop_rows).
+void refresh_rows(ks_mat* m, RowBuf& rows, const int32_t* ptr, const double* val, int* bad) {
+  if (!rows.code) return;
+  hipStream_t s = m->ctx->stream;
+  k_row_check<<<grid_map(m->n), kBlock, 0, s>>>(m->n, rows.state(), ptr, val, rows.code);
+  k_row_vals<<<1, kRowMax, 0, s>>>(rows.state(), rows.p, ptr, val, rows.v64(), rows.v32());
+  KS_HIPCK(hipGetLastError());
+  KS_HIPCK(hipMemcpyAsync(bad, &rows.state()->bad, sizeof(int), hipMemcpyDeviceToHost, s));
+}
+void drop_rows(RowBuf& rows, int bad) {
+  if (!bad) return;
+  rows.code = nullptr;
+  rows.release();
+}
+
 // The SpMV's 16-bit column indices of A and A^T, unless KS_MAT_COL32: row
 // patterns where they apply (not with KS_MAT_COL_DELTA), else int16 offsets
 // when every offset fits (hp, hc: A's host row pointers and columns; A^T's
 // offsets are A's negated, so both fit), delta-coded columns where those
-// apply, in the order KS_MAT_COL_DELTA asks for; int32 columns otherwise, and
+// apply, in the order KS_MAT_COL_DELTA asks for, and with the first two the
+// row classes, where those apply (the others are what new values fall back to); int32 columns otherwise, and
 // for a side whose SpMV runs on column panels (which read int32 columns).
 void build_index16(ks_mat* m, const int32_t* hp, const int32_t* hc) {
   const bool delta_first = (m->flags & KS_MAT_COL_DELTA) != 0;
   int off16 = -1;  // not looked at yet
-  auto side = [&](PatBuf& op, DBuf<int16_t>& o16, DBuf<uint16_t>& od, const Plan& pl,
-                  const PanelSet& ps, const int32_t* ptr, const int32_t* col) {
+  auto side = [&](RowBuf& rows, PatBuf& op, DBuf<int16_t>& o16, DBuf<uint16_t>& od, const Plan& pl,
+                  const PanelSet& ps, const int32_t* ptr, const int32_t* col, const double* val) {
     if (ps.np || pl.kind != 0) return;
+    if (!delta_first) build_rows(m, pl, rows, ptr, col, val);
     if (!delta_first && build_patterns(m, pl, op, ptr, col)) return;
     if (off16 < 0) off16 = offsets_fit16(m->n, hp, hc);
     if (off16 && !delta_first) build_col16(m, o16, ptr, col);
     else if (!build_col_delta(m, pl, od, ptr, col) && off16) build_col16(m, o16, ptr, col);
   };
-  side(m->pat, m->col16, m->cold, m->plan, m->panels, m->ptr.p, m->col.p);
-  if (m->has_t) side(m->tpat, m->tcol16, m->tcold, m->tplan, m->tpanels, m->tptr.p, m->tcol.p);
+  side(m->rows, m->pat, m->col16, m->cold, m->plan, m->panels, m->ptr.p, m->col.p, m->val.p);
+  if (m->has_t)
+    side(m->trows, m->tpat, m->tcol16, m->tcold, m->tplan, m->tpanels, m->tptr.p, m->tcol.p, m->tval.p);
 }
 
 // Bytes per column index of the entry format that a side with row patterns
@@ -1111,6 +1155,9 @@ ks_status ks_mat_update_values(ks_mat* m, const double* val, uint32_t flags) {
   }
   refresh_panels(m, m->panels);
   refresh_panels(m, m->tpanels);
+  int bad = 0, tbad = 0;
+  refresh_rows(m, m->rows, m->ptr.p, m->val.p, &bad);
+  refresh_rows(m, m->trows, m->tptr.p, m->tval.p, &tbad);
   if (m->val32.p) {
     k_convert<double, float><<<grid_map(m->nnz), kBlock, 0, c->stream>>>(m->nnz, m->val.p, m->val32.p, Gate{});
     KS_HIPCK(hipGetLastError());
@@ -1120,6 +1167,8 @@ ks_status ks_mat_update_values(ks_mat* m, const double* val, uint32_t flags) {
     KS_HIPCK(hipGetLastError());
   }
   KS_HIPCK(hipStreamSynchronize(c->stream));
+  drop_rows(m->rows, bad);
+  drop_rows(m->trows, tbad);
   return KS_OK;
   KS_API_CATCH(c)
 }

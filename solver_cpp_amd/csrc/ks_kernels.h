@@ -541,6 +541,15 @@ struct PatTile {
     else load<false>(ptr, code, val, r0, r1, j0, j1, nnz, t);
   }
 };
+// Row classes: see ks_rows.h.
+struct RowIx {
+  uint8_t v;
+};
+constexpr int kRowMax = 128;  // classes
+constexpr int kRowLen = 8;    // entries of a row
+// table: the offsets, the lengths, the greatest length
+constexpr int kRowTab = kRowMax * (kRowLen + 1) + 2;
+
 template <class T, class IX>
 struct TileOf {
   using type = TileData<T, IX>;
@@ -568,6 +577,141 @@ template <class E, class = void>
 struct HasProj : std::false_type {};
 template <class E>
 struct HasProj<E, std::void_t<decltype(E::kProj)>> : std::true_type {};
+
+// Classical Gram-Schmidt projection fused behind the SpMV: the partial
+// dots (y, V_v) over this workgroup's own rows, which it has just
+// written (visible to the whole workgroup after the loop's last
+// barrier; still in this XCD's L2), so y is not read back from HBM and
+// no separate projection launch runs.  The four wavefronts split the
+// work by columns and by tiles: gc column groups of cpg = nv / gc
+// columns (gc = 1, 2 or 4, the fewest with cpg <= CP when possible),
+// each taken by 4 / gc wavefronts that split the workgroup's tiles
+// among them (every (4/gc)-th tile), CP columns per pass, with the next
+// tile's bounds loaded while the current one is summed.  So every
+// wavefront has work at every column count, and a tile costs one round
+// trip per pass.  Rows are read in 16-byte chunks (y, V and ldv 16-byte
+// aligned, checked by the host; a tile of <= 256 rows is at most NCH
+// chunks per lane), a tile's rows outside its aligned chunks one per
+// lane.  Per pass the sums of a column's wavefronts are added in a
+// fixed order through LDS and written to part[v * kMaxGrid + workgroup].
+// sy: the y of the workgroup's first YT tiles (tile s at sy[s][row - (r0 & ~3)]).
+template <class T, int YT, int YW, class Epi>
+__device__ __forceinline__ void proj_tiles(const int32_t* __restrict__ tiles, const RowBlocks& rbs, const T (*sy)[YW],
+                                           const Epi& epi, const RedArgs& ra) {
+  constexpr int kYT = YT;
+  const int tid = threadIdx.x;
+  using VT = typename Chunk<T, 16 / sizeof(T)>::type;
+  constexpr int W = 16 / sizeof(T);
+  constexpr int kW = kBlock / 64;
+  static_assert(kW == 4, "four wavefronts per workgroup");
+  constexpr int CP = sizeof(T) == 4 ? 6 : 4;   // columns per pass (the most without spills)
+  constexpr int NCH = kTileRows / (64 * W);     // aligned chunks per lane per tile
+  __shared__ double sred[kW][CP];
+  // the wavefront index is uniform across the wavefront: scalar registers
+  // for the tile loop and its bounds
+  const int lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int64_t u0, uend, ustep;
+  rbs.range(u0, uend, ustep);
+  const int nv = epi.nv;
+  const int64_t ldv = epi.ldv;
+  const int gc = nv <= CP ? 1 : nv <= 2 * CP ? 2 : 4;
+  const int gt = kW / gc, cpg = (nv + gc - 1) / gc;
+  const int cbeg = (wv / gt) * cpg, cend = min(nv, cbeg + cpg);
+  const int64_t ws = (int64_t)gt * ustep;
+  // at least one pass: its column group 0 also writes the staged y out
+  for (int p0 = 0; p0 == 0 || p0 < cpg; p0 += CP) {
+    const int c0 = cbeg + p0;  // columns c0 + j < cend in this pass
+    double pa[CP];
+#pragma unroll
+    for (int j = 0; j < CP; ++j) pa[j] = 0.0;
+    const T* vb = epi.V + (int64_t)c0 * ldv;
+    int64_t u = u0 + (int64_t)(wv % gt) * ustep;
+    int ti = wv % gt;  // the tile's index among the workgroup's tiles
+    int64_t q0 = 0, q1 = 0;
+    if (u < uend) { q0 = tiles[u]; q1 = tiles[u + 1]; }
+    // one tile: y from LDS (a staged tile, kStaged) or from memory; the
+    // staged tiles come first in every wavefront's order, so two loops
+    // keep each load in one address space
+    auto tile = [&](auto staged_tag) {
+      constexpr bool kStaged = decltype(staged_tag)::value;
+      int64_t n0 = 0, n1 = 0;
+      if (u + ws < uend) { n0 = tiles[u + ws]; n1 = tiles[u + ws + 1]; }
+      const int64_t a = (q0 + W - 1) / W * W, b = q1 / W * W;
+      const int64_t base = q0 & ~(int64_t)3;
+      const T* ys = nullptr;  // row r of a staged tile at ys[r - base]
+      if constexpr (kStaged) {
+        ys = sy[ti];
+        if (p0 == 0 && wv < gt)
+          for (int64_t j = q0 + lane; j < q1; j += 64) epi.y[j] = ys[j - base];
+      }
+      {
+        VT yv[NCH], xv[NCH][CP];
+#pragma unroll
+        for (int h = 0; h < NCH; ++h) {
+          const int64_t r = a + (int64_t)W * (lane + 64 * h);
+          if (r + W <= b) {
+            if constexpr (kStaged) yv[h] = *reinterpret_cast<const VT*>(ys + (r - base));
+            else yv[h] = *reinterpret_cast<const VT*>(epi.y + r);
+#pragma unroll
+            for (int j = 0; j < CP; ++j)
+              if (c0 + j < cend) xv[h][j] = *reinterpret_cast<const VT*>(vb + (int64_t)j * ldv + r);
+          }
+        }
+#pragma unroll
+        for (int h = 0; h < NCH; ++h) {
+          const int64_t r = a + (int64_t)W * (lane + 64 * h);
+          if (r + W <= b) {
+#pragma unroll
+            for (int j = 0; j < CP; ++j)
+              if (c0 + j < cend) {
+                double t = 0.0;
+#pragma unroll
+                for (int e = 0; e < W; ++e) t += (double)yv[h][e] * (double)xv[h][j][e];
+                pa[j] += t;
+              }
+          }
+        }
+      }
+      // rows before the first and after the last aligned chunk (< 2W; none
+      // on tiles with chunk-aligned bounds), after the chunks
+      const int64_t hn = (a < q1 ? a : q1) - q0;
+      const int64_t tb = b > a ? b : a;
+      int64_t row = -1;
+      if (lane < hn) row = q0 + lane;
+      else if (lane >= W && lane - W < q1 - tb) row = tb + (lane - W);
+      if (row >= 0) {
+        double ye;
+        if constexpr (kStaged) ye = (double)ys[row - base];
+        else ye = (double)epi.y[row];
+#pragma unroll
+        for (int j = 0; j < CP; ++j)
+          if (c0 + j < cend) pa[j] += ye * (double)vb[(int64_t)j * ldv + row];
+      }
+      q0 = n0; q1 = n1;
+    };
+    if constexpr (kYT > 0)
+      for (; u < uend && ti < kYT; u += ws, ti += gt) tile(std::true_type{});
+    for (; u < uend; u += ws, ti += gt) tile(std::false_type{});
+#pragma unroll
+    for (int j = 0; j < CP; ++j) {
+      const double v = wave_sum(pa[j]);
+      if (lane == 0) sred[wv][j] = v;
+    }
+    __syncthreads();
+    if (tid < gc * CP) {
+      const int g = tid / CP, j = tid % CP, c = g * cpg + p0 + j;
+      if (p0 + j < cpg && c < nv) {
+        const double* q = &sred[g * gt][j];
+        double t;
+        if (gt == 4) t = (q[0] + q[CP]) + (q[2 * CP] + q[3 * CP]);
+        else if (gt == 2) t = q[0] + q[CP];
+        else t = q[0];
+        ra.part[(size_t)c * kMaxGrid + blockIdx.x] = t;
+      }
+    }
+    __syncthreads();
+  }
+}
 
 // IX = int16_t: the column index arrives as the offset col - row (every
 // offset of the matrix in [-32767, 32767]; stencil and other banded
@@ -797,134 +941,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kWgWaves
   }
   if constexpr (NV > 0) block_store<NV>(acc, ra);
   if constexpr (HasProj<Epi>::value) {
-    // Classical Gram-Schmidt projection fused behind the SpMV: the partial
-    // dots (y, V_v) over this workgroup's own rows, which it has just
-    // written (visible to the whole workgroup after the loop's last
-    // barrier; still in this XCD's L2), so y is not read back from HBM and
-    // no separate projection launch runs.  The four wavefronts split the
-    // work by columns and by tiles: gc column groups of cpg = nv / gc
-    // columns (gc = 1, 2 or 4, the fewest with cpg <= CP when possible),
-    // each taken by 4 / gc wavefronts that split the workgroup's tiles
-    // among them (every (4/gc)-th tile), CP columns per pass, with the next
-    // tile's bounds loaded while the current one is summed.  So every
-    // wavefront has work at every column count, and a tile costs one round
-    // trip per pass.  Rows are read in 16-byte chunks (y, V and ldv 16-byte
-    // aligned, checked by the host; a tile of <= 256 rows is at most NCH
-    // chunks per lane), a tile's rows outside its aligned chunks one per
-    // lane.  Per pass the sums of a column's wavefronts are added in a
-    // fixed order through LDS and written to part[v * kMaxGrid + workgroup].
     static_assert(NV == 0 && NX == 1, "projection epilogue takes a plain SpMV");
-    using VT = typename Chunk<T, 16 / sizeof(T)>::type;
-    constexpr int W = 16 / sizeof(T);
-    constexpr int kW = kBlock / 64;
-    static_assert(kW == 4, "four wavefronts per workgroup");
-    constexpr int CP = sizeof(T) == 4 ? 6 : 4;   // columns per pass (the most without spills)
-    constexpr int NCH = kTileRows / (64 * W);     // aligned chunks per lane per tile
-    __shared__ double sred[kW][CP];
-    // the wavefront index is uniform across the wavefront: scalar registers
-    // for the tile loop and its bounds
-    const int lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    int64_t u0, uend, ustep;
-    rbs.range(u0, uend, ustep);
-    const int nv = epi.nv;
-    const int64_t ldv = epi.ldv;
-    const int gc = nv <= CP ? 1 : nv <= 2 * CP ? 2 : 4;
-    const int gt = kW / gc, cpg = (nv + gc - 1) / gc;
-    const int cbeg = (wv / gt) * cpg, cend = min(nv, cbeg + cpg);
-    const int64_t ws = (int64_t)gt * ustep;
-    // at least one pass: its column group 0 also writes the staged y out
-    for (int p0 = 0; p0 == 0 || p0 < cpg; p0 += CP) {
-      const int c0 = cbeg + p0;  // columns c0 + j < cend in this pass
-      double pa[CP];
-#pragma unroll
-      for (int j = 0; j < CP; ++j) pa[j] = 0.0;
-      const T* vb = epi.V + (int64_t)c0 * ldv;
-      int64_t u = u0 + (int64_t)(wv % gt) * ustep;
-      int ti = wv % gt;  // the tile's index among the workgroup's tiles
-      int64_t q0 = 0, q1 = 0;
-      if (u < uend) { q0 = tiles[u]; q1 = tiles[u + 1]; }
-      // one tile: y from LDS (a staged tile, kStaged) or from memory; the
-      // staged tiles come first in every wavefront's order, so two loops
-      // keep each load in one address space
-      auto tile = [&](auto staged_tag) {
-        constexpr bool kStaged = decltype(staged_tag)::value;
-        int64_t n0 = 0, n1 = 0;
-        if (u + ws < uend) { n0 = tiles[u + ws]; n1 = tiles[u + ws + 1]; }
-        const int64_t a = (q0 + W - 1) / W * W, b = q1 / W * W;
-        const int64_t base = q0 & ~(int64_t)3;
-        const T* ys = nullptr;  // row r of a staged tile at ys[r - base]
-        if constexpr (kStaged) {
-          ys = sy[ti];
-          if (p0 == 0 && wv < gt)
-            for (int64_t j = q0 + lane; j < q1; j += 64) epi.y[j] = ys[j - base];
-        }
-        {
-          VT yv[NCH], xv[NCH][CP];
-#pragma unroll
-          for (int h = 0; h < NCH; ++h) {
-            const int64_t r = a + (int64_t)W * (lane + 64 * h);
-            if (r + W <= b) {
-              if constexpr (kStaged) yv[h] = *reinterpret_cast<const VT*>(ys + (r - base));
-              else yv[h] = *reinterpret_cast<const VT*>(epi.y + r);
-#pragma unroll
-              for (int j = 0; j < CP; ++j)
-                if (c0 + j < cend) xv[h][j] = *reinterpret_cast<const VT*>(vb + (int64_t)j * ldv + r);
-            }
-          }
-#pragma unroll
-          for (int h = 0; h < NCH; ++h) {
-            const int64_t r = a + (int64_t)W * (lane + 64 * h);
-            if (r + W <= b) {
-#pragma unroll
-              for (int j = 0; j < CP; ++j)
-                if (c0 + j < cend) {
-                  double t = 0.0;
-#pragma unroll
-                  for (int e = 0; e < W; ++e) t += (double)yv[h][e] * (double)xv[h][j][e];
-                  pa[j] += t;
-                }
-            }
-          }
-        }
-        // rows before the first and after the last aligned chunk (< 2W; none
-        // on tiles with chunk-aligned bounds), after the chunks
-        const int64_t hn = (a < q1 ? a : q1) - q0;
-        const int64_t tb = b > a ? b : a;
-        int64_t row = -1;
-        if (lane < hn) row = q0 + lane;
-        else if (lane >= W && lane - W < q1 - tb) row = tb + (lane - W);
-        if (row >= 0) {
-          double ye;
-          if constexpr (kStaged) ye = (double)ys[row - base];
-          else ye = (double)epi.y[row];
-#pragma unroll
-          for (int j = 0; j < CP; ++j)
-            if (c0 + j < cend) pa[j] += ye * (double)vb[(int64_t)j * ldv + row];
-        }
-        q0 = n0; q1 = n1;
-      };
-      if constexpr (kYT > 0)
-        for (; u < uend && ti < kYT; u += ws, ti += gt) tile(std::true_type{});
-      for (; u < uend; u += ws, ti += gt) tile(std::false_type{});
-#pragma unroll
-      for (int j = 0; j < CP; ++j) {
-        const double v = wave_sum(pa[j]);
-        if (lane == 0) sred[wv][j] = v;
-      }
-      __syncthreads();
-      if (tid < gc * CP) {
-        const int g = tid / CP, j = tid % CP, c = g * cpg + p0 + j;
-        if (p0 + j < cpg && c < nv) {
-          const double* q = &sred[g * gt][j];
-          double t;
-          if (gt == 4) t = (q[0] + q[CP]) + (q[2 * CP] + q[3 * CP]);
-          else if (gt == 2) t = q[0] + q[CP];
-          else t = q[0];
-          ra.part[(size_t)c * kMaxGrid + blockIdx.x] = t;
-        }
-      }
-      __syncthreads();
-    }
+    proj_tiles<T, kYT, kYW>(tiles, rbs, sy, epi, ra);
   }
 }
 
@@ -1941,48 +1959,59 @@ __global__ void k_col_delta(int64_t n, const int32_t* __restrict__ ptr, const in
   }
 }
 
-// Row patterns (PatIx), built by three kernels with no host step between
-// them.  k_pat_find enters every row's pattern hash in an open-addressing
-// table of kPatSlots slots (key 0: free; rep: a row with that key).
-// k_pat_table numbers the patterns by hash and writes the pattern table from
-// their rows.  k_pat_codes writes the row codes and compares every row with
-// its pattern entry by entry (two patterns of one hash).  Each sets `bad`
-// when the format does not apply, which ends the later ones.
-constexpr int kPatSlots = 2 * kPatMax;
+// Row patterns (PatIx, M = kPatMax) and row classes (RowIx, M = kRowMax: the
+// rows' values, compared bit for bit, belong to the pattern), built by three
+// kernels with no host step between them.  k_pat_find enters every row's hash
+// in an open-addressing table of 2 M slots (key 0: free; rep: a row with that
+// key).  k_pat_table numbers the patterns by hash and writes the pattern table
+// from their rows.  k_pat_codes / k_row_codes write the row codes and compare
+// every row with its pattern entry by entry (two patterns of one hash).  Each
+// sets `bad` when the format does not apply, which ends the later ones.
+template <int M>
 struct PatState {
-  unsigned long long key[kPatSlots];
-  int32_t rep[kPatSlots];
-  unsigned long long hash[kPatMax];  // by pattern number
+  unsigned long long key[2 * M];
+  int32_t rep[2 * M];
+  unsigned long long hash[M];  // by pattern number
+  int32_t row[M];              // a row of it
   int P, bad;
 };
-__device__ inline uint64_t pat_hash(const int32_t* __restrict__ col, int32_t a, int32_t e, int32_t r) {
+template <int M>
+__device__ inline uint64_t pat_hash(const int32_t* __restrict__ col, const double* __restrict__ val, int32_t a,
+                                    int32_t e, int32_t r) {
   uint64_t h = 0x9e3779b97f4a7c15ull + (uint64_t)(e - a);
-  for (int32_t j = a; j < e; ++j) {
-    h ^= (uint32_t)(col[j] - r);
+  auto mix = [&](uint64_t v) {
+    h ^= v;
     h *= 0xff51afd7ed558ccdull;
     h ^= h >> 32;
+  };
+  for (int32_t j = a; j < e; ++j) {
+    mix((uint32_t)(col[j] - r));
+    if constexpr (M == kRowMax) mix(__builtin_bit_cast(uint64_t, val[j]));
   }
   return h ? h : 1;
 }
-__global__ void k_pat_find(int64_t n, const int32_t* __restrict__ ptr, const int32_t* __restrict__ col, PatState* st) {
+template <int M>
+__global__ void k_pat_find(int64_t n, const int32_t* __restrict__ ptr, const int32_t* __restrict__ col,
+                           const double* __restrict__ val, PatState<M>* st) {
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r < n; r += stride) {
     if (*(volatile int*)&st->bad) return;
     const int32_t a = ptr[r], e = ptr[r + 1];
-    if (e - a > kPatTab - 1 - kPatMax) { st->bad = 1; return; }
-    const unsigned long long h = pat_hash(col, a, e, (int32_t)r);
-    int s = (int)(h % kPatSlots), tries = 0;
-    for (; tries < kPatSlots; ++tries, s = (s + 1) % kPatSlots) {
+    if (e - a > (M == kRowMax ? kRowLen : kPatTab - 1 - M)) { st->bad = 1; return; }
+    const unsigned long long h = pat_hash<M>(col, val, a, e, (int32_t)r);
+    int s = (int)(h % (2 * M)), tries = 0;
+    for (; tries < 2 * M; ++tries, s = (s + 1) % (2 * M)) {
       unsigned long long k = *(volatile unsigned long long*)(st->key + s);
       if (k == 0) k = atomicCAS(st->key + s, 0ull, h);  // the key that was there
       if (k == 0) st->rep[s] = (int32_t)r;              // this row entered it
       if (k == 0 || k == h) break;
     }
-    if (tries == kPatSlots) { st->bad = 1; return; }
+    if (tries == 2 * M) { st->bad = 1; return; }
   }
 }
-// one workgroup of kPatSlots threads
-__global__ void k_pat_table(PatState* st, const int32_t* __restrict__ ptr, const int32_t* __restrict__ col,
+// one workgroup of 2 M threads
+template <int M>
+__global__ void k_pat_table(PatState<M>* st, const int32_t* __restrict__ ptr, const int32_t* __restrict__ col,
                             int32_t* tab) {
   __shared__ int s_stride, s_P;
   if (st->bad) return;
@@ -1996,24 +2025,31 @@ __global__ void k_pat_table(PatState* st, const int32_t* __restrict__ ptr, const
     r = st->rep[s];
     a = ptr[r];
     len = ptr[r + 1] - a;
-    for (int q = 0; q < kPatSlots; ++q) p += st->key[q] && st->key[q] < k;
+    for (int q = 0; q < 2 * M; ++q) p += st->key[q] && st->key[q] < k;
     atomicMax(&s_stride, len);
     atomicAdd(&s_P, 1);
   }
   __syncthreads();
   const int P = s_P, stride = s_stride;
-  if (P > kPatMax || 1 + kPatMax + P * stride > kPatTab) {
+  const bool fits = M == kRowMax ? stride <= kRowLen : 1 + M + P * stride <= kPatTab;
+  if (P > M || !fits) {
     if (s == 0) st->bad = 1;
     return;
   }
-  if (s == 0) { tab[0] = stride; st->P = P; }
-  if (!k) return;
-  st->hash[p] = k;
-  tab[1 + p] = len;
-  for (int j = 0; j < len; ++j) tab[1 + kPatMax + p * stride + j] = col[a + j] - r;
+  if (s == 0) st->P = P;
+  if (k) { st->hash[p] = k; st->row[p] = r; }
+  if constexpr (M == kRowMax) {
+    if (k)
+      for (int j = 0; j < len; ++j) tab[p * kRowLen + j] = col[a + j] - r;
+  } else {
+    if (s == 0) tab[0] = stride;
+    if (!k) return;
+    tab[1 + p] = len;
+    for (int j = 0; j < len; ++j) tab[1 + M + p * stride + j] = col[a + j] - r;
+  }
 }
 // one workgroup per tile
-__global__ __launch_bounds__(kBlock) void k_pat_codes(PatState* st, const int32_t* __restrict__ tab,
+__global__ __launch_bounds__(kBlock) void k_pat_codes(PatState<kPatMax>* st, const int32_t* __restrict__ tab,
                                                       const int32_t* __restrict__ tiles,
                                                       const int32_t* __restrict__ tnz,
                                                       const int32_t* __restrict__ ptr,
@@ -2023,13 +2059,65 @@ __global__ __launch_bounds__(kBlock) void k_pat_codes(PatState* st, const int32_
   const int32_t r = tiles[t] + (int32_t)threadIdx.x, a0 = PatTile<double>::a0of(tnz[t]);
   if (r >= tiles[t + 1]) return;
   const int32_t a = ptr[r], e = ptr[r + 1], P = st->P;
-  const uint64_t h = pat_hash(col, a, e, r);
+  const uint64_t h = pat_hash<kPatMax>(col, nullptr, a, e, r);
   int p = 0;
   while (p < P && st->hash[p] != h) ++p;
   bool ok = p < P && tab[1 + p] == e - a;
   for (int32_t j = a; ok && j < e; ++j) ok = tab[1 + kPatMax + p * tab[0] + (j - a)] == col[j] - r;
   if (!ok) { st->bad = 1; return; }
   code[r].v = (uint16_t)(p << kPatShift | (a - a0));
+}
+__device__ inline bool same_bits(double a, double b) {
+  return __builtin_bit_cast(uint64_t, a) == __builtin_bit_cast(uint64_t, b);
+}
+__global__ void k_row_codes(int64_t n, PatState<kRowMax>* st, const int32_t* __restrict__ ptr,
+                            const int32_t* __restrict__ col, const double* __restrict__ val, RowIx* code) {
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r < n; r += stride) {
+    if (*(volatile int*)&st->bad) return;
+    const int32_t a = ptr[r], e = ptr[r + 1], P = st->P;
+    const uint64_t h = pat_hash<kRowMax>(col, val, a, e, (int32_t)r);
+    int p = 0;
+    while (p < P && st->hash[p] != h) ++p;
+    const int32_t q = p < P ? st->row[p] : 0, b = ptr[q];
+    bool ok = p < P && ptr[q + 1] - b == e - a;
+    for (int32_t j = 0; ok && j < e - a; ++j)
+      ok = col[a + j] - (int32_t)r == col[b + j] - q && same_bits(val[a + j], val[b + j]);
+    if (!ok) { st->bad = 1; return; }
+    code[r].v = (uint8_t)p;
+  }
+}
+// New values in the same pattern: do the rows of a class still agree?
+__global__ void k_row_check(int64_t n, PatState<kRowMax>* st, const int32_t* __restrict__ ptr,
+                            const double* __restrict__ val, const RowIx* __restrict__ code) {
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r < n; r += stride) {
+    if (*(volatile int*)&st->bad) return;
+    const int32_t a = ptr[r], e = ptr[r + 1], b = ptr[st->row[code[r].v]];
+    bool ok = true;
+    for (int32_t j = 0; j < e - a; ++j) ok &= same_bits(val[a + j], val[b + j]);
+    if (!ok) st->bad = 1;
+  }
+}
+// The table's values and lengths; one workgroup of kRowMax threads.
+__global__ void k_row_vals(const PatState<kRowMax>* st, int32_t* tab, const int32_t* __restrict__ ptr,
+                           const double* __restrict__ val, double* v64, float* v32) {
+  __shared__ int most;
+  const int p = threadIdx.x;
+  if (st->bad) return;
+  if (p == 0) most = 0;
+  __syncthreads();
+  if (p < st->P) {
+    const int32_t a = ptr[st->row[p]], len = ptr[st->row[p] + 1] - a;
+    for (int j = 0; j < len; ++j) {
+      v64[p * kRowLen + j] = val[a + j];
+      v32[p * kRowLen + j] = (float)val[a + j];
+    }
+    tab[kRowMax * kRowLen + p] = len;
+    atomicMax(&most, len);
+  }
+  __syncthreads();
+  if (p == 0) tab[kRowTab - 1] = most;
 }
 
 // out[0..m) = v: clears memory with a kernel (no memset node), for state
