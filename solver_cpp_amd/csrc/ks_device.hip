@@ -812,18 +812,14 @@ double resid_norm(ks_ctx* c, ks_mat* m, bool trans, const double* b, const doubl
   else
     r.alloc(m->n);
   auto A = m->view<double>(trans && m->has_t);
-  launch_spmv<double, 1>(c, A, x, EpiResid<double, FinStore>{b, r.p, FinStore{c->scal.p + 1, 1}}, Gate{}, 8.0 * m->n);
-  double v = 0;
-  KS_HIPCK(hipMemcpyAsync(&v, c->scal.p + 1, sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  launch_spmv<double, 1>(c, A, x, EpiResid<double, FinStore>{b, r.p, FinStore{c->hscal_dev + 1, 1}}, Gate{}, 8.0 * m->n);
   KS_HIPCK(hipStreamSynchronize(c->stream));
-  return v;
+  return c->hscal[1];
 }
 double norm_dev(ks_ctx* c, int64_t n, const double* x) {
-  launch_map<1>(c, n, OpDot<double>{x, x, c->scal.p + 2, 1}, Gate{}, KS_K_REDUCE, 8.0 * n);
-  double v = 0;
-  KS_HIPCK(hipMemcpyAsync(&v, c->scal.p + 2, sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  launch_map<1>(c, n, OpDot<double>{x, x, c->hscal_dev + 2, 1}, Gate{}, KS_K_REDUCE, 8.0 * n);
   KS_HIPCK(hipStreamSynchronize(c->stream));
-  return v;
+  return c->hscal[2];
 }
 
 int64_t total_inner_steps(Level& L) {
@@ -1010,10 +1006,11 @@ ks_status ks_ctx_create(int32_t device, ks_ctx** out) {
     c->stats.alloc(2 * KS_K_NCLASS + 1);
     c->coop.alloc(kCoopSlots);
     coop_reset(c);
-    c->scal.alloc(1024);
     KS_HIPCK(hipHostMalloc((void**)&c->hflags, 64 * sizeof(int), hipHostMallocMapped));
     std::memset(c->hflags, 0, 64 * sizeof(int));
     KS_HIPCK(hipHostGetDevicePointer((void**)&c->hflags_dev, c->hflags, 0));
+    c->hscal = reinterpret_cast<double*>(c->hflags + 32);
+    c->hscal_dev = reinterpret_cast<double*>(c->hflags_dev + 32);
     hipDeviceProp_t prop;
     KS_HIPCK(hipGetDeviceProperties(&prop, device));
     c->num_cus = prop.multiProcessorCount;
@@ -1045,7 +1042,6 @@ void ks_ctx_destroy(ks_ctx* c) {
   c->part.release();
   c->stats.release();
   c->coop.release();
-  c->scal.release();
   if (c->hflags) (void)hipHostFree(c->hflags);
   if (c->stream && c->own_stream) (void)hipStreamDestroy(c->stream);
   delete c;
@@ -1331,14 +1327,13 @@ ks_status ks_dot(ks_ctx* c, int64_t n, int32_t precision, const void* x, const v
   set_device(c);
   if (precision == KS_F32) {
     In<float> xi(c, (const float*)x, n, flags), yi(c, (const float*)y, n, flags);
-    launch_map<1>(c, n, OpDot<float>{xi.p, yi.p, c->scal.p, 0}, Gate{}, KS_K_REDUCE, 8.0 * n);
+    launch_map<1>(c, n, OpDot<float>{xi.p, yi.p, c->hscal_dev, 0}, Gate{}, KS_K_REDUCE, 8.0 * n);
   } else {
     In<double> xi(c, (const double*)x, n, flags), yi(c, (const double*)y, n, flags);
-    launch_map<1>(c, n, OpDot<double>{xi.p, yi.p, c->scal.p, 0}, Gate{}, KS_K_REDUCE, 16.0 * n);
+    launch_map<1>(c, n, OpDot<double>{xi.p, yi.p, c->hscal_dev, 0}, Gate{}, KS_K_REDUCE, 16.0 * n);
   }
-  KS_HIPCK(hipMemcpyAsync(out, c->scal.p, sizeof(double), hipMemcpyDeviceToHost, c->stream));
   KS_HIPCK(hipStreamSynchronize(c->stream));
-  if (n == 0) *out = 0.0;
+  *out = n == 0 ? 0.0 : *c->hscal;
   return KS_OK;
   KS_API_CATCH(c)
 }
@@ -1349,14 +1344,13 @@ ks_status ks_norm2(ks_ctx* c, int64_t n, int32_t precision, const void* x, doubl
   set_device(c);
   if (precision == KS_F32) {
     In<float> xi(c, (const float*)x, n, flags);
-    launch_map<1>(c, n, OpDot<float>{xi.p, xi.p, c->scal.p, 1}, Gate{}, KS_K_REDUCE, 4.0 * n);
+    launch_map<1>(c, n, OpDot<float>{xi.p, xi.p, c->hscal_dev, 1}, Gate{}, KS_K_REDUCE, 4.0 * n);
   } else {
     In<double> xi(c, (const double*)x, n, flags);
-    launch_map<1>(c, n, OpDot<double>{xi.p, xi.p, c->scal.p, 1}, Gate{}, KS_K_REDUCE, 8.0 * n);
+    launch_map<1>(c, n, OpDot<double>{xi.p, xi.p, c->hscal_dev, 1}, Gate{}, KS_K_REDUCE, 8.0 * n);
   }
-  KS_HIPCK(hipMemcpyAsync(out, c->scal.p, sizeof(double), hipMemcpyDeviceToHost, c->stream));
   KS_HIPCK(hipStreamSynchronize(c->stream));
-  if (n == 0) *out = 0.0;
+  *out = n == 0 ? 0.0 : *c->hscal;
   return KS_OK;
   KS_API_CATCH(c)
 }
