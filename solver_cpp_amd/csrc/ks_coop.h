@@ -368,4 +368,153 @@ __global__ __launch_bounds__(NT) void k_cg_coop(int64_t n, const int32_t* __rest
   team.close();
 }
 
+// BiCG (bicg.cpp:162-310), as k_cg_coop: a step is both products (A p and
+// A^T p*), the reduction of
+// (p*, A p), the updates, and the reduction of (r*, r) and (r, r).  vec holds
+// r, r*, then p and p* of even and of odd steps.  Both matrices' entries stay
+// in registers, so FP64 takes at most two rows per thread.
+// Measured (7-point grids, FP64, us a step, on chip against five launches):
+// 16^3 6.3 / 22.9, 32^3 8.6 / 23.9, 50^3 11.9 / 26.7, 64^3 20.7 / 29.8.
+template <class T, int NT, int RPT>
+__global__ __launch_bounds__(NT) void k_bicg_coop(int64_t n, const int32_t* __restrict__ ptr,
+                                                  const int32_t* __restrict__ col, const T* __restrict__ val,
+                                                  const int32_t* __restrict__ tptr, const int32_t* __restrict__ tcol,
+                                                  const T* __restrict__ tval, const double* __restrict__ src, T* xs,
+                                                  T* vec, int64_t ld, double* xout, Ctl* c, CoopArgs ca, int mode,
+                                                  int last, int iters, Gate g, StatArgs st) {
+  if (g.off()) return;
+  __shared__ int s_out;
+  Team<NT> team(ca, &s_out);
+  if (!team.good) return;
+  __shared__ T pl[RPT * NT], psl[RPT * NT];
+  CoopRows<T, NT, RPT> A, B;
+  A.load(n, ptr, col, val);
+  B.load(n, tptr, tcol, tval);
+  T x[RPT], r[RPT], rs[RPT], p[RPT], ps[RPT], q[RPT], qs[RPT];
+  const double eps = c->eps;
+  const long long maxloop = c->maxloop;
+  long long count = mode ? 1 : c->count;
+  // rz = (r*, r); rr = (r, r), which the test looks at
+  double bnorm = c->bnorm, rz = c->rr, rr = c->gamma, alpha = 0.0, beta = mode ? 0.0 : c->beta;
+  CoopHist hist{c->hist, mode == 1 ? 0 : c->nhist, c->hist_cap};
+  int stop = -1;
+  const bool boss = blockIdx.x == 0 && threadIdx.x == 0;
+  bool fresh = mode != 0;  // p is r, p* is r*
+  T* const rv = vec;
+  T* const rsv = vec + ld;
+  T* now = vec + (count & 1 ? 4 * ld : 2 * ld);  // this step's p, then p*
+  T* old = vec + (count & 1 ? 2 * ld : 4 * ld);
+#pragma unroll
+  for (int j = 0; j < RPT; ++j) {
+    x[j] = r[j] = rs[j] = p[j] = ps[j] = T(0);
+    if (A.has(j)) {
+      const int32_t i = A.row0 + A.at(j);
+      if (mode == 1) r[j] = rs[j] = (T)src[i];
+      else { x[j] = xs[i]; r[j] = rv[i]; rs[j] = rsv[i]; }
+      if (mode == 0) { p[j] = old[i]; ps[j] = old[ld + i]; }
+    }
+  }
+  if (mode == 1) {
+    double s[1] = {0.0};
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) {
+      if (A.has(j)) {
+        shared_store(rv + A.row0 + A.at(j), r[j]);
+        shared_store(rsv + A.row0 + A.at(j), rs[j]);
+      }
+      s[0] += (double)r[j] * (double)r[j];
+    }
+    team.all_sum(s);
+    rz = rr = s[0];
+    bnorm = sqrt(rr);
+    stop = team.good ? cg_stop(count, maxloop, rr, bnorm, eps) : 3;
+    if (boss) hist.add(count, maxloop, rr, bnorm);
+  }
+  int done = 0;
+  while (stop < 0 && done < iters) {
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) {
+      p[j] = fresh ? r[j] : (T)(beta * (double)p[j] + (double)r[j]);
+      ps[j] = fresh ? rs[j] : (T)(beta * (double)ps[j] + (double)rs[j]);
+      pl[A.at(j)] = p[j];
+      psl[A.at(j)] = ps[j];
+      if (A.has(j)) {
+        shared_store(now + A.row0 + A.at(j), p[j]);
+        shared_store(now + ld + A.row0 + A.at(j), ps[j]);
+      }
+    }
+    __syncthreads();
+    struct Raw {
+      T r, p;
+    };
+    if (fresh) {
+      const auto same = [](T v) { return v; };
+      A.mul(pl, [&](int32_t i) { return shared_load(rv + i); }, same, q);
+      B.mul(psl, [&](int32_t i) { return shared_load(rsv + i); }, same, qs);
+    } else {
+      const auto near = [&](Raw f) { return (T)(beta * (double)f.p + (double)f.r); };
+      A.mul(pl, [&](int32_t i) { return Raw{shared_load(rv + i), shared_load(old + i)}; }, near, q);
+      B.mul(psl, [&](int32_t i) { return Raw{shared_load(rsv + i), shared_load(old + ld + i)}; }, near, qs);
+    }
+    double s1[1] = {0.0};
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) s1[0] = fma((double)ps[j], (double)q[j], s1[0]);
+    team.all_sum(s1);
+    alpha = rz / s1[0];
+    double s[2] = {0.0, 0.0};
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) {
+      x[j] = (T)(alpha * (double)p[j] + (double)x[j]);
+      r[j] = (T)((-alpha) * (double)q[j] + (double)r[j]);
+      rs[j] = (T)((-alpha) * (double)qs[j] + (double)rs[j]);
+      if (A.has(j)) {
+        shared_store(rv + A.row0 + A.at(j), r[j]);
+        shared_store(rsv + A.row0 + A.at(j), rs[j]);
+      }
+      s[0] = fma((double)rs[j], (double)r[j], s[0]);
+      s[1] = fma((double)r[j], (double)r[j], s[1]);
+    }
+    team.all_sum(s);
+    if (!team.good) break;
+    beta = s[0] / rz;
+    rz = s[0];
+    rr = s[1];
+    ++count;
+    ++done;
+    fresh = false;
+    T* t = now;
+    now = old;
+    old = t;
+    stop = cg_stop(count, maxloop, rr, bnorm, eps);
+    if (boss) hist.add(count, maxloop, rr, bnorm);
+  }
+  if (team.good) {
+#pragma unroll
+    for (int j = 0; j < RPT; ++j)
+      if (A.has(j)) {
+        const int32_t i = A.row0 + A.at(j);
+        xs[i] = x[j];
+        if (xout && (stop >= 0 || last)) xout[i] = (double)x[j];
+      }
+    if (boss) {
+      if (mode == 1) { c->done = 0; c->ksz = 0; c->steps = 0; c->bnorm = bnorm; }
+      c->count = count;
+      c->nhist = hist.n;
+      const double num = sqrt(rr);
+      c->err = (bnorm == 0.0 && num == 0.0) ? 0.0 : num / bnorm;
+      c->rr = rz;
+      c->gamma = rr;
+      c->alpha = alpha;
+      c->beta = beta;
+      c->steps += done;
+      c->tsteps += done;
+      c->stop = 0;
+      c->status = 2;
+      if (stop >= 0) ctl_stop(c, stop);
+      st.count_many(2 * done);
+    }
+  }
+  team.close();
+}
+
 }  // namespace ks

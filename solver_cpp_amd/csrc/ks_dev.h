@@ -448,9 +448,9 @@ void klaunch_n(ks_ctx* c, int cls, void (*kernel)(P...), int G, A&&... args) {
 // 9.3 / 16.8, 80^3 23.0 / 25.0; VPCG with ten FP32 CG steps, 300 x 300 102 /
 // 173).
 template <class T>
-bool coop_fits(const ks_ctx* c, const MatView<T>& A) {
+bool coop_fits(const ks_ctx* c, const MatView<T>& A, int rpt = kCoopRpt) {
   return !c->coop_off && A.kind == 0 && A.max_row <= kCoopRow &&
-         A.n <= (int64_t)kCoopRpt * kCoopThreads * std::min(c->num_cus, kCoopMaxWg);
+         A.n <= (int64_t)rpt * kCoopThreads * std::min(c->num_cus, kCoopMaxWg);
 }
 inline CoopArgs coop_args(ks_ctx* c) {
   return CoopArgs{c->coop.p, reinterpret_cast<unsigned*>(c->stats.p + 2 * KS_K_NCLASS), c->coop_spin};

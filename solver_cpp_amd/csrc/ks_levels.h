@@ -806,16 +806,28 @@ struct BicgLevel : Level {
   DBuf<T> r, rs, p, ps, q, xown;
   T* x = nullptr;
   double* xout = nullptr;
+  DBuf<T> vec;                  // on chip: r, rs, p, ps and two more, in one allocation
+  bool coop = false;            // on chip: a unit is kCoopIters steps in one launch (k_bicg_coop)
+  const double* src = nullptr;  // on chip: the right-hand side
+  static constexpr int kRpt = sizeof(T) == 8 ? 2 : kCoopRpt;  // rows per thread: what the registers hold twice
   void setup(ks_ctx* cx, const MatView<T>& a, const MatView<T>& at, const LevelCfg& cf) {
     c = cx; A = a; AT = at; n = a.n; cfg = cf;
-    r.alloc(n); rs.alloc(n); p.alloc(n); ps.alloc(n); q.alloc(n);
+    coop = coop_fits(c, A, kRpt) && coop_fits(c, AT, kRpt) && cfg.maxloop > 0;
+    if (coop) {
+      const int64_t ld = pad64(n);
+      vec.alloc(6 * ld);
+      r.borrow(vec.p, n); rs.borrow(vec.p + ld, n); p.borrow(vec.p + 2 * ld, n); ps.borrow(vec.p + 3 * ld, n);
+    } else {
+      r.alloc(n); rs.alloc(n); p.alloc(n); ps.alloc(n); q.alloc(n);
+    }
     if (sizeof(T) != 8) xown.alloc(n);
     setup_ctl(0, 0);
   }
   void enqueue_init(const double* b, double* x_out) override {
     xout = x_out;
     x = sizeof(T) == 8 ? (T*)x_out : xown.p;
-    const double* src = b;
+    src = b;
+    if (coop && !x0given) return;  // the first launch starts the solve
     if (x0given) {
       launch_map<1>(c, n, OpSetBnorm{b, ctl()}, gouter(), KS_K_REDUCE, 8.0 * n);
       launch_spmv<T, 1>(c, A, x, EpiResid<T, FinNone>{b, r.p, FinNone{}}, gouter(), 8.0 * n);
@@ -826,6 +838,23 @@ struct BicgLevel : Level {
   }
   // no finisher: OpAxpy2F and OpXpby2F take the totals they need
   void enqueue_unit(int64_t u) override {
+    if (coop) {
+      const int mode = u > 0 ? 0 : x0given ? 2 : 1;
+      const int iters = (int)std::min<int64_t>(kCoopIters, cfg.maxloop - u * kCoopIters);
+      const StatArgs st = stat(c, sizeof(T) == 8 ? KS_K_SPMV64 : KS_K_SPMV32, spmv_bytes<T>(A) + 10.0 * sizeof(T) * n);
+      auto go = [&](auto kernel) {
+        kernel<<<coop_grid(c, n), kCoopThreads, 0, c->stream>>>(
+            n, A.ptr, A.col, A.val, AT.ptr, AT.col, AT.val, src, x, vec.p, pad64(n), sizeof(T) == 8 ? nullptr : xout,
+            ctl(), coop_args(c), mode, u + 1 == max_units(), iters, mode == 1 ? gouter() : gstep(), st);
+      };
+      switch (coop_rows(c, n)) {
+        case 1: go(k_bicg_coop<T, kCoopThreads, 1>); break;
+        case 2: go(k_bicg_coop<T, kCoopThreads, 2>); break;
+        default: go(k_bicg_coop<T, kCoopThreads, kRpt>); break;
+      }
+      KS_HIPCK(hipGetLastError());
+      return;
+    }
     const int slot = (int)(u & 1);
     const int gd = launch_spmv<T, 1>(c, A, p.p, EpiDot<T, FinAlpha>{ps.p, q.p, FinAlpha{ctl()}}, gstep(),
                                      sizeof(T) * (double)n, false);
@@ -837,14 +866,19 @@ struct BicgLevel : Level {
     launch_map<0>(c, n, OpXpby2F<T>{p.p, r.p, ps.p, rs.p, ctl(), c->part.p, gu, slot, 0.0}, gstep(), KS_K_AXPY,
                   6.0 * sizeof(T) * n);
   }
-  int64_t max_units() const override { return cfg.maxloop > 0 ? cfg.maxloop : 0; }
+  int64_t max_units() const override {
+    if (coop) return (cfg.maxloop + (int64_t)kCoopIters - 1) / kCoopIters;
+    return cfg.maxloop > 0 ? cfg.maxloop : 0;
+  }
+  bool on_chip() const override { return coop; }
   void enqueue_finish() override {
-    if (sizeof(T) != 8) {
+    if (sizeof(T) != 8 && !coop) {
       k_convert<T, double><<<grid_map(n), kBlock, 0, c->stream>>>(n, x, xout, gouter());
       KS_HIPCK(hipGetLastError());
     }
   }
   double unit_seconds_estimate() const override {
+    if (coop) return 8e-6 * std::min(cfg.maxloop, kCoopIters);
     return std::max(5 * 4e-6, (2 * spmv_bytes<T>(n, A.nnz) + 20.0 * sizeof(T) * n) / 4e12);
   }
 };

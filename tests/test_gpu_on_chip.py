@@ -180,3 +180,57 @@ def test_two_threads(ctx):
     for t in ts:
         t.join()
     assert all(np.array_equal(x, ref) for xs in got for x in xs)
+
+
+# BiCG holds A and A^T: in FP64 at most two rows per thread
+BICG = [("bicg", "NO", {}), ("vpgmres", "bicg", dict(outer_restart=20, inner_maxloop=10, inner_precision=32))]
+
+
+def _upwind(n, seed=12):
+    # nonsymmetric, diagonally dominant by rows and columns
+    ptr, col, val, b = _tridiag(n, seed)
+    row = np.repeat(np.arange(n), np.diff(ptr))
+    return ptr, col, np.where(col < row, 1.1 * val, val), b
+
+
+@pytest.mark.parametrize("outer,inner,kw", BICG)
+@pytest.mark.parametrize("n", [1, 2, WG - 1, WG + 1, 64 * WG + 3, 256 * WG, 256 * WG + 1, 512 * WG, 512 * WG + 1,
+                               1024 * WG + 1])
+def test_bicg_sizes(ctx, both, n, outer, inner, kw):
+    from solver_cpp_amd import api
+    ptr, col, val, b = _upwind(n)
+    A = api.Matrix(ctx, ptr, col, val, fp32=True, transpose=True)
+    _same(*both(A, b, outer, inner, outer_eps=1e-12, outer_maxloop=500, **kw))
+    x0 = np.random.default_rng(13).standard_normal(n)
+    _same(*both(A, b, outer, inner, x0=x0, outer_eps=1e-12, outer_maxloop=500, **kw))
+    A.close()
+
+
+@pytest.mark.parametrize("outer,inner,kw", BICG)
+def test_bicg_stencil_and_right_sides(ctx, both, outer, inner, kw):
+    # 7-point upwind rows with neighbours in other workgroups; b of zeros, NaN and Inf
+    from solver_cpp_amd import api
+    ptr, col, val = P.convdiff3d(17, pe=0.8)[:3]
+    val = np.where(col == np.repeat(np.arange(len(ptr) - 1), np.diff(ptr)), val + 2.0, val)
+    b = np.random.default_rng(14).uniform(-1, 1, len(ptr) - 1)
+    A = api.Matrix(ctx, ptr, col, val, fp32=True, transpose=True)
+    _same(*both(A, b, outer, inner, outer_eps=1e-12, outer_maxloop=500, **kw))
+    for v in (0.0, np.nan, np.inf):
+        c = np.zeros_like(b)
+        c[700] = v
+        (x, r, _), (y, s, _) = both(A, c, outer, inner, outer_eps=1e-10, outer_maxloop=30, **kw)
+        assert r["status"] == s["status"] and r["iters"] == s["iters"]
+    A.close()
+
+
+@pytest.mark.parametrize("maxloop", [1, 2, 1023, 1024, 1025, 2049])
+def test_bicg_ends_at_maxloop(ctx, both, maxloop):
+    from solver_cpp_amd import api
+    ptr, col, val, b = _upwind(3 * WG)
+    A = api.Matrix(ctx, ptr, col, val, transpose=True)
+    (x, r, h), (y, s, g) = both(A, b, "bicg", outer_eps=0.0, outer_maxloop=maxloop)
+    if s["status"] == 2 and r["status"] == 2:
+        assert r["iters"] == s["iters"] == maxloop + 1 and r["n_hist"] == s["n_hist"] == maxloop
+    m = min(10, len(h), len(g))
+    assert np.array_equal(h[:m, 0], g[:m, 0]) and np.allclose(h[:m, 1], g[:m, 1], rtol=1e-6)
+    A.close()
