@@ -2040,11 +2040,13 @@ template <int M>
 __global__ void k_pat_find(int64_t n, const int32_t* __restrict__ ptr, const int32_t* __restrict__ col,
                            const double* __restrict__ val, PatState<M>* st) {
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  unsigned long long last = 0;  // a key that is in the table: most rows repeat it
   for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r < n; r += stride) {
-    if (*(volatile int*)&st->bad) return;
     const int32_t a = ptr[r], e = ptr[r + 1];
     if (e - a > (M == kRowMax ? kRowLen : kPatTab - 1 - M)) { st->bad = 1; return; }
     const unsigned long long h = pat_hash<M>(col, val, a, e, (int32_t)r);
+    if (h == last) continue;
+    if (*(volatile int*)&st->bad) return;
     int s = (int)(h % (2 * M)), tries = 0;
     for (; tries < 2 * M; ++tries, s = (s + 1) % (2 * M)) {
       unsigned long long k = *(volatile unsigned long long*)(st->key + s);
@@ -2053,6 +2055,7 @@ __global__ void k_pat_find(int64_t n, const int32_t* __restrict__ ptr, const int
       if (k == 0 || k == h) break;
     }
     if (tries == 2 * M) { st->bad = 1; return; }
+    last = h;
   }
 }
 // one workgroup of 2 M threads
