@@ -351,11 +351,12 @@ bool build_patterns(ks_mat* m, const Plan& pl, PatBuf& pat, const int32_t* ptr, 
 
 // Row classes (RowIx) of the CSR (ptr, col, val) with plan pl, under
 // build_patterns' conditions, for matrices of kRowMinNnz entries or more.  Not
-// for a borrowed matrix, whose values the caller may change in place.
-void build_rows(ks_mat* m, const Plan& pl, RowBuf& rows, const int32_t* ptr, const int32_t* col, const double* val) {
+// for a borrowed matrix, whose values the caller may change in place.  Returns
+// the number of classes (0: none).
+int build_rows(ks_mat* m, const Plan& pl, RowBuf& rows, const int32_t* ptr, const int32_t* col, const double* val) {
   if (pl.kind != 0 || !(pl.wg64 || pl.wg32) || pl.wg.long_rows || m->nnz < kRowMinNnz || m->n > kRowMaxN ||
       (m->flags & KS_MAT_BORROW))
-    return;
+    return 0;
   ks_ctx* c = m->ctx;
   hipStream_t s = c->stream;
   rows.alloc(RowBuf::kHead + (m->n + 3) / 4);
@@ -367,11 +368,18 @@ void build_rows(ks_mat* m, const Plan& pl, RowBuf& rows, const int32_t* ptr, con
   k_row_codes<<<grid_map(m->n), kBlock, 0, s>>>(m->n, st, ptr, col, val, code);
   k_row_vals<<<1, kRowMax, 0, s>>>(st, rows.p, ptr, val, rows.v64(), rows.v32());
   KS_HIPCK(hipGetLastError());
-  int bad = 0;
-  KS_HIPCK(hipMemcpyAsync(&bad, &st->bad, sizeof(int), hipMemcpyDeviceToHost, s));
+  struct {
+    int P, bad;
+  } end = {0, 0};  // as PatState ends
+  static_assert(offsetof(PatState<kRowMax>, bad) == offsetof(PatState<kRowMax>, P) + sizeof(int), "P, then bad");
+  KS_HIPCK(hipMemcpyAsync(&end, &st->P, sizeof(end), hipMemcpyDeviceToHost, s));
   KS_HIPCK(hipStreamSynchronize(s));
-  if (bad) rows.release();
-  else rows.code = code;
+  if (end.bad) {
+    rows.release();
+    return 0;
+  }
+  rows.code = code;
+  return end.P;
 }
 
 // New values: refreshes a side's classes; *bad (after the stream's next
@@ -384,10 +392,12 @@ void refresh_rows(ks_mat* m, RowBuf& rows, const int32_t* ptr, const double* val
   KS_HIPCK(hipGetLastError());
   KS_HIPCK(hipMemcpyAsync(bad, &rows.state()->bad, sizeof(int), hipMemcpyDeviceToHost, s));
 }
-void drop_rows(RowBuf& rows, int bad) {
+void drop_rows(ks_mat* m, RowBuf& rows, int bad, const Plan& pl, PatBuf& pat, bool other, const int32_t* ptr,
+               const int32_t* col) {
   if (!bad) return;
   rows.code = nullptr;
   rows.release();
+  if (!pat.code && !other) build_patterns(m, pl, pat, ptr, col);
 }
 
 // The SpMV's 16-bit column indices of A and A^T, unless KS_MAT_COL32: row
@@ -395,7 +405,8 @@ void drop_rows(RowBuf& rows, int bad) {
 // when every offset fits (hp, hc: A's host row pointers and columns; A^T's
 // offsets are A's negated, so both fit), delta-coded columns where those
 // apply, in the order KS_MAT_COL_DELTA asks for, and with the first two the
-// row classes, where those apply (the others are what new values fall back to); int32 columns otherwise, and
+// row classes, where those apply (what new values fall back to is built with them
+// or, of few classes, when that happens); int32 columns otherwise, and
 // for a side whose SpMV runs on column panels (which read int32 columns).
 void build_index16(ks_mat* m, const int32_t* hp, const int32_t* hc) {
   const bool delta_first = (m->flags & KS_MAT_COL_DELTA) != 0;
@@ -403,7 +414,10 @@ void build_index16(ks_mat* m, const int32_t* hp, const int32_t* hc) {
   auto side = [&](RowBuf& rows, PatBuf& op, DBuf<int16_t>& o16, DBuf<uint16_t>& od, const Plan& pl,
                   const PanelSet& ps, const int32_t* ptr, const int32_t* col, const double* val) {
     if (ps.np || pl.kind != 0) return;
-    if (!delta_first) build_rows(m, pl, rows, ptr, col, val);
+    // up to kPatMax classes have no more patterns, whose table fits: those are
+    // built when new values end the classes (ks_mat_update_values)
+    const int classes = delta_first ? 0 : build_rows(m, pl, rows, ptr, col, val);
+    if (classes > 0 && classes <= kPatMax) return;
     if (!delta_first && build_patterns(m, pl, op, ptr, col)) return;
     if (off16 < 0) off16 = offsets_fit16(m->n, hp, hc);
     if (off16 && !delta_first) build_col16(m, o16, ptr, col);
@@ -1163,8 +1177,8 @@ ks_status ks_mat_update_values(ks_mat* m, const double* val, uint32_t flags) {
     KS_HIPCK(hipGetLastError());
   }
   KS_HIPCK(hipStreamSynchronize(c->stream));
-  drop_rows(m->rows, bad);
-  drop_rows(m->trows, tbad);
+  drop_rows(m, m->rows, bad, m->plan, m->pat, m->col16.p || m->cold.p, m->ptr.p, m->col.p);
+  drop_rows(m, m->trows, tbad, m->tplan, m->tpat, m->tcol16.p || m->tcold.p, m->tptr.p, m->tcol.p);
   return KS_OK;
   KS_API_CATCH(c)
 }
@@ -1209,7 +1223,7 @@ ks_status ks_mat_index_bytes(const ks_mat* m, int32_t trans, int32_t precision, 
   KS_API_TRY
   set_device(c);
   const auto v = m->view<double>(trans != 0);
-  *bytes = !v.pat ? (precision == KS_F64 ? v.ib : m->view<float>(trans != 0).ib) : entry_index_bytes(m, trans != 0);
+  *bytes = !v.pat && !v.row ? (precision == KS_F64 ? v.ib : m->view<float>(trans != 0).ib) : entry_index_bytes(m, trans != 0);
   return KS_OK;
   KS_API_CATCH(c)
 }
