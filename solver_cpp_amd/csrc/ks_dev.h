@@ -151,7 +151,7 @@ struct ks_ctx {
   ks::DBuf<unsigned long long> stats;    // launches[8], bytes[8], on-chip solves' state (tag, fail)
   ks::DBuf<unsigned long long> coop;     // on-chip solves' reduction slots (kCoopSlots)
   bool coop_off = false;                 // solve with one launch per operation
-  int coop_spin = ks::kCoopSpin;         // polls of one bounded wait
+  int coop_spin = ks::kCoopSpin;         // polls of one bounded wait; 0: no on-chip solves
   int* hflags = nullptr;                 // host-mapped flags (host view)
   int* hflags_dev = nullptr;             // same memory, device view
   // scalar results in the same memory (host and device views): the finisher
@@ -449,7 +449,7 @@ void klaunch_n(ks_ctx* c, int cls, void (*kernel)(P...), int G, A&&... args) {
 // 173).
 template <class T>
 bool coop_fits(const ks_ctx* c, const MatView<T>& A, int rpt = kCoopRpt) {
-  return !c->coop_off && A.kind == 0 && A.max_row <= kCoopRow &&
+  return !c->coop_off && c->coop_spin > 0 && A.kind == 0 && A.max_row <= kCoopRow &&
          A.n <= (int64_t)rpt * kCoopThreads * std::min(c->num_cus, kCoopMaxWg);
 }
 inline CoopArgs coop_args(ks_ctx* c) {
