@@ -176,9 +176,14 @@ const char* ks_ctx_last_error(const ks_ctx* ctx);
  * wait for each other (on-chip solves).  `polls` bounds each such wait
  * (default 2^21, about a second); when one runs out, for instance because
  * another process holds the GPU, the solve is repeated with one launch per
- * operation.  0 makes every such solve take that way.  No reference
- * counterpart. */
+ * operation, and so are the context's next 64 solves (twice as many after each
+ * further failure in a row, up to 4096; this call ends that).  0 makes every
+ * such solve take that way.  No reference counterpart. */
 ks_status ks_ctx_set_wait_limit(ks_ctx* ctx, int32_t polls);
+/* On-chip solves this context has begun, and how many of them were repeated
+ * because a wait ran out (either pointer may be NULL).  No reference
+ * counterpart. */
+ks_status ks_ctx_on_chip(const ks_ctx* ctx, int64_t* solves, int64_t* repeated);
 /* hipStream_t the context launches on (as void*), for callers that order
  * their own work against it. */
 void* ks_ctx_stream(ks_ctx* ctx);

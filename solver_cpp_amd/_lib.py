@@ -27,6 +27,7 @@ _SIGS = {
     "ks_ctx_destroy": (None, [_vp]),
     "ks_ctx_last_error": (C.c_char_p, [_vp]),
     "ks_ctx_set_wait_limit": (_i32, [_vp, _i32]),
+    "ks_ctx_on_chip": (_i32, [_vp, C.POINTER(_i64), C.POINTER(_i64)]),
     "ks_ctx_stream": (_vp, [_vp]),
     "ks_ctx_synchronize": (_i32, [_vp]),
     "ks_mat_create_csr": (_i32, [_vp, _i64, _i64, _vp, _vp, _vp, _u32, _pp]),

@@ -103,6 +103,12 @@ class Context:
         """Bound on one wait inside an on-chip solve (ks_ctx_set_wait_limit)."""
         self.check(self.lib.ks_ctx_set_wait_limit(self.h, int(polls)), "set_wait_limit")
 
+    def on_chip(self):
+        """On-chip solves begun, and of them repeated because a wait ran out."""
+        n, r = C.c_int64(), C.c_int64()
+        self.check(self.lib.ks_ctx_on_chip(self.h, C.byref(n), C.byref(r)), "on_chip")
+        return dict(solves=n.value, repeated=r.value)
+
     def synchronize(self):
         self.check(self.lib.ks_ctx_synchronize(self.h), "synchronize")
 

@@ -20,8 +20,10 @@
 //
 // Every wait is bounded (CoopArgs::spin polls).  A wait that runs out (the
 // workgroups were not resident together, for instance beside another process)
-// sets *fail and ends the launch; later launches return at once and the host
-// repeats the solve with one launch per operation.
+// sets the fail word and ends the launch: its workgroups make no further wait,
+// later launches return at once, the solve's and the host's stop flags keep the
+// outer solver's steps from running on, and the host repeats the solve with one
+// launch per operation (and does the context's next solves that way: ks_ctx).
 #pragma once
 #include "ks_kernels.h"
 
@@ -43,6 +45,8 @@ constexpr int64_t kCoopSlots = 2 * 2 * (int64_t)kCoopVals * kCoopMaxWg;
 struct CoopArgs {
   unsigned long long* slots;  // kCoopSlots words: [parity][value][workgroup][2]
   unsigned* state;            // [0] tag of the last reduction, [1] fail
+  int* stop;                  // a failure sets it: the stop flag of the solve around this one (nullable)
+  int* host_stop;             // and the flag that the host looks at
   int spin;
 };
 
@@ -86,13 +90,15 @@ struct Team {
 
   __device__ Team(const CoopArgs& args, int* out_) : a(args), out(out_) {
     round = a.state[0];
-    good = a.state[1] == 0;
+    good = shared_load(a.state + 1) == 0;
     if (threadIdx.x == 0) *out = 0;  // ordered by the first reduction's barrier
   }
-  // v[i] summed over all threads of all workgroups, i < NV, in every thread.
+  // v[i] summed over all threads of all workgroups, i < NV, in every thread;
+  // nothing once a wait has run out.
   template <int NV>
   __device__ void all_sum(double (&v)[NV]) {
     static_assert(NV <= kCoopVals, "slots");
+    if (!good) return;
     __shared__ double red[NV][kWaves];
     __shared__ double tot[NV];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, W = gridDim.x;
@@ -146,8 +152,11 @@ struct Team {
   // at the end of the launch: the next launch's first tag, or the failure
   __device__ void close() {
     if (threadIdx.x != 0) return;
-    if (!good) a.state[1] = 1;
-    else if (blockIdx.x == 0) a.state[0] = round;
+    if (!good) {
+      shared_store(a.state + 1, 1u);
+      if (a.stop) shared_store(a.stop, 1);
+      *(volatile int*)a.host_stop = 1;
+    } else if (blockIdx.x == 0) a.state[0] = round;
   }
 };
 

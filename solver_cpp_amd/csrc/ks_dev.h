@@ -151,6 +151,13 @@ struct ks_ctx {
   ks::DBuf<unsigned long long> stats;    // launches[8], bytes[8], on-chip solves' state (tag, fail)
   ks::DBuf<unsigned long long> coop;     // on-chip solves' reduction slots (kCoopSlots)
   bool coop_off = false;                 // solve with one launch per operation
+  // After a wait ran out, solves go by launches for coop_rest more of them,
+  // coop_pause the next time (twice as many after each failure in a row): where
+  // the GPU stays shared, what the waits cost (about a second each) is spread
+  // over ever more solves.
+  static constexpr int kPause = 64, kMaxPause = 4096;
+  int coop_rest = 0, coop_pause = kPause;
+  int64_t coop_solves = 0, coop_repeats = 0;  // on-chip solves begun, and of them repeated
   int coop_spin = ks::kCoopSpin;         // polls of one bounded wait; 0: no on-chip solves
   int* hflags = nullptr;                 // host-mapped flags (host view)
   int* hflags_dev = nullptr;             // same memory, device view
@@ -452,8 +459,10 @@ bool coop_fits(const ks_ctx* c, const MatView<T>& A, int rpt = kCoopRpt) {
   return !c->coop_off && c->coop_spin > 0 && A.kind == 0 && A.max_row <= kCoopRow &&
          A.n <= (int64_t)rpt * kCoopThreads * std::min(c->num_cus, kCoopMaxWg);
 }
-inline CoopArgs coop_args(ks_ctx* c) {
-  return CoopArgs{c->coop.p, reinterpret_cast<unsigned*>(c->stats.p + 2 * KS_K_NCLASS), c->coop_spin};
+// outer_stop: the stop flag of the solve that this one is an inner solve of
+inline CoopArgs coop_args(ks_ctx* c, const int* outer_stop) {
+  return CoopArgs{c->coop.p, reinterpret_cast<unsigned*>(c->stats.p + 2 * KS_K_NCLASS), const_cast<int*>(outer_stop),
+                  c->hflags_dev, c->coop_spin};
 }
 // rows per thread: as few as the CUs allow
 inline int coop_rows(const ks_ctx* c, int64_t n) {

@@ -871,7 +871,10 @@ bool run_level(ks_ctx* c, ks_mat* m, Level& Lv, const ks_params* p, unsigned pro
                double* rbuf) {
   Level* L = &Lv;
   std::unique_lock<std::mutex> lk;
-  if (L->on_chip()) lk = std::unique_lock<std::mutex>(coop_mutex(c->device));
+  if (L->on_chip()) {
+    lk = std::unique_lock<std::mutex>(coop_mutex(c->device));
+    ++c->coop_solves;
+  }
   L->x0given = (p->flags & KS_X0_GIVEN) != 0;
   double r0 = 0;
   if (L->x0given) r0 = resid_norm(c, m, trans, b, x, rbuf);
@@ -888,8 +891,12 @@ bool run_level(ks_ctx* c, ks_mat* m, Level& Lv, const ks_params* p, unsigned pro
   KS_HIPCK(hipMemcpy(st, c->stats.p, sizeof(st), hipMemcpyDeviceToHost));
   if (L->on_chip() && (st[2 * KS_K_NCLASS] >> 32)) {
     coop_reset(c);
+    ++c->coop_repeats;
+    c->coop_rest = c->coop_pause;
+    c->coop_pause = std::min(2 * c->coop_pause, ks_ctx::kMaxPause);
     return false;
   }
+  if (L->on_chip()) c->coop_pause = ks_ctx::kPause;
   // tags are 32 bits: start again long before they could meet an old one
   if (L->on_chip() && (uint32_t)st[2 * KS_K_NCLASS] > (1u << 31)) coop_reset(c);
   double ms[KS_K_NCLASS] = {0};
@@ -927,10 +934,18 @@ bool run_level(ks_ctx* c, ks_mat* m, Level& Lv, const ks_params* p, unsigned pro
   return true;
 }
 
+// Whether a solve may not run on chip: when the caller's `off` says so, or for
+// the context's next solves after a wait ran out.
+bool coop_rests(ks_ctx* c, bool off) {
+  if (off || c->coop_rest == 0) return off;
+  --c->coop_rest;
+  return true;
+}
+
 void solve_impl(ks_ctx* c, ks_mat* m, const ks_params* p, bool trans, const double* b, double* x, double* hist,
                 int64_t hist_cap, ks_result* res, double* x0norm_out) {
   // per-class times need the operations' own launches
-  c->coop_off = p->profile > 0;
+  c->coop_off = coop_rests(c, p->profile > 0);
   DBuf<double> x0;  // the initial guess, should an on-chip solve have to be repeated
   for (;;) {
     auto L = make_solver(c, m, p, trans, hist ? hist_cap : 0);
@@ -1065,6 +1080,14 @@ const char* ks_ctx_last_error(const ks_ctx* c) { return c ? c->err.c_str() : "nu
 ks_status ks_ctx_set_wait_limit(ks_ctx* c, int32_t polls) {
   if (!c || polls < 0) return KS_ERR_BAD_INPUT;
   c->coop_spin = polls;
+  c->coop_rest = 0;
+  c->coop_pause = ks_ctx::kPause;
+  return KS_OK;
+}
+ks_status ks_ctx_on_chip(const ks_ctx* c, int64_t* solves, int64_t* repeated) {
+  if (!c) return KS_ERR_BAD_INPUT;
+  if (solves) *solves = c->coop_solves;
+  if (repeated) *repeated = c->coop_repeats;
   return KS_OK;
 }
 void* ks_ctx_stream(ks_ctx* c) { return c ? (void*)c->stream : nullptr; }
@@ -1523,7 +1546,7 @@ ks_status ks_solve_noalloc(ks_ctx* c, ks_mat* m, const ks_params* p, const doubl
                 "scratch holds three padded vectors and the control state at the maximum size");
   std::lock_guard<std::mutex> lk(scratch_table().call[c->device]);
   // an on-chip solve that has to be repeated would need a copy of the guess
-  c->coop_off = (p->flags & KS_X0_GIVEN) != 0;
+  c->coop_off = coop_rests(c, (p->flags & KS_X0_GIVEN) != 0);
   for (;;) {
     CgLevel<double> L;
     L.setup(c, m->view<double>(false), outer_cfg(p, 0), c->scratch);

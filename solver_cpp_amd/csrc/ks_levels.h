@@ -670,7 +670,7 @@ struct CgLevel : Level {
       const StatArgs st = stat(c, sizeof(T) == 8 ? KS_K_SPMV64 : KS_K_SPMV32, spmv_bytes<T>(A) + 10.0 * sizeof(T) * n);
       auto go = [&](auto kernel) {
         kernel<<<coop_grid(c, n), kCoopThreads, 0, c->stream>>>(n, A.ptr, A.col, A.val, src, x, r.p, ld,
-                                                             sizeof(T) == 8 ? nullptr : xout, ctl(), coop_args(c), mode,
+                                                             sizeof(T) == 8 ? nullptr : xout, ctl(), coop_args(c, outer_stop), mode,
                                                              u + 1 == max_units(), iters,
                                                              mode == 1 ? gouter() : gstep(), st);
       };
@@ -845,7 +845,7 @@ struct BicgLevel : Level {
       auto go = [&](auto kernel) {
         kernel<<<coop_grid(c, n), kCoopThreads, 0, c->stream>>>(
             n, A.ptr, A.col, A.val, AT.ptr, AT.col, AT.val, src, x, vec.p, pad64(n), sizeof(T) == 8 ? nullptr : xout,
-            ctl(), coop_args(c), mode, u + 1 == max_units(), iters, mode == 1 ? gouter() : gstep(), st);
+            ctl(), coop_args(c, outer_stop), mode, u + 1 == max_units(), iters, mode == 1 ? gouter() : gstep(), st);
       };
       switch (coop_rows(c, n)) {
         case 1: go(k_bicg_coop<T, kCoopThreads, 1>); break;
