@@ -255,6 +255,7 @@ struct MatView {
 // behind it (null: the side has none).
 struct PatBuf : DBuf<int32_t> {
   const PatIx* code = nullptr;
+  int entry_ib = 4;  // bytes per column index of the entry format it stands in for
 };
 
 // Row classes (RowIx) of one side: the table at p, then its values in FP64 and
@@ -263,6 +264,7 @@ struct RowBuf : DBuf<int32_t> {
   static constexpr int64_t kV64 = kRowTab, kV32 = kV64 + 2 * kRowMax * kRowLen, kState = kV32 + kRowMax * kRowLen;
   static constexpr int64_t kHead = kState + (sizeof(PatState<kRowMax>) / 4 + 64) / 64 * 64;
   RowIx* code = nullptr;
+  int entry_ib = 4;  // bytes per column index of the entry format it stands in for
   double* v64() const { return reinterpret_cast<double*>(p + kV64); }
   float* v32() const { return reinterpret_cast<float*>(p + kV32); }
   PatState<kRowMax>* state() const { return reinterpret_cast<PatState<kRowMax>*>(p + kState); }

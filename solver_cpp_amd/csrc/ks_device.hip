@@ -323,6 +323,24 @@ bool build_col_delta(const ks_mat* m, const Plan& pl, DBuf<uint16_t>& out, const
   return !hb;
 }
 
+// What the pattern kernels found, once they have run (PatState's last fields).
+struct PatEnd {
+  int P, bad, far, uncoded;
+  // bytes per index of the entry format that the side would have
+  int index_bytes(const Plan& pl) const { return !far || (!uncoded && pl.wg.lane1) ? 2 : 4; }
+};
+template <int M>
+PatEnd pat_end(ks_ctx* c, const PatState<M>* st) {
+  static_assert(sizeof(PatEnd) == 4 * sizeof(int) && offsetof(PatState<M>, bad) == offsetof(PatState<M>, P) + sizeof(int) &&
+                    offsetof(PatState<M>, far) == offsetof(PatState<M>, P) + 2 * sizeof(int) &&
+                    offsetof(PatState<M>, uncoded) == offsetof(PatState<M>, P) + 3 * sizeof(int),
+                "PatState ends as PatEnd");
+  PatEnd e{};
+  KS_HIPCK(hipMemcpyAsync(&e, &st->P, sizeof(e), hipMemcpyDeviceToHost, c->stream));
+  KS_HIPCK(hipStreamSynchronize(c->stream));
+  return e;
+}
+
 // Row patterns (PatIx) of the CSR (ptr, col) with plan pl: when its SpMV runs
 // on workgroup tiles, none of them one long row, and its rows have at most
 // kPatMax patterns whose table fits kPatTab.  `pat` holds the table, the
@@ -341,12 +359,14 @@ bool build_patterns(ks_mat* m, const Plan& pl, PatBuf& pat, const int32_t* ptr, 
   k_pat_codes<<<(unsigned)pl.wg.ntiles, kBlock, 0, s>>>(st, pat.p, pl.wg.tiles.p, pl.wg.tnz.p, ptr, col,
                                                         reinterpret_cast<PatIx*>(pat.p + head));
   KS_HIPCK(hipGetLastError());
-  int bad = 0;
-  KS_HIPCK(hipMemcpyAsync(&bad, &st->bad, sizeof(int), hipMemcpyDeviceToHost, s));
-  KS_HIPCK(hipStreamSynchronize(s));
-  if (bad) pat.release();
-  else pat.code = reinterpret_cast<PatIx*>(pat.p + head);
-  return !bad;
+  const PatEnd end = pat_end(c, st);
+  if (end.bad) {
+    pat.release();
+    return false;
+  }
+  pat.code = reinterpret_cast<PatIx*>(pat.p + head);
+  pat.entry_ib = end.index_bytes(pl);
+  return true;
 }
 
 // Row classes (RowIx) of the CSR (ptr, col, val) with plan pl, under
@@ -368,17 +388,13 @@ int build_rows(ks_mat* m, const Plan& pl, RowBuf& rows, const int32_t* ptr, cons
   k_row_codes<<<grid_map(m->n), kBlock, 0, s>>>(m->n, st, ptr, col, val, code);
   k_row_vals<<<1, kRowMax, 0, s>>>(st, rows.p, ptr, val, rows.v64(), rows.v32());
   KS_HIPCK(hipGetLastError());
-  struct {
-    int P, bad;
-  } end = {0, 0};  // as PatState ends
-  static_assert(offsetof(PatState<kRowMax>, bad) == offsetof(PatState<kRowMax>, P) + sizeof(int), "P, then bad");
-  KS_HIPCK(hipMemcpyAsync(&end, &st->P, sizeof(end), hipMemcpyDeviceToHost, s));
-  KS_HIPCK(hipStreamSynchronize(s));
+  const PatEnd end = pat_end(c, st);
   if (end.bad) {
     rows.release();
     return 0;
   }
   rows.code = code;
+  rows.entry_ib = end.index_bytes(pl);
   return end.P;
 }
 
@@ -426,22 +442,6 @@ void build_index16(ks_mat* m, const int32_t* hp, const int32_t* hc) {
   side(m->rows, m->pat, m->col16, m->cold, m->plan, m->panels, m->ptr.p, m->col.p, m->val.p);
   if (m->has_t)
     side(m->trows, m->tpat, m->tcol16, m->tcold, m->tplan, m->tpanels, m->tptr.p, m->tcol.p, m->tval.p);
-}
-
-// Bytes per column index of the entry format that a side with row patterns
-// would have without them: 2 where int16 offsets or delta codes apply.
-int entry_index_bytes(const ks_mat* m, bool trans) {
-  ks_ctx* c = m->ctx;
-  const int32_t *ptr = trans ? m->tptr.p : m->ptr.p, *col = trans ? m->tcol.p : m->col.p;
-  DBuf<int> bad(1);
-  k_fill<int><<<1, kBlock, 0, c->stream>>>(1, bad.p, 0);
-  k_col_reach<<<grid_map(m->n), kBlock, 0, c->stream>>>(m->n, ptr, col, bad.p);
-  KS_HIPCK(hipGetLastError());
-  int hb = 0;
-  KS_HIPCK(hipMemcpyAsync(&hb, bad.p, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-  KS_HIPCK(hipStreamSynchronize(c->stream));
-  DBuf<uint16_t> tmp;
-  return !hb || build_col_delta(m, trans ? m->tplan : m->plan, tmp, ptr, col) ? 2 : 4;
 }
 
 // Split the CSR (hp, hc: host row pointers and columns of A or A^T) into
@@ -1242,13 +1242,12 @@ ks_status ks_mat_info(const ks_mat* m, int64_t* n, int64_t* nnz, int32_t* kind, 
 ks_status ks_mat_index_bytes(const ks_mat* m, int32_t trans, int32_t precision, int32_t* bytes) {
   if (!m || !bytes || (precision != KS_F64 && precision != KS_F32)) return KS_ERR_BAD_INPUT;
   if (trans && !m->has_t) return KS_ERR_BAD_INPUT;
-  ks_ctx* c = m->ctx;
-  KS_API_TRY
-  set_device(c);
-  const auto v = m->view<double>(trans != 0);
-  *bytes = !v.pat && !v.row ? (precision == KS_F64 ? v.ib : m->view<float>(trans != 0).ib) : entry_index_bytes(m, trans != 0);
+  const PatBuf& pat = trans ? m->tpat : m->pat;
+  const RowBuf& rows = trans ? m->trows : m->rows;
+  if (rows.code) *bytes = rows.entry_ib;
+  else if (pat.code) *bytes = pat.entry_ib;
+  else *bytes = precision == KS_F64 ? m->view<double>(trans != 0).ib : m->view<float>(trans != 0).ib;
   return KS_OK;
-  KS_API_CATCH(c)
 }
 
 ks_status ks_mat_spmv_bytes(const ks_mat* m, int32_t trans, int32_t precision, double* bytes) {

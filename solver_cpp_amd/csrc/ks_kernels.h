@@ -1978,16 +1978,6 @@ __global__ void k_col_offsets(int64_t n, const int32_t* __restrict__ ptr, const 
     for (int32_t j = ptr[r], e = ptr[r + 1]; j < e; ++j) out[j] = (int16_t)(col[j] - r);
 }
 
-// *bad is set when an entry lies over 32767 columns from its row.
-__global__ void k_col_reach(int64_t n, const int32_t* __restrict__ ptr, const int32_t* __restrict__ col, int* bad) {
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r < n; r += stride)
-    for (int32_t j = ptr[r], e = ptr[r + 1]; j < e; ++j) {
-      const int64_t d = (int64_t)col[j] - r;
-      if (d < -32767 || d > 32767) *bad = 1;
-    }
-}
-
 // Delta-coded columns (see k_spmv_stream): out[first] = col - r + kDeltaBias,
 // out[j] = col[j] - col[j - 1] after it; *bad is set when a row is not
 // sorted or a code does not fit 16 bits (the host then keeps int32 columns)
@@ -2020,6 +2010,8 @@ struct PatState {
   unsigned long long hash[M];  // by pattern number
   int32_t row[M];              // a row of it
   int P, bad;
+  int far;      // some offset does not fit int16 offsets
+  int uncoded;  // some row does not fit delta codes
 };
 template <int M>
 __device__ inline uint64_t pat_hash(const int32_t* __restrict__ col, const double* __restrict__ val, int32_t a,
@@ -2086,7 +2078,17 @@ __global__ void k_pat_table(PatState<M>* st, const int32_t* __restrict__ ptr, co
     return;
   }
   if (s == 0) st->P = P;
-  if (k) { st->hash[p] = k; st->row[p] = r; }
+  if (k) {
+    st->hash[p] = k;
+    st->row[p] = r;
+    int32_t prev = r - kDeltaBias;  // as k_col_offsets and k_col_delta see the row
+    for (int j = 0; j < len; ++j) {
+      const int64_t d = (int64_t)col[a + j] - r, code = (int64_t)col[a + j] - prev;
+      if (d < -32767 || d > 32767) st->far = 1;
+      if (code < 0 || code > 65535) st->uncoded = 1;
+      prev = col[a + j];
+    }
+  }
   if constexpr (M == kRowMax) {
     if (k)
       for (int j = 0; j < len; ++j) tab[p * kRowLen + j] = col[a + j] - r;
