@@ -45,7 +45,7 @@ struct BinView {
   const int32_t* snz = nullptr;      // first entry, nseg + 1
   const uint64_t* mask = nullptr;    // run starts, kBinWords per segment
   const uint16_t* before = nullptr;  // starts before each word
-  const int32_t* shift = nullptr;    // xg index minus place, by run, nblk per segment
+  const int32_t* shift = nullptr;    // xg index minus place, by run, nblk per segment (one 0 without entries)
   const int32_t* unit = nullptr;     // first pass: block, first and last + 1 entry of xg
   const uint16_t* lcol = nullptr;    // column within its block, in xg's order
   const uint16_t* place = nullptr;   // CSR place in the segment, ordered by segment, then block
@@ -97,6 +97,7 @@ __global__ __launch_bounds__(kBlock) void k_bin_fill(int nblk, int64_t nseg, con
       }
       p += len;
     }
+    if (r == 0) shift[s * nblk] = 0;  // a segment without entries: BinLoad reads xg[0]
   }
   __syncthreads();
   for (int k = threadIdx.x; k < kBinWords; k += kBlock) {
@@ -163,9 +164,14 @@ struct BinLoad {
   static constexpr int U = kBinEntries / kBinSum;
   T x[U];
   int p[U];
-  __device__ __forceinline__ static int at(int u, int cnt) { return min((int)threadIdx.x + u * kBinSum, cnt - 1); }
-  // run numbers first, then their shifts, then every entry.  Not for a
-  // segment without entries: it has no run, and no last place.
+  __device__ __forceinline__ static int at(int u, int cnt) {
+    return min((int)threadIdx.x + u * kBinSum, max(cnt, 1) - 1);
+  }
+  // where a segment's loads start: at the matrix's first entry for a segment
+  // without entries, so that they need no branch (which costs registers: six
+  // to eight spilled in every FP64 k_bin_sum)
+  __device__ __forceinline__ static int32_t first(int32_t j0, int cnt) { return cnt > 0 ? j0 : 0; }
+  // run numbers first, then their shifts, then every entry; j0: first()
   __device__ __forceinline__ void load(const BinView& B, int64_t s, int32_t j0, int cnt, const T* __restrict__ xg) {
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint64_t* mask = B.mask + s * kBinWords + w;
@@ -258,13 +264,12 @@ __global__ __launch_bounds__(kBinSum) __attribute__((amdgpu_waves_per_eu(4))) vo
   rbs.range(s, end, step);
   for (; s < end; s += step) {
     const int32_t r0 = B.seg[s], r1 = B.seg[s + 1], j0 = B.snz[s], cnt = B.snz[s + 1] - j0;
+    const int32_t jl = BinLoad<T>::first(j0, cnt);
     BinLoad<T> x;
     T v[U];
-    if (cnt > 0) {
-      x.load(B, s, j0, cnt, xg);
+    x.load(B, s, jl, cnt, xg);
 #pragma unroll
-      for (int u = 0; u < U; ++u) v[u] = ld_stream(val + j0 + BinLoad<T>::at(u, cnt));
-    }
+    for (int u = 0; u < U; ++u) v[u] = ld_stream(val + jl + BinLoad<T>::at(u, cnt));
     x.stage(cnt, sp);
     __syncthreads();
 #pragma unroll
@@ -303,7 +308,7 @@ __global__ __launch_bounds__(kBinSum) __attribute__((amdgpu_waves_per_eu(4))) vo
   for (; s < end; s += step) {
     const int32_t r0 = B.seg[s], r1 = B.seg[s + 1], j0 = B.snz[s], cnt = B.snz[s + 1] - j0;
     BinLoad<double> x;
-    if (cnt > 0) x.load(B, s, j0, cnt, xg);
+    x.load(B, s, BinLoad<double>::first(j0, cnt), cnt, xg);
     x.stage(cnt, sp);
     __syncthreads();
     for (int32_t rb = r0 + w; rb < r1; rb += kBinSum)
