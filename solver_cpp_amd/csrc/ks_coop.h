@@ -191,10 +191,11 @@ struct CoopRows {
   __device__ bool local(int32_t i) const { return (unsigned)(i - row0) < (unsigned)own; }
   // Row sums in CSR order, products rounded before the add, as the SpMV
   // kernels form them.  far(c) loads what x of another workgroup's row c is
-  // formed from, near(that) forms it: the loads of two rows go out together
-  // before the first is used (waited for one by one they cost 0.7 us each).
+  // formed from, near(that, beta) forms it: the loads of two rows go out
+  // together before the first is used (waited for one by one they cost 0.7 us
+  // each).
   template <class Far, class Near>
-  __device__ __forceinline__ void mul(const T* xl, Far far, Near near, T (&y)[RPT]) const {
+  __device__ __forceinline__ void mul(const T* xl, double beta, Far far, Near near, T (&y)[RPT]) const {
     constexpr int J = RPT < 2 ? RPT : 2;
 #pragma unroll
     for (int j0 = 0; j0 < RPT; j0 += J) {
@@ -204,6 +205,10 @@ struct CoopRows {
 #pragma unroll
         for (int k = 0; k < kCoopRow; ++k)
           if (k < len[j0 + j] && !local(c[j0 + j][k])) f[j][k] = far(c[j0 + j][k]);
+      // near()'s beta comes after the loads: the compiler otherwise moves its
+      // one fma up to each load and waits for them one by one (256 x 256: 6.3
+      // against 5.9 us a step)
+      asm volatile("" : "+v"(beta));
 #pragma unroll
       for (int j = 0; j < J; ++j) {
         T s = T(0);
@@ -211,13 +216,21 @@ struct CoopRows {
         for (int k = 0; k < kCoopRow; ++k)
           if (k < len[j0 + j]) {
             const int32_t i = c[j0 + j][k];
-            s = mul_add_rn(s, a[j0 + j][k], local(i) ? xl[i - row0] : near(f[j][k]));
+            s = mul_add_rn(s, a[j0 + j][k], local(i) ? xl[i - row0] : near(f[j][k], beta));
           }
         y[j0 + j] = s;
       }
     }
   }
 };
+
+// beta p + r, a row's new direction.  Its owner forms it and so does every
+// workgroup that gathers it, and the two must agree bit for bit: one rounding,
+// not what the compiler makes of a product and a sum at each place.
+template <class T>
+__device__ __forceinline__ T direction(double beta, T p, T r) {
+  return (T)fma(beta, (double)p, (double)r);
+}
 
 // Whether a CG-family solve ends at count with (r, r) = rr; -1 goes on, else
 // its status (cg_check's rule).
@@ -310,7 +323,7 @@ __global__ __launch_bounds__(NT) void k_cg_coop(int64_t n, const int32_t* __rest
   while (stop < 0 && done < iters) {
 #pragma unroll
     for (int j = 0; j < RPT; ++j) {
-      p[j] = fresh ? r[j] : (T)(beta * (double)p[j] + (double)r[j]);
+      p[j] = fresh ? r[j] : direction(beta, p[j], r[j]);
       pl[A.at(j)] = p[j];
       if (A.has(j)) shared_store(now + A.row0 + A.at(j), p[j]);
     }
@@ -319,10 +332,10 @@ __global__ __launch_bounds__(NT) void k_cg_coop(int64_t n, const int32_t* __rest
       T r, p;
     };
     if (fresh)
-      A.mul(pl, [&](int32_t i) { return shared_load(vec + i); }, [](T ri) { return ri; }, q);
+      A.mul(pl, beta, [&](int32_t i) { return shared_load(vec + i); }, [](T ri, double) { return ri; }, q);
     else
-      A.mul(pl, [&](int32_t i) { return Raw{shared_load(vec + i), shared_load(old + i)}; },
-            [&](Raw f) { return (T)(beta * (double)f.p + (double)f.r); }, q);
+      A.mul(pl, beta, [&](int32_t i) { return Raw{shared_load(vec + i), shared_load(old + i)}; },
+            [](Raw f, double b) { return direction(b, f.p, f.r); }, q);
     double s[1] = {0.0};
 #pragma unroll
     for (int j = 0; j < RPT; ++j) s[0] = fma((double)p[j], (double)q[j], s[0]);
@@ -443,8 +456,8 @@ __global__ __launch_bounds__(NT) void k_bicg_coop(int64_t n, const int32_t* __re
   while (stop < 0 && done < iters) {
 #pragma unroll
     for (int j = 0; j < RPT; ++j) {
-      p[j] = fresh ? r[j] : (T)(beta * (double)p[j] + (double)r[j]);
-      ps[j] = fresh ? rs[j] : (T)(beta * (double)ps[j] + (double)rs[j]);
+      p[j] = fresh ? r[j] : direction(beta, p[j], r[j]);
+      ps[j] = fresh ? rs[j] : direction(beta, ps[j], rs[j]);
       pl[A.at(j)] = p[j];
       psl[A.at(j)] = ps[j];
       if (A.has(j)) {
@@ -457,13 +470,13 @@ __global__ __launch_bounds__(NT) void k_bicg_coop(int64_t n, const int32_t* __re
       T r, p;
     };
     if (fresh) {
-      const auto same = [](T v) { return v; };
-      A.mul(pl, [&](int32_t i) { return shared_load(rv + i); }, same, q);
-      B.mul(psl, [&](int32_t i) { return shared_load(rsv + i); }, same, qs);
+      const auto same = [](T v, double) { return v; };
+      A.mul(pl, beta, [&](int32_t i) { return shared_load(rv + i); }, same, q);
+      B.mul(psl, beta, [&](int32_t i) { return shared_load(rsv + i); }, same, qs);
     } else {
-      const auto near = [&](Raw f) { return (T)(beta * (double)f.p + (double)f.r); };
-      A.mul(pl, [&](int32_t i) { return Raw{shared_load(rv + i), shared_load(old + i)}; }, near, q);
-      B.mul(psl, [&](int32_t i) { return Raw{shared_load(rsv + i), shared_load(old + ld + i)}; }, near, qs);
+      const auto near = [](Raw f, double b) { return direction(b, f.p, f.r); };
+      A.mul(pl, beta, [&](int32_t i) { return Raw{shared_load(rv + i), shared_load(old + i)}; }, near, q);
+      B.mul(psl, beta, [&](int32_t i) { return Raw{shared_load(rsv + i), shared_load(old + ld + i)}; }, near, qs);
     }
     double s1[1] = {0.0};
 #pragma unroll
