@@ -393,10 +393,12 @@ __global__ __launch_bounds__(NT) void k_cg_coop(int64_t n, const int32_t* __rest
 // BiCG (bicg.cpp:162-310), as k_cg_coop: a step is both products (A p and
 // A^T p*), the reduction of
 // (p*, A p), the updates, and the reduction of (r*, r) and (r, r).  vec holds
-// r, r*, then p and p* of even and of odd steps.  Both matrices' entries stay
-// in registers, so FP64 takes at most two rows per thread.
-// Measured (7-point grids, FP64, us a step, on chip against five launches):
-// 16^3 6.3 / 22.9, 32^3 8.6 / 23.9, 50^3 11.9 / 26.7, 64^3 20.7 / 29.8.
+// r, r*, then p and p* of even and of odd steps.  Both matrices' entries are
+// kept, so a thread takes at most two rows (at two, 380 bytes of them in scratch
+// in FP64 and 190 in FP32; BicgLevel::kRpt).
+// Measured (7-point grids, us a step, on chip against five launches): FP64 16^3
+// 6.1 / 23.2, 32^3 8.0 / 23.6, 50^3 11.5 / 27.2, 64^3 20.7 / 28.4; FP32 inside
+// VPGMRES 16^3 7.8 / 24.9, 50^3 13.4 / 25.5, 64^3 18.1 / 25.5.
 template <class T, int NT, int RPT>
 __global__ __launch_bounds__(NT) void k_bicg_coop(int64_t n, const int32_t* __restrict__ ptr,
                                                   const int32_t* __restrict__ col, const T* __restrict__ val,

@@ -450,7 +450,7 @@ void klaunch_n(ks_ctx* c, int cls, void (*kernel)(P...), int G, A&&... args) {
 }
 
 // Whether a solve with A runs on chip (ks_coop.h): rows of at most kCoopRow
-// entries, at most kCoopRpt per thread of one workgroup per CU.  The line is
+// entries, at most `rpt` per thread of one workgroup per CU.  The line is
 // what the registers hold; up to it a step is the faster one on chip (CG, us a
 // step, on chip against three launches: 32 x 32 3.8 / 13.5, 256 x 256 6.4 /
 // 13.3, 512 x 512 8.6 / 16.4, 724 x 724 13.7 / 23.0, 32^3 6.4 / 14.7, 64^3

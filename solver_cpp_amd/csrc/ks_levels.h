@@ -809,7 +809,11 @@ struct BicgLevel : Level {
   DBuf<T> vec;                  // on chip: r, rs, p, ps and two more, in one allocation
   bool coop = false;            // on chip: a unit is kCoopIters steps in one launch (k_bicg_coop)
   const double* src = nullptr;  // on chip: the right-hand side
-  static constexpr int kRpt = sizeof(T) == 8 ? 2 : kCoopRpt;  // rows per thread: what the registers hold twice
+  // rows per thread, of A and A^T each: with four the entries lie in scratch
+  // even in FP32, and a step is slower than by launches (7-point 287496 rows
+  // 52 against 27 us, 512000 53 against 33; 5-point 270400 38 against 26, 524176
+  // 43 against 31)
+  static constexpr int kRpt = 2;
   void setup(ks_ctx* cx, const MatView<T>& a, const MatView<T>& at, const LevelCfg& cf) {
     c = cx; A = a; AT = at; n = a.n; cfg = cf;
     coop = coop_fits(c, A, kRpt) && coop_fits(c, AT, kRpt) && cfg.maxloop > 0;
@@ -849,7 +853,6 @@ struct BicgLevel : Level {
       };
       switch (coop_rows(c, n)) {
         case 1: go(k_bicg_coop<T, kCoopThreads, 1>); break;
-        case 2: go(k_bicg_coop<T, kCoopThreads, 2>); break;
         default: go(k_bicg_coop<T, kCoopThreads, kRpt>); break;
       }
       KS_HIPCK(hipGetLastError());

@@ -1,0 +1,43 @@
+"""Which solves run on chip: up to the sizes where that is the faster way."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+CU_ROWS = 256 * 512  # one row per thread of 256 workgroups
+
+
+def _tridiag(n):
+    i = np.arange(n)
+    row = np.concatenate([i[1:], i, i[:-1]])
+    col = np.concatenate([i[:-1], i, i[1:]])
+    val = np.concatenate([np.full(n - 1, -1.1), np.full(n, 3.0), np.full(n - 1, -0.9)])
+    return _csr(n, row, col, val)
+
+
+def _csr(n, row, col, val):
+    o = np.lexsort((col, row))
+    ptr = np.zeros(n + 1, np.int32)
+    ptr[1:] = np.cumsum(np.bincount(row, minlength=n))
+    return ptr, col[o].astype(np.int32), val[o]
+
+
+def _runs_on_chip(ctx, A, b, outer, inner, **kw):
+    from solver_cpp_amd import api
+    before = ctx.on_chip()
+    x, r, _ = api.solve(ctx, A, b, outer, inner, history=False, outer_eps=1e-10, outer_maxloop=300, **kw)
+    assert r["status"] == 0 and r["relres_true"] < 1e-9
+    after = ctx.on_chip()
+    assert after["repeated"] == before["repeated"]
+    return after["solves"] > before["solves"]
+
+
+@pytest.mark.parametrize("prec", [64, 32])
+@pytest.mark.parametrize("n", [2 * CU_ROWS, 2 * CU_ROWS + 1, 4 * CU_ROWS])
+def test_bicg_takes_two_rows_per_thread(ctx, n, prec):
+    from solver_cpp_amd import api
+    A = api.Matrix(ctx, *_tridiag(n), fp32=True, transpose=True)
+    b = np.random.default_rng(71).uniform(-1, 1, n)
+    got = _runs_on_chip(ctx, A, b, "vpgmres", "bicg", outer_restart=20, inner_maxloop=10, inner_precision=prec)
+    assert got == (n <= 2 * CU_ROWS)
+    A.close()
