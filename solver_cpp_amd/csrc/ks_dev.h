@@ -229,6 +229,7 @@ struct MatView {
   bool wg_tiles = false;
   int L = 8;
   int64_t max_row = 0;
+  bool scattered = false;  // rows that an on-chip solve would gather one by one (A's: A^T has the same distances)
   int64_t ntiles = 0;
   const int32_t* tiles = nullptr;
   const int32_t* tnz = nullptr;
@@ -321,6 +322,7 @@ struct ks_mat {
   ks::BinSet bins, tbins;
   ks::DBuf<double> xg;  // their x by entry, used by one product at a time
   int64_t max_row = 0, max_trow = 0;
+  bool scattered = false;
 
   template <class T>
   ks::MatView<T> view(bool trans) const;
@@ -350,6 +352,7 @@ inline ks::MatView<double> ks_mat::view<double>(bool trans) const {
   v.n = n; v.nnz = nnz;
   const ks::Plan& pl = trans ? tplan : plan;
   v.max_row = trans ? max_trow : max_row;
+  v.scattered = scattered;
   if (trans) { v.ptr = tptr.p; v.col = tcol.p; v.val = tval.p; }
   else { v.ptr = ptr.p; v.col = col.p; v.val = val.p; }
   v.set_plan(pl);
@@ -366,6 +369,7 @@ inline ks::MatView<float> ks_mat::view<float>(bool trans) const {
   v.n = n; v.nnz = nnz;
   const ks::Plan& pl = trans ? tplan : plan;
   v.max_row = trans ? max_trow : max_row;
+  v.scattered = scattered;
   if (trans) { v.ptr = tptr.p; v.col = tcol.p; v.val = tval32.p; }
   else { v.ptr = ptr.p; v.col = col.p; v.val = val32.p; }
   v.set_plan(pl);
@@ -450,14 +454,19 @@ void klaunch_n(ks_ctx* c, int cls, void (*kernel)(P...), int G, A&&... args) {
 }
 
 // Whether a solve with A runs on chip (ks_coop.h): rows of at most kCoopRow
-// entries, at most `rpt` per thread of one workgroup per CU.  The line is
-// what the registers hold; up to it a step is the faster one on chip (CG, us a
-// step, on chip against three launches: 32 x 32 3.8 / 13.5, 256 x 256 6.4 /
-// 13.3, 512 x 512 8.6 / 16.4, 724 x 724 13.7 / 23.0, 32^3 6.4 / 14.7, 64^3
-// 9.3 / 16.8, 80^3 23.0 / 25.0; VPCG with ten FP32 CG steps, 300 x 300 102 /
-// 173).
+// entries, at most `rpt` per thread of one workgroup per CU.  Four rows per
+// thread of CG is about where a step stops being the faster one on chip (some of
+// their entries lie in scratch: 370 bytes in FP64, 80 in FP32).  CG, us a step, on
+// chip against three launches: 5-point 256 x 256 6.0 / 14.5, 512 x 512 8.3 /
+// 16.6, 724 x 724 14.2 / 21.4; 7-point 32^3 6.2 / 15.4, 63^3 9.3 / 21.3, 80^3
+// 22.9 / 22.8, and in FP32 inside VPGMRES 13.3 / 20.6.  Rows that gather more
+// than 2.5 elements one by one take at most two per thread: seven entries at
+// random, FP64 262144 rows 26 / 33, 350000 51 / 42, 500000 61 / 47; five, 22 / 28,
+// 40 / 38, 51 / 41; three (two of them far), 18 / 23, 27 / 29, 36 / 34, and in FP32
+// 500000 24 / 27.
 template <class T>
 bool coop_fits(const ks_ctx* c, const MatView<T>& A, int rpt = kCoopRpt) {
+  if (A.scattered) rpt = std::min(rpt, 2);
   return !c->coop_off && c->coop_spin > 0 && A.kind == 0 && A.max_row <= kCoopRow &&
          A.n <= (int64_t)rpt * kCoopThreads * std::min(c->num_cus, kCoopMaxWg);
 }

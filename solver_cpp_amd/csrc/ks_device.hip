@@ -175,6 +175,25 @@ bool bin_choice(uint32_t flags, int64_t n, int64_t nnz, int64_t max_row, const i
          gathers_far(n, hp, hc);
 }
 
+// Whether a row gathers more than 2.5 elements one by one from other
+// workgroups of an on-chip solve (mean over sampled rows): entries half a
+// workgroup's rows or more away whose neighbour the next row does not gather
+// (a stencil's rows gather runs).  Only asked where that decides (coop_fits).
+bool scattered_rows(int64_t n, const int32_t* hp, const int32_t* hc) {
+  constexpr int64_t kWgRows = (int64_t)kCoopRpt * kCoopThreads;
+  if (n <= kWgRows * kCoopMaxWg / 2 || n > kWgRows * kCoopMaxWg) return false;
+  int64_t far = 0, rows = 0;
+  for (int64_t r = 0; r + 1 < n; r += 61) {
+    if (hp[r + 1] - hp[r] > kCoopRow || hp[r + 2] - hp[r + 1] > kCoopRow) continue;
+    ++rows;
+    for (int32_t j = hp[r]; j < hp[r + 1]; ++j) {
+      if (std::llabs((int64_t)hc[j] - r) < kWgRows / 2) continue;
+      far += std::find(hc + hp[r + 1], hc + hp[r + 2], hc[j] + 1) == hc + hp[r + 2];
+    }
+  }
+  return 2 * far > 5 * rows;
+}
+
 // Column blocks of the CSR (ptr, col; hp: host row pointers).
 void build_bins(ks_mat* m, BinSet& bs, const int32_t* hp, const int32_t* ptr, const int32_t* col) {
   ks_ctx* c = m->ctx;
@@ -1150,6 +1169,7 @@ ks_status ks_mat_create_csr(ks_ctx* c, int64_t n, int64_t nnz, const int32_t* pt
   m->max_row = mx;
   KS_CHECK(!((flags & KS_MAT_COL32) && (flags & KS_MAT_COL_DELTA)), KS_ERR_BAD_INPUT,
            "KS_MAT_COL32 and KS_MAT_COL_DELTA exclude each other");
+  m->scattered = scattered_rows(n, hp.data(), hc.data());
   if (bin_choice(flags, n, nnz, mx, hp.data(), hc.data())) {
     m->plan.L = choose_lanes(n, nnz);
     m->plan.kind = 2;  // no tiles: the bins are the plan

@@ -41,3 +41,43 @@ def test_bicg_takes_two_rows_per_thread(ctx, n, prec):
     got = _runs_on_chip(ctx, A, b, "vpgmres", "bicg", outer_restart=20, inner_maxloop=10, inner_precision=prec)
     assert got == (n <= 2 * CU_ROWS)
     A.close()
+
+
+def _random_rows(n, pairs):
+    # the diagonal, and both directions of `pairs` random permutations
+    rng = np.random.default_rng(72)
+    i = np.arange(n)
+    row, col, val = [i], [i], [np.full(n, 2.2 * pairs)]
+    for _ in range(pairs):
+        p = rng.permutation(n)
+        row, col, val = row + [i, p], col + [p, i], val + [np.full(n, -1.0)] * 2
+    return _csr(n, np.concatenate(row), np.concatenate(col), np.concatenate(val))
+
+
+def _box(nx, ny, nz):
+    from solver_cpp_amd import gen
+    ptr, col, val = gen.stencil(3, nx, ny, nz)
+    return ptr, col, np.where(col == np.repeat(np.arange(nx * ny * nz), np.diff(ptr)), val + 1.0, val)
+
+
+@pytest.mark.parametrize("outer,inner,kw", [("cg", "NO", {}),
+                                            ("vpcg", "cg", dict(inner_maxloop=10, inner_precision=32))])
+@pytest.mark.parametrize("name,make,yes", [
+    ("random_7_two_rows", lambda: _random_rows(2 * CU_ROWS, 3), True),
+    ("random_7_four_rows", lambda: _random_rows(2 * CU_ROWS + 1, 3), False),
+    ("random_5_four_rows", lambda: _random_rows(4 * CU_ROWS, 2), False),
+    ("random_3_four_rows", lambda: _random_rows(300_000, 1), True),
+    ("thin_box", lambda: _box(2048, 16, 16), True),  # four neighbours in other workgroups, in runs
+    ("cube", lambda: _box(70, 70, 70), True),
+    ("line", lambda: _tridiag(4 * CU_ROWS), True),
+    ("line_too_long", lambda: _tridiag(4 * CU_ROWS + 1), False),
+])
+def test_cg_with_four_rows_per_thread_gathers_runs(ctx, name, make, yes, outer, inner, kw):
+    from solver_cpp_amd import api
+    ptr, col, val = make()
+    if name.startswith("line"):
+        val = np.where(val < 0, -1.0, val)  # symmetric
+    A = api.Matrix(ctx, ptr, col, val, fp32=True, spd=True)
+    b = np.random.default_rng(73).uniform(-1, 1, len(ptr) - 1)
+    assert _runs_on_chip(ctx, A, b, outer, inner, **kw) == yes
+    A.close()
