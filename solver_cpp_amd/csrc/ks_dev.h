@@ -540,6 +540,12 @@ int spmv_L(ks_ctx* c, const MatView<T>& A, const T* x, const Epi& epi, Gate g, i
   return G;
 }
 
+// The epilogues of column panels, whose views have int32 columns only.
+template <class E, class = void>
+struct IsPanel : std::false_type {};
+template <class E>
+struct IsPanel<E, std::void_t<decltype(E::kPanel)>> : std::true_type {};
+
 // The workgroup CSR-stream SpMV in the view's column index format, on G
 // workgroups.  With reductions (NV > 0 or a projection) G is always the int32
 // kernel's grid (stream_grid): the grid, and so the reduction partials and
@@ -550,26 +556,27 @@ int spmv_L(ks_ctx* c, const MatView<T>& A, const T* x, const Epi& epi, Gate g, i
 template <class T, int NX, int NV, class Epi>
 void launch_stream(ks_ctx* c, int cls, const MatView<T>& A, int G, const T* x0, const T* x1, const Epi& epi, Gate g,
                    double bytes) {
-  if (A.row)
-    klaunch(c, cls, k_spmv_rows<T, NX, NV, Epi>, G, 0, A.n, A.ntiles, A.tiles, A.rtab, A.row, A.rval, x0, x1, epi,
-             g, red(c), stat(c, cls, bytes));
-  else if (A.pat)
-    klaunch(c, cls, k_spmv_stream<T, NX, NV, Epi, PatIx>, G, 0, A.n, A.ntiles, A.tiles, A.tnz, A.ptab, A.pat, A.val,
-            x0, x1, epi, g, red(c), stat(c, cls, bytes));
-  else if (A.col16)
-    klaunch(c, cls, k_spmv_stream<T, NX, NV, Epi, int16_t>, G, 0, A.n, A.ntiles, A.tiles, A.tnz, A.ptr, A.col16,
-            A.val, x0, x1, epi, g, red(c), stat(c, cls, bytes));
-  else if (A.cold)
-    klaunch(c, cls, k_spmv_stream<T, NX, NV, Epi, uint16_t>, G, 0, A.n, A.ntiles, A.tiles, A.tnz, A.ptr, A.cold,
-            A.val, x0, x1, epi, g, red(c), stat(c, cls, bytes));
-  else
-    klaunch(c, cls, k_spmv_stream<T, NX, NV, Epi>, G, 0, A.n, A.ntiles, A.tiles, A.tnz, A.ptr, A.col, A.val, x0, x1,
-            epi, g, red(c), stat(c, cls, bytes));
+  if constexpr (!IsPanel<Epi>::value) {
+    if (A.row)
+      return klaunch(c, cls, k_spmv_rows<T, NX, NV, Epi>, G, 0, A.n, A.ntiles, A.tiles, A.rtab, A.row, A.rval, x0, x1,
+                     epi, g, red(c), stat(c, cls, bytes));
+    if (A.pat)
+      return klaunch(c, cls, k_spmv_stream<T, NX, NV, Epi, PatIx>, G, 0, A.n, A.ntiles, A.tiles, A.tnz, A.ptab, A.pat,
+                     A.val, x0, x1, epi, g, red(c), stat(c, cls, bytes));
+    if (A.col16)
+      return klaunch(c, cls, k_spmv_stream<T, NX, NV, Epi, int16_t>, G, 0, A.n, A.ntiles, A.tiles, A.tnz, A.ptr,
+                     A.col16, A.val, x0, x1, epi, g, red(c), stat(c, cls, bytes));
+    if (A.cold)
+      return klaunch(c, cls, k_spmv_stream<T, NX, NV, Epi, uint16_t>, G, 0, A.n, A.ntiles, A.tiles, A.tnz, A.ptr,
+                     A.cold, A.val, x0, x1, epi, g, red(c), stat(c, cls, bytes));
+  }
+  klaunch(c, cls, k_spmv_stream<T, NX, NV, Epi>, G, 0, A.n, A.ntiles, A.tiles, A.tnz, A.ptr, A.col, A.val, x0, x1,
+          epi, g, red(c), stat(c, cls, bytes));
 }
 
 template <class T, int NX, int NV, class Epi>
 int stream_grid(ks_ctx* c, const MatView<T>& A) {
-  if constexpr (NV == 0 && !HasProj<Epi>::value) {
+  if constexpr (NV == 0 && !HasProj<Epi>::value && !IsPanel<Epi>::value) {
     if (A.row) return grid_rows(c, k_spmv_rows<T, NX, NV, Epi>, A.ntiles);
     if (A.pat) return grid_rows(c, k_spmv_stream<T, NX, NV, Epi, PatIx>, A.ntiles);
     if (A.col16) return grid_rows(c, k_spmv_stream<T, NX, NV, Epi, int16_t>, A.ntiles);
@@ -634,6 +641,7 @@ int spmv_dispatch(ks_ctx* c, const MatView<T>& A, const T* x, const Epi& epi, Ga
 // row sums into pacc; the last adds pacc to its own and runs the epilogue.
 template <class T>
 struct EpiPanelAcc {
+  static constexpr bool kPanel = true;
   T* acc;
   int first;
   __device__ void prep() {}
@@ -643,6 +651,7 @@ struct EpiPanelAcc {
 };
 template <class T, class Epi>
 struct EpiPanelLast {
+  static constexpr bool kPanel = true;
   Epi e;
   const T* acc;
   __device__ void prep() { e.prep(); }
