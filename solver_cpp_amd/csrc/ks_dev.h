@@ -230,6 +230,7 @@ struct MatView {
   int L = 8;
   int64_t max_row = 0;
   bool scattered = false;  // rows that an on-chip solve would gather one by one (A's: A^T has the same distances)
+  bool runs = false;       // wavefronts gather runs of x (A's; looked at only without row patterns)
   int64_t ntiles = 0;
   const int32_t* tiles = nullptr;
   const int32_t* tnz = nullptr;
@@ -322,7 +323,7 @@ struct ks_mat {
   ks::BinSet bins, tbins;
   ks::DBuf<double> xg;  // their x by entry, used by one product at a time
   int64_t max_row = 0, max_trow = 0;
-  bool scattered = false;
+  bool scattered = false, runs = false;
 
   template <class T>
   ks::MatView<T> view(bool trans) const;
@@ -353,6 +354,7 @@ inline ks::MatView<double> ks_mat::view<double>(bool trans) const {
   const ks::Plan& pl = trans ? tplan : plan;
   v.max_row = trans ? max_trow : max_row;
   v.scattered = scattered;
+  v.runs = runs;
   if (trans) { v.ptr = tptr.p; v.col = tcol.p; v.val = tval.p; }
   else { v.ptr = ptr.p; v.col = col.p; v.val = val.p; }
   v.set_plan(pl);
@@ -370,6 +372,7 @@ inline ks::MatView<float> ks_mat::view<float>(bool trans) const {
   const ks::Plan& pl = trans ? tplan : plan;
   v.max_row = trans ? max_trow : max_row;
   v.scattered = scattered;
+  v.runs = runs;
   if (trans) { v.ptr = tptr.p; v.col = tcol.p; v.val = tval32.p; }
   else { v.ptr = ptr.p; v.col = col.p; v.val = val32.p; }
   v.set_plan(pl);
@@ -546,43 +549,71 @@ struct IsPanel : std::false_type {};
 template <class E>
 struct IsPanel<E, std::void_t<decltype(E::kPanel)>> : std::true_type {};
 
+// Whether k_spmv_stream's gathers go out ahead of the next tile's loads: where the
+// lanes of a wavefront gather runs of x (row patterns, or A.runs with at most ten
+// entries a lane, about what goes out ahead) and rows are long enough to fill the
+// slots.  Measured, us per product, ahead / behind:
+//  runs: 7-point 150^3 by patterns FP32 26.6 / 30.0, FP64 49.9 / 48.3, 40^3 FP64 5.2 /
+//  5.5; 16 x 16 blocks, 2^20 rows, FP64 31.5 / 34.9; 2^22 rows of five diagonals and a
+//  varying column, int16, FP32 36.9 / 39.2, FP64 58.3 / 60.1;
+//  longer rows: 27-point 150^3 by int32 columns FP64 255 / 244, FP32 172 / 161;
+//  no runs: 2^22 rows of 1 .. 19 entries anywhere FP64 656 / 520, FP32 462 / 373, of 1
+//  .. 7 FP64 473 / 404; 2^20 rows of 1 .. 199 within 5000 columns FP64 444 / 385, FP32
+//  334 / 272;
+//  short rows, 2^22: one entry FP64 43.5 / 32.2, FP32 24.8 / 23.2, two FP64 45.4 / 35.9,
+//  three by patterns FP64 44.3 / 33.7, FP32 26.2 / 26.4.
+template <class T>
+bool gathers_ahead(const MatView<T>& A) {
+  const double mean = (double)A.nnz / (double)std::max<int64_t>(A.n, 1);
+  if (mean <= (sizeof(T) == 8 ? 3.5 : 2.5)) return false;
+  if (A.pat) return true;
+  const int nr = (int)std::min<double>(kTileRows, kTileNnz / mean);  // of a full tile
+  return A.runs && mean <= 10.0 * tile_lanes(nr, (int)(nr * mean));
+}
+
 // The workgroup CSR-stream SpMV in the view's column index format, on G
 // workgroups.  With reductions (NV > 0 or a projection) G is always the int32
 // kernel's grid (stream_grid): the grid, and so the reduction partials and
 // their summation order, is the same in every index format, so a solve's
 // results do not depend on the format (the 16-bit kernels, which need fewer
 // registers, may have room for more workgroups than they are given).
-// Without reductions each format fills its own residency.
+// Without reductions each kernel fills its own residency.
+template <class T, int NX, int NV, class Epi, class F>
+auto with_stream_kernel(const MatView<T>& A, F f) {  // f(kernel, its first index array, its second)
+  auto pick = [&](auto ahead) {
+    constexpr bool K = decltype(ahead)::value;
+    if (A.pat) return f(k_spmv_stream<T, NX, NV, Epi, PatIx, K>, A.ptab, A.pat);
+    if (A.col16) return f(k_spmv_stream<T, NX, NV, Epi, int16_t, K>, A.ptr, A.col16);
+    if (A.cold) return f(k_spmv_stream<T, NX, NV, Epi, uint16_t, K>, A.ptr, A.cold);
+    return f(k_spmv_stream<T, NX, NV, Epi, int32_t, K>, A.ptr, A.col);
+  };
+  if constexpr (IsPanel<Epi>::value) return f(k_spmv_stream<T, NX, NV, Epi, int32_t, false>, A.ptr, A.col);
+  else return gathers_ahead(A) ? pick(std::true_type{}) : pick(std::false_type{});
+}
 template <class T, int NX, int NV, class Epi>
 void launch_stream(ks_ctx* c, int cls, const MatView<T>& A, int G, const T* x0, const T* x1, const Epi& epi, Gate g,
                    double bytes) {
-  if constexpr (!IsPanel<Epi>::value) {
+  if constexpr (!IsPanel<Epi>::value)
     if (A.row)
       return klaunch(c, cls, k_spmv_rows<T, NX, NV, Epi>, G, 0, A.n, A.ntiles, A.tiles, A.rtab, A.row, A.rval, x0, x1,
                      epi, g, red(c), stat(c, cls, bytes));
-    if (A.pat)
-      return klaunch(c, cls, k_spmv_stream<T, NX, NV, Epi, PatIx>, G, 0, A.n, A.ntiles, A.tiles, A.tnz, A.ptab, A.pat,
-                     A.val, x0, x1, epi, g, red(c), stat(c, cls, bytes));
-    if (A.col16)
-      return klaunch(c, cls, k_spmv_stream<T, NX, NV, Epi, int16_t>, G, 0, A.n, A.ntiles, A.tiles, A.tnz, A.ptr,
-                     A.col16, A.val, x0, x1, epi, g, red(c), stat(c, cls, bytes));
-    if (A.cold)
-      return klaunch(c, cls, k_spmv_stream<T, NX, NV, Epi, uint16_t>, G, 0, A.n, A.ntiles, A.tiles, A.tnz, A.ptr,
-                     A.cold, A.val, x0, x1, epi, g, red(c), stat(c, cls, bytes));
-  }
-  klaunch(c, cls, k_spmv_stream<T, NX, NV, Epi>, G, 0, A.n, A.ntiles, A.tiles, A.tnz, A.ptr, A.col, A.val, x0, x1,
-          epi, g, red(c), stat(c, cls, bytes));
+  with_stream_kernel<T, NX, NV, Epi>(A, [&](auto kernel, const int32_t* ptr, auto col) {
+    klaunch(c, cls, kernel, G, 0, A.n, A.ntiles, A.tiles, A.tnz, ptr, col, A.val, x0, x1, epi, g, red(c),
+            stat(c, cls, bytes));
+  });
 }
 
 template <class T, int NX, int NV, class Epi>
 int stream_grid(ks_ctx* c, const MatView<T>& A) {
-  if constexpr (NV == 0 && !HasProj<Epi>::value && !IsPanel<Epi>::value) {
+  if constexpr (IsPanel<Epi>::value) {
+    return grid_rows(c, k_spmv_stream<T, NX, NV, Epi, int32_t, false>, A.ntiles);
+  } else if constexpr (NV == 0 && !HasProj<Epi>::value) {
     if (A.row) return grid_rows(c, k_spmv_rows<T, NX, NV, Epi>, A.ntiles);
-    if (A.pat) return grid_rows(c, k_spmv_stream<T, NX, NV, Epi, PatIx>, A.ntiles);
-    if (A.col16) return grid_rows(c, k_spmv_stream<T, NX, NV, Epi, int16_t>, A.ntiles);
-    if (A.cold) return grid_rows(c, k_spmv_stream<T, NX, NV, Epi, uint16_t>, A.ntiles);
+    return with_stream_kernel<T, NX, NV, Epi>(
+        A, [&](auto kernel, const int32_t*, auto) { return grid_rows(c, kernel, A.ntiles); });
+  } else {
+    return grid_rows(c, k_spmv_stream<T, NX, NV, Epi, int32_t, true>, A.ntiles);
   }
-  return grid_rows(c, k_spmv_stream<T, NX, NV, Epi>, A.ntiles);
 }
 
 template <class T, int NX, int NV, class Epi>

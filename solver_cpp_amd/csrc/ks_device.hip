@@ -194,6 +194,23 @@ bool scattered_rows(int64_t n, const int32_t* hp, const int32_t* hc) {
   return 2 * far > 5 * rows;
 }
 
+// Whether the lanes of a wavefront gather runs of x: over half of the entries of
+// some thousand sampled rows lie within a cache line (8 columns) of the entry that
+// the next lane gathers with them, which is the next row's entry at the same place,
+// or with several lanes a row (over 8 entries on average) the row's next one.
+bool gathers_runs(int64_t n, const int32_t* hp, const int32_t* hc) {
+  const bool lanes = hp[n] > 8 * n;
+  auto near = [&](int32_t a, int32_t b) { return std::abs((int64_t)hc[a] - hc[b]) <= 8; };
+  int64_t runs = 0, all = 0;
+  for (int64_t r = 0; r + 1 < n; r += n / 1024 | 1)
+    for (int32_t j = hp[r], e = std::min(hp[r + 1], hp[r] + 64); j < e; ++j) {
+      const int32_t below = hp[r + 1] + (j - hp[r]);
+      ++all;
+      runs += (below < hp[r + 2] && near(j, below)) || (lanes && j + 1 < hp[r + 1] && near(j, j + 1));
+    }
+  return 2 * runs > all;
+}
+
 // Column blocks of the CSR (ptr, col; hp: host row pointers).
 void build_bins(ks_mat* m, BinSet& bs, const int32_t* hp, const int32_t* ptr, const int32_t* col) {
   ks_ctx* c = m->ctx;
@@ -1182,6 +1199,13 @@ ks_status ks_mat_create_csr(ks_ctx* c, int64_t n, int64_t nnz, const int32_t* pt
   }
   if (flags & KS_MAT_TRANSPOSE) build_transpose(m.get());
   if (!(flags & KS_MAT_COL32) && nnz > 0) build_index16(m.get(), hp.data(), hc.data());
+  // asked where a product reads column indices, or may once new values end its classes
+  auto entries = [](const Plan& pl, const RowBuf& rows, const PatBuf& pat, bool other) {
+    return pl.kind == 0 && !pat.code && (!rows.code || other);
+  };
+  if (entries(m->plan, m->rows, m->pat, m->col16.p || m->cold.p) ||
+      (m->has_t && entries(m->tplan, m->trows, m->tpat, m->tcol16.p || m->tcold.p)))
+    m->runs = gathers_runs(n, hp.data(), hc.data());
   if (flags & KS_MAT_FP32_COPY) ensure_fp32(m.get());
   KS_HIPCK(hipStreamSynchronize(c->stream));
   *out = m.release();

@@ -394,6 +394,11 @@ struct Chunk {
   typedef U type __attribute__((ext_vector_type(W)));
 };
 
+// How a tile is loaded: every chunk of its window by every lane (the window lies
+// below nnz), the chunks that hold entries of the tile (the same), or entry by
+// entry where a chunk would pass nnz.
+enum class Load { kAll, kWindow, kEntries };
+
 // One array's share of a tile for one thread: NTH threads cover a window of
 // WIN entries from a0, thread t taking the W-entry chunks at a0 + W t +
 // W NTH i, so each load instruction reads one chunk per lane from
@@ -402,16 +407,16 @@ template <class U, int NTH, int WIN, int W>
 struct TileArr {
   static constexpr int kN = WIN / (W * NTH);
   U x[kN][W];
-  // kFull: the whole window [a0, a0 + WIN) lies below nnz (uniform across
+  // kWindow: the whole window [a0, a0 + WIN) lies below nnz (uniform across
   // the tile), so no lane needs the entry-by-entry path; keeping that path
   // out of the common case keeps the chunk loads back to back.  full(a0, nnz)
   // is that condition.
-  template <bool kFull>
+  template <Load kLoad>
   __device__ __forceinline__ void load(const U* __restrict__ p, int32_t a0, int32_t j1, int32_t nnz, int t) {
 #pragma unroll
     for (int i = 0; i < kN; ++i) {
       const int32_t e = a0 + W * t + W * NTH * i;
-      if constexpr (kFull) {
+      if constexpr (kLoad == Load::kAll) {
         // every lane loads, those past the tile its first chunk again (one
         // more cache line): no branch, so the number of loads in flight is
         // known and earlier ones can be waited for without these
@@ -420,7 +425,7 @@ struct TileArr {
 #pragma unroll
         for (int h = 0; h < W; ++h) x[i][h] = q[h];
       } else if (e < j1) {
-        if (e + W - 1 < nnz) {
+        if (kLoad == Load::kWindow || e + W - 1 < nnz) {
           const typename Chunk<U, W>::type q = ld_stream(reinterpret_cast<const typename Chunk<U, W>::type*>(p + e));
 #pragma unroll
           for (int h = 0; h < W; ++h) x[i][h] = q[h];
@@ -463,22 +468,23 @@ struct QuadTile {
   TileArr<IX, NTH, WIN, WC> c;
   int32_t pr;
   __device__ static __forceinline__ bool full(int32_t j0, int32_t nnz) { return a0of(j0) + WIN <= nnz; }
-  // kFull: full(j0, nnz) holds; a row longer than a tile is loaded in place
-  template <bool kFull>
+  // kAll, kWindow: full(j0, nnz) holds; a row longer than a tile is loaded in place
+  template <Load kLoad>
   __device__ __forceinline__ void load(const int32_t* __restrict__ ptr, const IX* __restrict__ col,
                                        const T* __restrict__ val, int32_t r0, int32_t r1, int32_t j0, int32_t j1,
                                        int32_t nnz, int t) {
     const int32_t a0 = a0of(j0);
-    v.template load<kFull>(val, a0, j1, nnz, t);
-    c.template load<kFull>(col, a0, j1, nnz, t);
-    pr = ptr[t < r1 - r0 ? r0 + t : r1];
+    v.template load<kLoad>(val, a0, j1, nnz, t);
+    c.template load<kLoad>(col, a0, j1, nnz, t);
+    if constexpr (kLoad == Load::kAll) pr = ptr[t < r1 - r0 ? r0 + t : r1];
+    else pr = t < r1 - r0 ? ptr[r0 + t] : 0;
   }
   __device__ __forceinline__ void load(const int32_t* __restrict__ ptr, const IX* __restrict__ col,
                                        const T* __restrict__ val, int32_t r0, int32_t r1, int32_t j0, int32_t j1,
                                        int32_t nnz, int t) {
     if (j1 - j0 > WIN - kA + 1) return;
-    if (full(j0, nnz)) load<true>(ptr, col, val, r0, r1, j0, j1, nnz, t);
-    else load<false>(ptr, col, val, r0, r1, j0, j1, nnz, t);
+    if (full(j0, nnz)) load<Load::kWindow>(ptr, col, val, r0, r1, j0, j1, nnz, t);
+    else load<Load::kEntries>(ptr, col, val, r0, r1, j0, j1, nnz, t);
   }
   __device__ __forceinline__ void stage(T* sv, IX* sc, int32_t j0, int32_t j1, int t) const {
     const int32_t span = j1 - a0of(j0);
@@ -491,7 +497,7 @@ using TileData = QuadTile<T, kBlock, kTileWin, IX>;
 
 // Lanes per row of a CSR-stream tile of nr rows and cnt entries: more than
 // one only for rows averaging over 8 entries.
-__device__ __forceinline__ int tile_lanes(int nr, int cnt) {
+__host__ __device__ __forceinline__ int tile_lanes(int nr, int cnt) {
   int tpr = 1;
   while (tpr < 64 && tpr * 2 * nr <= kBlock && tpr * 8 * nr < cnt) tpr *= 2;
   return tpr;
@@ -528,17 +534,17 @@ struct PatTile {
   TileArr<T, kBlock, kTileWin, W> v;
   int32_t pr;
   __device__ static __forceinline__ bool full(int32_t j0, int32_t nnz) { return a0of(j0) + kTileWin <= nnz; }
-  template <bool kFull>
+  template <Load kLoad>
   __device__ __forceinline__ void load(const int32_t*, const PatIx* __restrict__ code, const T* __restrict__ val,
                                        int32_t r0, int32_t r1, int32_t j0, int32_t j1, int32_t nnz, int t) {
-    v.template load<kFull>(val, a0of(j0), j1, nnz, t);
+    v.template load<kLoad>(val, a0of(j0), j1, nnz, t);
     const int grp = t / tile_lanes(r1 - r0, j1 - j0);
     pr = (int32_t)code[grp < r1 - r0 ? r0 + grp : r0].v;
   }
   __device__ __forceinline__ void load(const int32_t* ptr, const PatIx* __restrict__ code, const T* __restrict__ val,
                                        int32_t r0, int32_t r1, int32_t j0, int32_t j1, int32_t nnz, int t) {
-    if (full(j0, nnz)) load<true>(ptr, code, val, r0, r1, j0, j1, nnz, t);
-    else load<false>(ptr, code, val, r0, r1, j0, j1, nnz, t);
+    if (full(j0, nnz)) load<Load::kWindow>(ptr, code, val, r0, r1, j0, j1, nnz, t);
+    else load<Load::kEntries>(ptr, code, val, r0, r1, j0, j1, nnz, t);
   }
 };
 // Row classes: see ks_rows.h.
@@ -727,8 +733,13 @@ __device__ __forceinline__ void proj_tiles(const int32_t* __restrict__ tiles, co
 // row is a tile of its own.
 // In every format the row sums are the same: entry for entry, the same x is
 // gathered in the same order.
+// kAhead: whether the x gathers go out before the next tile's loads or behind
+// them (gathers_ahead, which holds the figures).  Vector memory answers loads in
+// the order they were issued, so gathers that go first wait for an L2 hit and not
+// for HBM; but each takes a cache line a lane where the lanes of a wavefront do not
+// share lines, and then the next tile's loads queue up behind them.
 constexpr int32_t kDeltaBias = 49152;
-// x gathers of a row in flight before the next tile's loads: the rows of a
+// kAhead: x gathers of a row before the next tile's loads: the rows of a
 // 7-point stencil whole, where the registers hold them without spilling (the
 // kernels with int32 or, in FP64, any per-entry indices keep fewer).
 template <class T, int NX, class IX>
@@ -736,7 +747,7 @@ constexpr int kGathers = std::is_same<IX, PatIx>::value         ? 8
                          : sizeof(IX) == 4 || (sizeof(T) == 8 && NX == 2) ? 4
                          : sizeof(T) == 4                       ? 8
                                                                 : 6;
-template <class T, int NX, int NV, class Epi, class IX = int32_t>
+template <class T, int NX, int NV, class Epi, class IX, bool kAhead>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kWgWaves<T, NX, NV>))) void k_spmv_stream(int64_t n, int64_t ntiles, const int32_t* __restrict__ tiles,
                                                         const int32_t* __restrict__ tnz,
                                                         const int32_t* __restrict__ ptr,
@@ -861,6 +872,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kWgWaves
         d.stage(sv, sc, j0, j1, tid);
       }
       __syncthreads();
+      if constexpr (!kAhead) {  // in flight during the sums
+        if (more) d.load(ptr, col, val, nr0, nr1, nj0, nj1, nnz, tid);
+        nx = bounds(t + 2 * step);
+      }
       // the row's entries s .. e - 1 of the window (none without a row)
       int s, e;
       [[maybe_unused]] const int32_t* off = nullptr;  // kPat: the row's offsets, its first entry's at off[s]
@@ -870,8 +885,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kWgWaves
         e = act ? s + stab[1 + p] : s;
         off = stab + (1 + kPatMax + p * pstride) - s;
       } else {
-        s = sptr[act ? grp : nr];
-        e = sptr[act ? grp + 1 : nr];
+        if constexpr (kAhead) {
+          s = sptr[act ? grp : nr];
+          e = sptr[act ? grp + 1 : nr];
+        } else {
+          s = e = 0;
+          if (act) { s = sptr[grp]; e = sptr[grp + 1]; }
+        }
       }
       const int64_t row = r0 + (act ? grp : 0);
       const int cb = kRel || kPat ? (int)row : kDelta ? (int)row - kDeltaBias : 0;
@@ -881,13 +901,25 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kWgWaves
         else if constexpr (kDelta) return cd += (int)sc[k];
         else return cb + (int)sc[k];
       };
-      // Vector memory answers loads in the order they were issued, so the x
-      // gathers of the row's first kGB entries and the epilogue's operand go
-      // out before the next tile's loads: the sums then wait for an L2 hit
-      // and not for HBM (160^3: FP32 34.9 -> 29.6 us with row patterns, int16
-      // offsets 47.8 -> 42.7 us in FP32 and 75.0 -> 69.4 us in FP64; a second
-      // tile in flight behind it gave nothing more).  Slots past the row's end
-      // gather x of its row.
+      // kAhead: the gathers of the row's first kGB entries and the epilogue's
+      // operand, then the next tile's loads (160^3: FP32 34.9 -> 29.6 us with row
+      // patterns, int16 offsets 47.8 -> 42.7 us in FP32 and 75.0 -> 69.4 us in FP64;
+      // a second tile in flight behind it gave nothing more).  Slots past the
+      // row's end gather x of its row.
+      auto finish = [&](T a0, T a1, auto pv) {
+        for (int off = tpr >> 1; off > 0; off >>= 1) {
+          a0 += __shfl_xor(a0, off, 64);
+          if (NX == 2) a1 += __shfl_xor(a1, off, 64);
+        }
+        if (act && lane == 0) {
+          if constexpr (kYT > 0) {
+            if (slot < kYT) sy[slot][(r0 & 3) + grp] = epi.value(a0);
+            else epi.row(row, a0, a1, acc, pv);
+          } else {
+            epi.row(row, a0, a1, acc, pv);
+          }
+        }
+      };
       auto sums = [&](auto next_tag) {
         constexpr int kNext = decltype(next_tag)::value;  // next tile: 0 none, 1 its full window, 2 entry by entry
         T g0[kGB], g1[kGB];
@@ -899,7 +931,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kWgWaves
           if (NX == 2) g1[q] = x1[c];
         }
         const auto pv = epi.pre(row);
-        if constexpr (kNext == 1) d.template load<true>(ptr, col, val, nr0, nr1, nj0, nj1, nnz, tid);
+        if constexpr (kNext == 1) d.template load<Load::kAll>(ptr, col, val, nr0, nr1, nj0, nj1, nnz, tid);
         if constexpr (kNext == 2) d.load(ptr, col, val, nr0, nr1, nj0, nj1, nnz, tid);
         T a0 = 0, a1 = 0;
 #pragma unroll
@@ -919,23 +951,26 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kWgWaves
           a0 = mul_add_rn(a0, v, x0[c]);
           if (NX == 2) a1 = mul_add_rn(a1, v, x1[c]);
         }
-        for (int off = tpr >> 1; off > 0; off >>= 1) {
-          a0 += __shfl_xor(a0, off, 64);
-          if (NX == 2) a1 += __shfl_xor(a1, off, 64);
-        }
-        if (act && lane == 0) {
-          if constexpr (kYT > 0) {
-            if (slot < kYT) sy[slot][(r0 & 3) + grp] = epi.value(a0);
-            else epi.row(row, a0, a1, acc, pv);
-          } else {
-            epi.row(row, a0, a1, acc, pv);
-          }
-        }
+        finish(a0, a1, pv);
       };
-      if (!more) sums(std::integral_constant<int, 0>{});
-      else if (nj1 - nj0 <= kTileNnz && d.full(nj0, nnz)) sums(std::integral_constant<int, 1>{});
-      else sums(std::integral_constant<int, 2>{});
-      nx = bounds(t + 2 * step);  // after the LDS reads, which share the scalar loads' counter
+      if constexpr (!kAhead) {
+        if (act) {
+          T a0 = 0, a1 = 0;
+#pragma unroll 2
+          for (int k = s + lane; k < e; k += tpr) {
+            const T v = sv[k];
+            const int c = column(k);
+            a0 = mul_add_rn(a0, v, x0[c]);
+            if (NX == 2) a1 = mul_add_rn(a1, v, x1[c]);
+          }
+          finish(a0, a1, epi.pre(row));
+        }
+      } else {
+        if (!more) sums(std::integral_constant<int, 0>{});
+        else if (nj1 - nj0 <= kTileNnz && d.full(nj0, nnz)) sums(std::integral_constant<int, 1>{});
+        else sums(std::integral_constant<int, 2>{});
+        nx = bounds(t + 2 * step);  // after the LDS reads, which share the scalar loads' counter
+      }
       __syncthreads();
     }
   }
