@@ -18,6 +18,9 @@
 // first, with the codes of the next ones behind: 192^3 in FP32 takes 18.0 us
 // with two, 18.5 with one and 19.7 with four, 96^3 in FP64 8.5, 7.8 and 8.5.
 // Class data from scalar registers, for wavefronts of one class, gave nothing.
+// Rows of at most two entries gather two (five, the next size, cost more than the
+// entries' own format where x lies in the L2: one entry, 300000 rows, FP64 5.6 us, with
+// two gathers 4.7; 2^22 rows 18.9 and 15.1).
 // Measured against row patterns (7-point, us): FP64 96^3 18 -> 8.6, 128^3
 // 28 -> 12.9, 160^3 57 -> 23; FP32 160^3 30 -> 11.3, 192^3 50 -> 18.2.
 //
@@ -126,7 +129,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
       }
     }
   };
-  if (most <= 5) sweep(std::integral_constant<int, 5>{});
+  if (most <= 2) sweep(std::integral_constant<int, 2>{});
+  else if (most <= 5) sweep(std::integral_constant<int, 5>{});
   else if (most <= 7) sweep(std::integral_constant<int, 7>{});
   else sweep(std::integral_constant<int, 8>{});
   if constexpr (NV > 0) block_store<NV>(acc, ra);
