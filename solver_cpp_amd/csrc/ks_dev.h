@@ -261,12 +261,16 @@ struct PatBuf : DBuf<int32_t> {
 };
 
 // Row classes (RowIx) of one side: the table at p, then its values in FP64 and
-// FP32, the state and the codes (null: the side has none).
+// FP32, the state, the codes (null: the side has none), and room for the row
+// patterns that stand in for at most kPatMax classes once new values end them.
 struct RowBuf : DBuf<int32_t> {
   static constexpr int64_t kV64 = kRowTab, kV32 = kV64 + 2 * kRowMax * kRowLen, kState = kV32 + kRowMax * kRowLen;
   static constexpr int64_t kHead = kState + (sizeof(PatState<kRowMax>) / 4 + 64) / 64 * 64;
   RowIx* code = nullptr;
+  int classes = 0;
   int entry_ib = 4;  // bytes per column index of the entry format it stands in for
+  static int64_t pat_at(int64_t n) { return (kHead + (n + 3) / 4 + 63) / 64 * 64; }
+  static int64_t words(int64_t n) { return pat_at(n) + kPatTab + (n + 1) / 2; }
   double* v64() const { return reinterpret_cast<double*>(p + kV64); }
   float* v32() const { return reinterpret_cast<float*>(p + kV32); }
   PatState<kRowMax>* state() const { return reinterpret_cast<PatState<kRowMax>*>(p + kState); }

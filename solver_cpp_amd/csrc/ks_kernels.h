@@ -2173,17 +2173,69 @@ __global__ void k_row_codes(int64_t n, PatState<kRowMax>* st, const int32_t* __r
     code[r].v = (uint8_t)p;
   }
 }
-// New values in the same pattern: do the rows of a class still agree?
-__global__ void k_row_check(int64_t n, PatState<kRowMax>* st, const int32_t* __restrict__ ptr,
-                            const double* __restrict__ val, const RowIx* __restrict__ code) {
+// New values in the same pattern: the table's values, by workgroup 0, and whether
+// the rows of a class still agree; *host (host-mapped) is set where they do not.
+__global__ __launch_bounds__(kBlock) void k_row_check(int64_t n, PatState<kRowMax>* st,
+                                                      const int32_t* __restrict__ ptr, const double* __restrict__ val,
+                                                      const RowIx* __restrict__ code, double* v64, float* v32,
+                                                      int* host) {
+  if (blockIdx.x == 0 && (int)threadIdx.x < st->P) {
+    const int p = threadIdx.x;
+    const int32_t a = ptr[st->row[p]], len = ptr[st->row[p] + 1] - a;
+    for (int j = 0; j < len; ++j) {
+      v64[p * kRowLen + j] = val[a + j];
+      v32[p * kRowLen + j] = (float)val[a + j];
+    }
+  }
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r < n; r += stride) {
     if (*(volatile int*)&st->bad) return;
     const int32_t a = ptr[r], e = ptr[r + 1], b = ptr[st->row[code[r].v]];
     bool ok = true;
     for (int32_t j = 0; j < e - a; ++j) ok &= same_bits(val[a + j], val[b + j]);
-    if (!ok) st->bad = 1;
+    if (!ok) {
+      // the first of the wavefront's, and of all, tells: a write to host memory from
+      // every row takes 0.8 ms at 2^22 rows
+      const int first = __ffsll((unsigned long long)__ballot(1)) - 1;
+      if ((int)(threadIdx.x & 63) == first && atomicExch(&st->bad, 1) == 0) *(volatile int*)host = 1;
+      return;
+    }
   }
+}
+// Row patterns from the table rtab of P <= kPatMax row classes, whose lists of
+// offsets are all the matrix has: the pattern table (k_pat_table's layout), and
+// each class's pattern at tab[kPatTab - kPatMax].  One wavefront.
+__global__ __launch_bounds__(64) void k_class_patterns(int P, const int32_t* __restrict__ rtab, int32_t* tab) {
+  static_assert(1 + kPatMax + kPatMax * kRowLen <= kPatTab - kPatMax, "the table and the classes' patterns fit");
+  const int p = threadIdx.x;
+  const int32_t* lens = rtab + kRowMax * kRowLen;
+  const int len = p < P ? lens[p] : 0;
+  int first = p;  // the first class of the same list
+  for (int q = 0; q < p && p < P && first == p; ++q) {
+    bool same = lens[q] == len;
+    for (int j = 0; same && j < len; ++j) same = rtab[q * kRowLen + j] == rtab[p * kRowLen + j];
+    if (same) first = q;
+  }
+  const uint64_t firsts = __ballot(p < P && first == p);
+  int stride = len > 1 ? len : 1;
+  for (int off = 32; off > 0; off >>= 1) stride = max(stride, __shfl_xor(stride, off, 64));
+  if (p == 0) tab[0] = stride;
+  if (p >= P) return;
+  const int id = __popcll(firsts & ((1ull << first) - 1));
+  tab[kPatTab - kPatMax + p] = id;
+  if (first != p) return;
+  tab[1 + id] = len;
+  for (int j = 0; j < len; ++j) tab[1 + kPatMax + id * stride + j] = rtab[p * kRowLen + j];
+}
+// one workgroup per tile
+__global__ __launch_bounds__(kBlock) void k_class_codes(const int32_t* __restrict__ tab, const int32_t* __restrict__ tiles,
+                                                        const int32_t* __restrict__ tnz,
+                                                        const int32_t* __restrict__ ptr,
+                                                        const RowIx* __restrict__ cls, PatIx* code) {
+  const int64_t t = blockIdx.x;
+  const int32_t r = tiles[t] + (int32_t)threadIdx.x;
+  if (r >= tiles[t + 1]) return;
+  code[r].v = (uint16_t)(tab[kPatTab - kPatMax + cls[r].v] << kPatShift | (ptr[r] - PatTile<double>::a0of(tnz[t])));
 }
 // The table's values and lengths; one workgroup of kRowMax threads.
 __global__ void k_row_vals(const PatState<kRowMax>* st, int32_t* tab, const int32_t* __restrict__ ptr,
