@@ -150,6 +150,7 @@ struct ks_ctx {
   ks::DBuf<double> part2;                // kMaxGrid partials of a norm whose finisher is deferred
   ks::DBuf<unsigned long long> stats;    // launches[8], bytes[8], on-chip solves' state (tag, fail)
   ks::DBuf<unsigned long long> coop;     // on-chip solves' reduction slots (kCoopSlots)
+  ks::DBuf<unsigned long long> found;    // what a new matrix's rows repeat: two PatFound, while it is created
   bool coop_off = false;                 // solve with one launch per operation
   // After a wait ran out, solves go by launches for coop_rest more of them,
   // coop_pause the next time (twice as many after each failure in a row): where

@@ -359,80 +359,65 @@ bool build_col_delta(const ks_mat* m, const Plan& pl, DBuf<uint16_t>& out, const
   return !hb;
 }
 
-// What the pattern kernels found, once they have run (PatState's last fields).
+// What a side's pattern kernels found, once they have run (pat_end).
 struct PatEnd {
   int P, bad, far, uncoded;
+  explicit PatEnd(const volatile int* h) : P(h[0]), bad(h[1]), far(h[2]), uncoded(h[3]) {}
   // bytes per index of the entry format that the side would have
   int index_bytes(const Plan& pl) const { return !far || (!uncoded && pl.wg.lane1) ? 2 : 4; }
 };
-template <int M>
-PatEnd pat_end(ks_ctx* c, const PatState<M>* st) {
-  static_assert(sizeof(PatEnd) == 4 * sizeof(int) && offsetof(PatState<M>, bad) == offsetof(PatState<M>, P) + sizeof(int) &&
-                    offsetof(PatState<M>, far) == offsetof(PatState<M>, P) + 2 * sizeof(int) &&
-                    offsetof(PatState<M>, uncoded) == offsetof(PatState<M>, P) + 3 * sizeof(int),
-                "PatState ends as PatEnd");
-  PatEnd e{};
-  KS_HIPCK(hipMemcpyAsync(&e, &st->P, sizeof(e), hipMemcpyDeviceToHost, c->stream));
-  KS_HIPCK(hipStreamSynchronize(c->stream));
-  return e;
-}
+// ints of the context's host-mapped flags: k_row_check's, k_pat_count's, pat_end's
+constexpr int kFlagCheck = 8, kFlagCount = 12, kFlagEnd = 16;
 
-// Row patterns (PatIx) of the CSR (ptr, col) with plan pl: when its SpMV runs
-// on workgroup tiles, none of them one long row, and its rows have at most
-// kPatMax patterns whose table fits kPatTab.  `pat` holds the table, the
-// codes and (while they are built) the state in one allocation.  Returns
-// false, with nothing kept, otherwise.
-bool build_patterns(ks_mat* m, const Plan& pl, PatBuf& pat, const int32_t* ptr, const int32_t* col) {
-  if (pl.kind != 0 || !(pl.wg64 || pl.wg32) || pl.wg.long_rows) return false;
-  ks_ctx* c = m->ctx;
-  hipStream_t s = c->stream;
+// Row patterns (PatIx) of the CSR (ptr, col) with plan pl from what k_pat_find
+// found: `pat` holds the table, the state and the codes in one allocation; *host
+// receives the end state (patterns whose table does not fit set `bad`).
+void enqueue_patterns(ks_mat* m, const Plan& pl, PatBuf& pat, const PatState<kPatMax>* found, const int32_t* ptr,
+                      const int32_t* col, int* host) {
+  hipStream_t s = m->ctx->stream;
   constexpr int64_t head = kPatTab + pad64(sizeof(PatState<kPatMax>) / 4 + 1);
   pat.alloc(head + (m->n + 1) / 2);
   auto* st = reinterpret_cast<PatState<kPatMax>*>(pat.p + kPatTab);
-  k_fill<int32_t><<<1, kBlock, 0, s>>>(head, pat.p, 0);
-  k_pat_find<kPatMax><<<grid_map(m->n), kBlock, 0, s>>>(m->n, ptr, col, nullptr, st);
-  k_pat_table<kPatMax><<<1, 2 * kPatMax, 0, s>>>(st, ptr, col, pat.p);
-  k_pat_codes<<<(unsigned)pl.wg.ntiles, kBlock, 0, s>>>(st, pat.p, pl.wg.tiles.p, pl.wg.tnz.p, ptr, col,
-                                                        reinterpret_cast<PatIx*>(pat.p + head));
-  KS_HIPCK(hipGetLastError());
-  const PatEnd end = pat_end(c, st);
-  if (end.bad) {
-    pat.release();
-    return false;
-  }
   pat.code = reinterpret_cast<PatIx*>(pat.p + head);
-  pat.entry_ib = end.index_bytes(pl);
-  return true;
+  k_fill<int32_t><<<1, kBlock, 0, s>>>(head, pat.p, 0);
+  k_pat_table<kPatMax><<<1, 2 * kPatMax, 0, s>>>(found, st, ptr, col, pat.p);
+  k_pat_codes<<<(unsigned)pl.wg.ntiles, kBlock, 0, s>>>(st, pat.p, pl.wg.tiles.p, pl.wg.tnz.p, ptr, col,
+                                                        const_cast<PatIx*>(pat.code));
+  k_pat_end<<<1, 1, 0, s>>>(st, host);
+  KS_HIPCK(hipGetLastError());
 }
 
-// Row classes (RowIx) of the CSR (ptr, col, val) with plan pl, under
-// build_patterns' conditions, for matrices of kRowMinNnz entries or more.  Not
-// for a borrowed matrix, whose values the caller may change in place.  Returns
-// the number of classes (0: none).
-int build_rows(ks_mat* m, const Plan& pl, RowBuf& rows, const int32_t* ptr, const int32_t* col, const double* val) {
-  if (pl.kind != 0 || !(pl.wg64 || pl.wg32) || pl.wg.long_rows || m->nnz < kRowMinNnz || m->n > kRowMaxN ||
-      (m->flags & KS_MAT_BORROW))
-    return 0;
-  ks_ctx* c = m->ctx;
-  hipStream_t s = c->stream;
+// Row classes (RowIx) of the CSR (ptr, col, val), the same way.
+void enqueue_rows(ks_mat* m, RowBuf& rows, const PatState<kRowMax>* found, const int32_t* ptr, const int32_t* col,
+                  const double* val, int* host) {
+  hipStream_t s = m->ctx->stream;
   rows.alloc(RowBuf::words(m->n));
   PatState<kRowMax>* st = rows.state();
-  RowIx* code = reinterpret_cast<RowIx*>(rows.p + RowBuf::kHead);
+  rows.code = reinterpret_cast<RowIx*>(rows.p + RowBuf::kHead);
   k_fill<int32_t><<<1, kBlock, 0, s>>>(RowBuf::kHead, rows.p, 0);
-  k_pat_find<kRowMax><<<grid_map(m->n), kBlock, 0, s>>>(m->n, ptr, col, val, st);
-  k_pat_table<kRowMax><<<1, 2 * kRowMax, 0, s>>>(st, ptr, col, rows.p);
-  k_row_codes<<<grid_map(m->n), kBlock, 0, s>>>(m->n, st, ptr, col, val, code);
-  k_row_vals<<<1, kRowMax, 0, s>>>(st, rows.p, ptr, val, rows.v64(), rows.v32());
+  k_pat_table<kRowMax><<<1, 2 * kRowMax, 0, s>>>(found, st, ptr, col, rows.p);
+  k_row_codes<<<grid_map(m->n), kBlock, 0, s>>>(m->n, st, ptr, col, val, rows.code);
+  k_row_vals<<<1, kRowMax, 0, s>>>(st, rows.p, ptr, val, rows.v64(), rows.v32(), host);
   KS_HIPCK(hipGetLastError());
-  const PatEnd end = pat_end(c, st);
-  if (end.bad) {
-    rows.release();
-    return 0;
+}
+
+// Distinct lists of offsets among some 500 sampled rows, or kRowMax + 1 once there
+// are more: so many rule row classes and patterns out before the GPU looks.
+int sampled_lists(int64_t n, const int32_t* hp, const int32_t* hc) {
+  std::vector<uint64_t> seen;
+  for (int64_t r = 0; r < n; r += n / 512 | 1) {
+    uint64_t h = 0x9e3779b97f4a7c15ull + (uint64_t)(hp[r + 1] - hp[r]);
+    for (int32_t j = hp[r]; j < hp[r + 1]; ++j) {
+      h ^= (uint32_t)(hc[j] - (int32_t)r);
+      h *= 0xff51afd7ed558ccdull;
+      h ^= h >> 32;
+    }
+    auto at = std::lower_bound(seen.begin(), seen.end(), h);
+    if (at != seen.end() && *at == h) continue;
+    if (seen.size() == kRowMax) return kRowMax + 1;
+    seen.insert(at, h);
   }
-  rows.code = code;
-  rows.classes = end.P;
-  rows.entry_ib = end.index_bytes(pl);
-  return end.P;
+  return (int)seen.size();
 }
 
 // New values: refreshes a side's classes; c->hflags[flag] (after the stream's
@@ -473,24 +458,90 @@ void drop_rows(ks_mat* m, RowBuf& rows, int flag, const Plan& pl, PatBuf& pat, c
 // row classes, where those apply (what new values fall back to is built with them
 // or, of few classes, when that happens); int32 columns otherwise, and
 // for a side whose SpMV runs on column panels (which read int32 columns).
+// Row classes need rows of at most kRowLen entries, kRowMinNnz entries in all and
+// values that only ks_mat_update_values changes; both they and patterns workgroup
+// tiles, none of them one long row.
 void build_index16(ks_mat* m, const int32_t* hp, const int32_t* hc) {
+  ks_ctx* c = m->ctx;
+  hipStream_t s = c->stream;
   const bool delta_first = (m->flags & KS_MAT_COL_DELTA) != 0;
-  int off16 = -1;  // not looked at yet
-  auto side = [&](RowBuf& rows, PatBuf& op, DBuf<int16_t>& o16, DBuf<uint16_t>& od, const Plan& pl,
-                  const PanelSet& ps, const int32_t* ptr, const int32_t* col, const double* val) {
-    if (ps.np || pl.kind != 0) return;
-    // up to kPatMax classes have no more patterns, whose table fits: those are
-    // built when new values end the classes (ks_mat_update_values)
-    const int classes = delta_first ? 0 : build_rows(m, pl, rows, ptr, col, val);
-    if (classes > 0 && classes <= kPatMax) return;
-    if (!delta_first && build_patterns(m, pl, op, ptr, col)) return;
-    if (off16 < 0) off16 = offsets_fit16(m->n, hp, hc);
-    if (off16 && !delta_first) build_col16(m, o16, ptr, col);
-    else if (!build_col_delta(m, pl, od, ptr, col) && off16) build_col16(m, o16, ptr, col);
+  struct Side {
+    RowBuf& rows;
+    PatBuf& pat;
+    DBuf<int16_t>& o16;
+    DBuf<uint16_t>& od;
+    const Plan& pl;
+    const PanelSet& ps;
+    const int32_t *ptr, *col;
+    const double* val;
+    int64_t max_row;
+    int kinds;
   };
-  side(m->rows, m->pat, m->col16, m->cold, m->plan, m->panels, m->ptr.p, m->col.p, m->val.p);
-  if (m->has_t)
-    side(m->trows, m->tpat, m->tcol16, m->tcold, m->tplan, m->tpanels, m->tptr.p, m->tcol.p, m->tval.p);
+  Side side[2] = {{m->rows, m->pat, m->col16, m->cold, m->plan, m->panels, m->ptr.p, m->col.p, m->val.p, m->max_row, 0},
+                  {m->trows, m->tpat, m->tcol16, m->tcold, m->tplan, m->tpanels, m->tptr.p, m->tcol.p, m->tval.p,
+                   m->max_trow, 0}};
+  const int sides = m->has_t ? 2 : 1;
+  int looked = -1, any = 0;
+  for (int i = 0; i < sides; ++i) {
+    Side& d = side[i];
+    const Plan& pl = d.pl;
+    if (delta_first || d.ps.np || pl.kind != 0 || !(pl.wg64 || pl.wg32) || pl.wg.long_rows) continue;
+    if (looked < 0) looked = sampled_lists(m->n, hp, hc);  // of A; A^T's are about as many
+    if (looked > kRowMax) continue;
+    if (d.max_row <= kRowLen && m->nnz >= kRowMinNnz && m->n <= kRowMaxN && !(m->flags & KS_MAT_BORROW))
+      d.kinds |= kFindRows;
+    if (d.max_row < kPatTab - kPatMax && (looked <= kPatMax || i > 0)) d.kinds |= kFindPats;
+    any |= d.kinds;
+  }
+  if (any) {
+    constexpr int64_t words = sizeof(PatFound) / 8;
+    PatFound* found = reinterpret_cast<PatFound*>(c->found.p);
+    k_fill<unsigned long long><<<grid_map(2 * words), kBlock, 0, s>>>(2 * words, c->found.p, 0ull);
+    auto look = [&](const Side& d) { return PatSide{d.ptr, d.col, d.val, d.kinds}; };
+    k_pat_find<<<dim3(grid_map(m->n), sides), kBlock, 0, s>>>(m->n, look(side[0]), look(side[1]), found);
+    k_pat_count<<<1, sides, 0, s>>>(found, c->hflags_dev + kFlagCount);
+    KS_HIPCK(hipGetLastError());
+    KS_HIPCK(hipStreamSynchronize(s));
+    volatile int* h = c->hflags;
+    for (int i = 0; i < sides; ++i) {
+      Side& d = side[i];
+      const int classes = h[kFlagCount + 2 * i], pats = h[kFlagCount + 2 * i + 1];
+      if (classes) enqueue_rows(m, d.rows, &found[i].row, d.ptr, d.col, d.val, c->hflags_dev + kFlagEnd + 8 * i);
+      // up to kPatMax classes have no more patterns, whose table fits: those are
+      // built when new values end the classes (drop_rows)
+      if (pats && (classes == 0 || classes > kPatMax))
+        enqueue_patterns(m, d.pl, d.pat, &found[i].pat, d.ptr, d.col, c->hflags_dev + kFlagEnd + 8 * i + 4);
+    }
+    KS_HIPCK(hipStreamSynchronize(s));
+    for (int i = 0; i < sides; ++i) {
+      Side& d = side[i];
+      if (d.rows.code) {
+        const PatEnd end(h + kFlagEnd + 8 * i);
+        d.rows.classes = end.P;
+        d.rows.entry_ib = end.index_bytes(d.pl);
+        if (end.bad) {
+          d.rows.code = nullptr;
+          d.rows.release();
+        }
+      }
+      if (d.pat.code) {
+        const PatEnd end(h + kFlagEnd + 8 * i + 4);
+        d.pat.entry_ib = end.index_bytes(d.pl);
+        if (end.bad) {
+          d.pat.code = nullptr;
+          d.pat.release();
+        }
+      }
+    }
+  }
+  int off16 = -1;  // not looked at yet
+  for (int i = 0; i < sides; ++i) {
+    Side& d = side[i];
+    if (d.ps.np || d.pl.kind != 0 || d.pat.code || (d.rows.code && d.rows.classes <= kPatMax)) continue;
+    if (off16 < 0) off16 = offsets_fit16(m->n, hp, hc);
+    if (off16 && !delta_first) build_col16(m, d.o16, d.ptr, d.col);
+    else if (!build_col_delta(m, d.pl, d.od, d.ptr, d.col) && off16) build_col16(m, d.o16, d.ptr, d.col);
+  }
 }
 
 // Split the CSR (hp, hc: host row pointers and columns of A or A^T) into
@@ -1083,6 +1134,7 @@ ks_status ks_ctx_create(int32_t device, ks_ctx** out) {
     KS_HIPCK(hipMemsetAsync(c->part2.p, 0, sizeof(double) * kMaxGrid, c->stream));
     c->stats.alloc(2 * KS_K_NCLASS + 1);
     c->coop.alloc(kCoopSlots);
+    c->found.alloc(2 * sizeof(PatFound) / 8);
     coop_reset(c);
     KS_HIPCK(hipHostMalloc((void**)&c->hflags, 64 * sizeof(int), hipHostMallocMapped));
     std::memset(c->hflags, 0, 64 * sizeof(int));
@@ -1120,6 +1172,7 @@ void ks_ctx_destroy(ks_ctx* c) {
   c->part.release();
   c->stats.release();
   c->coop.release();
+  c->found.release();
   if (c->hflags) (void)hipHostFree(c->hflags);
   if (c->stream && c->own_stream) (void)hipStreamDestroy(c->stream);
   delete c;
@@ -1245,8 +1298,8 @@ ks_status ks_mat_update_values(ks_mat* m, const double* val, uint32_t flags) {
   }
   refresh_panels(m, m->panels);
   refresh_panels(m, m->tpanels);
-  refresh_rows(m, m->rows, m->ptr.p, m->val.p, 8);
-  refresh_rows(m, m->trows, m->tptr.p, m->tval.p, 9);
+  refresh_rows(m, m->rows, m->ptr.p, m->val.p, kFlagCheck);
+  refresh_rows(m, m->trows, m->tptr.p, m->tval.p, kFlagCheck + 1);
   if (m->val32.p) {
     k_convert<double, float><<<grid_map(m->nnz), kBlock, 0, c->stream>>>(m->nnz, m->val.p, m->val32.p, Gate{});
     KS_HIPCK(hipGetLastError());
@@ -1256,8 +1309,8 @@ ks_status ks_mat_update_values(ks_mat* m, const double* val, uint32_t flags) {
     KS_HIPCK(hipGetLastError());
   }
   KS_HIPCK(hipStreamSynchronize(c->stream));
-  drop_rows(m, m->rows, 8, m->plan, m->pat, m->ptr.p);
-  drop_rows(m, m->trows, 9, m->tplan, m->tpat, m->tptr.p);
+  drop_rows(m, m->rows, kFlagCheck, m->plan, m->pat, m->ptr.p);
+  drop_rows(m, m->trows, kFlagCheck + 1, m->tplan, m->tpat, m->tptr.p);
   return KS_OK;
   KS_API_CATCH(c)
 }

@@ -2031,13 +2031,13 @@ __global__ void k_col_delta(int64_t n, const int32_t* __restrict__ ptr, const in
 }
 
 // Row patterns (PatIx, M = kPatMax) and row classes (RowIx, M = kRowMax: the
-// rows' values, compared bit for bit, belong to the pattern), built by three
-// kernels with no host step between them.  k_pat_find enters every row's hash
-// in an open-addressing table of 2 M slots (key 0: free; rep: a row with that
-// key).  k_pat_table numbers the patterns by hash and writes the pattern table
-// from their rows.  k_pat_codes / k_row_codes write the row codes and compare
-// every row with its pattern entry by entry (two patterns of one hash).  Each
-// sets `bad` when the format does not apply, which ends the later ones.
+// rows' values, compared bit for bit, belong to the pattern).  One pass,
+// k_pat_find, enters every row's hashes in open-addressing tables of 2 M slots (key
+// 0: free; rep: a row with that key), in memory of the context; where k_pat_count
+// tells the host that they are few, memory is allocated and k_pat_table numbers the
+// patterns by hash and writes the pattern table from their rows, and k_pat_codes /
+// k_row_codes write the row codes and compare every row with its pattern entry by
+// entry (two patterns of one hash).  `bad` is set when the format does not apply.
 template <int M>
 struct PatState {
   unsigned long long key[2 * M];
@@ -2063,45 +2063,87 @@ __device__ inline uint64_t pat_hash(const int32_t* __restrict__ col, const doubl
   }
   return h ? h : 1;
 }
+// what k_pat_find finds of one side
+struct PatFound {
+  PatState<kRowMax> row;
+  PatState<kPatMax> pat;
+};
+enum { kFindRows = 1, kFindPats = 2 };
+// Enters hash h of row r; false once the rows have too many of them.  last: a key
+// that is in the table (most rows repeat the one before).
 template <int M>
-__global__ void k_pat_find(int64_t n, const int32_t* __restrict__ ptr, const int32_t* __restrict__ col,
-                           const double* __restrict__ val, PatState<M>* st) {
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  unsigned long long last = 0;  // a key that is in the table: most rows repeat it
-  for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r < n; r += stride) {
-    const int32_t a = ptr[r], e = ptr[r + 1];
-    if (e - a > (M == kRowMax ? kRowLen : kPatTab - 1 - M)) { st->bad = 1; return; }
-    const unsigned long long h = pat_hash<M>(col, val, a, e, (int32_t)r);
-    if (h == last) continue;
-    if (*(volatile int*)&st->bad) return;
-    int s = (int)(h % (2 * M)), tries = 0;
-    for (; tries < 2 * M; ++tries, s = (s + 1) % (2 * M)) {
-      unsigned long long k = *(volatile unsigned long long*)(st->key + s);
-      if (k == 0) k = atomicCAS(st->key + s, 0ull, h);  // the key that was there
-      if (k == 0) st->rep[s] = (int32_t)r;              // this row entered it
-      if (k == 0 || k == h) break;
+__device__ inline bool pat_enter(PatState<M>* st, unsigned long long h, int32_t r, unsigned long long& last) {
+  if (h == last) return true;
+  if (*(volatile int*)&st->bad) return false;
+  int s = (int)(h % (2 * M)), tries = 0;
+  for (; tries < 2 * M; ++tries, s = (s + 1) % (2 * M)) {
+    unsigned long long k = *(volatile unsigned long long*)(st->key + s);
+    if (k == 0) k = atomicCAS(st->key + s, 0ull, h);  // the key that was there
+    if (k == 0) {                                     // this row entered it
+      st->rep[s] = r;
+      if (atomicAdd(&st->P, 1) >= M) st->bad = 1;
     }
-    if (tries == 2 * M) { st->bad = 1; return; }
-    last = h;
+    if (k == 0 || k == h) break;
+    if (tries % 8 == 7 && *(volatile int*)&st->bad) return false;
   }
+  if (tries == 2 * M) {
+    st->bad = 1;
+    return false;
+  }
+  last = h;
+  return true;
+}
+// One side of a matrix; kinds: kFindRows, kFindPats or both.
+struct PatSide {
+  const int32_t *ptr, *col;
+  const double* val;
+  int kinds;
+};
+// grid: rows, sides
+__global__ void k_pat_find(int64_t n, PatSide one, PatSide two, PatFound* found) {
+  const PatSide d = blockIdx.y ? two : one;
+  PatFound* f = found + blockIdx.y;
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  unsigned long long last_row = 0, last_pat = 0;
+  bool rows = d.kinds & kFindRows, pats = d.kinds & kFindPats;
+  for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r < n && (rows || pats); r += stride) {
+    const int32_t a = d.ptr[r], e = d.ptr[r + 1];
+    if (rows) rows = pat_enter(&f->row, pat_hash<kRowMax>(d.col, d.val, a, e, (int32_t)r), (int32_t)r, last_row);
+    if (pats) pats = pat_enter(&f->pat, pat_hash<kPatMax>(d.col, nullptr, a, e, (int32_t)r), (int32_t)r, last_pat);
+  }
+}
+// PatState's last fields to host-mapped memory
+template <int M>
+__device__ inline void pat_end(const PatState<M>* st, int* host) {
+  host[0] = st->P;
+  host[1] = st->bad;
+  host[2] = st->far;
+  host[3] = st->uncoded;
+}
+__global__ void k_pat_end(const PatState<kPatMax>* st, int* host) { pat_end(st, host); }
+// host[2 s], host[2 s + 1]: how many classes and patterns side s has (0: too many
+// of them), to host-mapped memory
+__global__ void k_pat_count(const PatFound* f, int* host) {
+  const int s = threadIdx.x;
+  host[2 * s] = f[s].row.bad ? 0 : f[s].row.P;
+  host[2 * s + 1] = f[s].pat.bad ? 0 : f[s].pat.P;
 }
 // one workgroup of 2 M threads
 template <int M>
-__global__ void k_pat_table(PatState<M>* st, const int32_t* __restrict__ ptr, const int32_t* __restrict__ col,
-                            int32_t* tab) {
+__global__ void k_pat_table(const PatState<M>* found, PatState<M>* st, const int32_t* __restrict__ ptr,
+                            const int32_t* __restrict__ col, int32_t* tab) {
   __shared__ int s_stride, s_P;
-  if (st->bad) return;
   const int s = threadIdx.x;
   if (s == 0) { s_stride = 1; s_P = 0; }
   __syncthreads();
-  const unsigned long long k = st->key[s];
+  const unsigned long long k = found->key[s];
   int32_t r = 0, a = 0, len = 0;
   int p = 0;
   if (k) {
-    r = st->rep[s];
+    r = found->rep[s];
     a = ptr[r];
     len = ptr[r + 1] - a;
-    for (int q = 0; q < 2 * M; ++q) p += st->key[q] && st->key[q] < k;
+    for (int q = 0; q < 2 * M; ++q) p += found->key[q] && found->key[q] < k;
     atomicMax(&s_stride, len);
     atomicAdd(&s_P, 1);
   }
@@ -2237,11 +2279,12 @@ __global__ __launch_bounds__(kBlock) void k_class_codes(const int32_t* __restric
   if (r >= tiles[t + 1]) return;
   code[r].v = (uint16_t)(tab[kPatTab - kPatMax + cls[r].v] << kPatShift | (ptr[r] - PatTile<double>::a0of(tnz[t])));
 }
-// The table's values and lengths; one workgroup of kRowMax threads.
+// The table's values and lengths, and the end state; one workgroup of kRowMax threads.
 __global__ void k_row_vals(const PatState<kRowMax>* st, int32_t* tab, const int32_t* __restrict__ ptr,
-                           const double* __restrict__ val, double* v64, float* v32) {
+                           const double* __restrict__ val, double* v64, float* v32, int* host) {
   __shared__ int most;
   const int p = threadIdx.x;
+  if (p == 0) pat_end(st, host);
   if (st->bad) return;
   if (p == 0) most = 0;
   __syncthreads();
