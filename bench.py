@@ -162,7 +162,7 @@ def main():
     bytes_per = by_tot / max(launches, 1)
     ms_per = ms_tot / max(launches, 1)
     bytes_per32 = bytes_per - A.spmv_bytes(False, 32) + 8 * nnz + 12 * n + 4  # the same launches, int32 CSR
-    achieved = bytes_per32 / (ms_per * 1e-3) / 1e9 if launches else None
+    csr_rate = bytes_per32 / (ms_per * 1e-3) / 1e9 if launches else None
     moved = bytes_per / (ms_per * 1e-3) / 1e9 if launches else None
 
     out = {
@@ -182,8 +182,8 @@ def main():
                        "byte_model": "the format the kernel reads (its SpMV bytes + 4*n*nv)",
                        "int32_csr": {"what": "the same launches by the metric's byte model, 8*nnz + 12*n + 4 + 4*n*nv",
                                      "bytes_per_launch": bytes_per32,
-                                     "GBps": round(achieved, 1) if achieved else None,
-                                     "ratio_to_peak": round(achieved / HBM_PEAK_GBS, 4) if achieved else None},
+                                     "GBps": round(csr_rate, 1) if csr_rate else None,
+                                     "ratio_to_peak": round(csr_rate / HBM_PEAK_GBS, 4) if csr_rate else None},
                        "profiled_solves": a.prof_steps,
                        "profiled_s_per_solve": round(sum(rr["seconds"] for rr in prof) / max(len(prof), 1), 6)}
     out["solve_bytes_GBps"] = round(r0["bytes"] / r0["seconds"] / 1e9, 1)
@@ -210,7 +210,7 @@ def main():
     out["spmv"] = {"poisson3d_160": spmv_line(A, n, nnz, trans=False)}
     A.close()
     if not a.headline_only:
-        out["hbm_ceiling"] = hbm_ceiling(ctx, achieved, moved)
+        out["hbm_ceiling"] = hbm_ceiling(ctx, moved)
         out["spmv"].update(spmv_configs(ctx))
         out["adjoint"] = adjoint_times(ctx)
     if not a.no_cpu:
@@ -379,17 +379,16 @@ def calib_copy(a):
     return 2 * src.numel() * 8
 
 
-def hbm_ceiling(ctx, achieved, moved):
+def hbm_ceiling(ctx, achieved):
     """What plain streaming kernels reach on this box (1 GiB, best of four
     grids): the practical ceiling beside the published 8 TB/s, and the
-    roofline kernel's rates as fractions of the read ceiling."""
+    roofline kernel's rate (`roofline.achieved`) as a fraction of the read ceiling."""
     rd = ctx.stream_rate("read")
     out = {"what": "plain non-temporal 16-byte streaming kernels over 1 GiB (ks_bench_stream), best of 4 grids",
            "read_GBps": round(rd, 1), "copy_GBps": round(ctx.stream_rate("copy"), 1),
            "read_frac_of_peak": round(rd / HBM_PEAK_GBS, 4)}
-    if achieved and moved:
+    if achieved:
         out["roofline_achieved_frac_of_read"] = round(achieved / rd, 4)
-        out["roofline_format_frac_of_read"] = round(moved / rd, 4)
     return out
 
 
@@ -406,7 +405,7 @@ def spmv_gbps(A, n, nnz, prec, trans=False, reps=30):
     by32 = (sv + 4) * nnz + 4 * (n + 1) + 2 * sv * n
     by = A.spmv_bytes(trans, prec)
     return {"us": round(ms * 1e3, 2), "GBps": round(by32 / (ms * 1e-3) / 1e9, 1),
-            "frac_of_8TBps": round(by32 / (ms * 1e-3) / 8e12, 4), "index_bytes": A.index_bytes(trans, prec),
+            "frac_of_8TBps": round(by32 / (ms * 1e-3) / 8e12, 4), "format_bytes": by,
             "format_GBps": round(by / (ms * 1e-3) / 1e9, 1), "format_frac": round(by / (ms * 1e-3) / 8e12, 4)}
 
 
