@@ -154,7 +154,9 @@ typedef struct ks_result {
   double relres_true;        /* ||b-Ax||/||b|| recomputed in FP64 */
   double log10_check;        /* log10(||b-Ax||/||b-Ax0||): Check_error (blas.cpp:266-301) */
   double seconds;            /* device-synchronised wall time of the solve */
-  double bytes;              /* algorithmic HBM bytes of all launched kernels */
+  double bytes;              /* algorithmic HBM bytes of all launched kernels (an on-chip solve:
+                                matrix and vectors once per launch, and what each step stores;
+                                not what its workgroups read from each other through the caches) */
   double prof_ms[KS_K_NCLASS];      /* hipEvent time per kernel class (profile=1) */
   int64_t prof_launches[KS_K_NCLASS];
   double prof_bytes[KS_K_NCLASS];   /* algorithmic bytes per kernel class */

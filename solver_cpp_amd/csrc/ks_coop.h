@@ -384,7 +384,7 @@ __global__ __launch_bounds__(NT) void k_cg_coop(int64_t n, const int32_t* __rest
       c->stop = 0;
       c->status = 2;
       if (stop >= 0) ctl_stop(c, stop);
-      st.count_many(done);
+      st.count_many(done, (unsigned long long)done * 2 * sizeof(T) * n);  // p and r of each step
     }
   }
   team.close();
@@ -535,7 +535,7 @@ __global__ __launch_bounds__(NT) void k_bicg_coop(int64_t n, const int32_t* __re
       c->stop = 0;
       c->status = 2;
       if (stop >= 0) ctl_stop(c, stop);
-      st.count_many(2 * done);
+      st.count_many(2 * done, (unsigned long long)done * 4 * sizeof(T) * n);
     }
   }
   team.close();

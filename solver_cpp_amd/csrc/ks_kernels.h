@@ -101,11 +101,11 @@ struct StatArgs {
       atomicAdd(bytes + cls, nbytes);
     }
   }
-  // by one thread, for a launch that did the work of m
-  __device__ void count_many(int m) const {
+  // by one thread, for an on-chip launch of m products: nbytes, and `more` in its steps
+  __device__ void count_many(int m, unsigned long long more) const {
     if (!launches) return;
     atomicAdd(launches + cls, (unsigned long long)m);
-    atomicAdd(bytes + cls, nbytes * (unsigned long long)m);
+    atomicAdd(bytes + cls, nbytes + more);
   }
 };
 

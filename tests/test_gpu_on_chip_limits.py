@@ -81,3 +81,22 @@ def test_cg_with_four_rows_per_thread_gathers_runs(ctx, name, make, yes, outer, 
     b = np.random.default_rng(73).uniform(-1, 1, len(ptr) - 1)
     assert _runs_on_chip(ctx, A, b, outer, inner, **kw) == yes
     A.close()
+
+
+@pytest.mark.parametrize("outer,maxloop", [("cg", 300), ("cg", 2000), ("bicg", 300)])
+def test_counted_bytes(ctx, outer, maxloop):
+    # the matrix and the vectors once a launch of at most 1024 steps, and each
+    # step's stores; by launches, the products and vector passes of every step
+    from solver_cpp_amd import api
+    n = 20_000
+    ptr, col, val = _tridiag(n)
+    nnz = len(col)
+    A = api.Matrix(ctx, ptr, col, val, transpose=True)
+    b = np.random.default_rng(74).uniform(-1, 1, n)
+    x, r, _ = api.solve(ctx, A, b, outer, history=False, outer_eps=0.0, outer_maxloop=maxloop)
+    launches = -(-r["steps"] // 1024)
+    csr, sides = 12 * nnz + 4 * (n + 1), 1 if outer == "cg" else 2
+    per_launch = sides * csr + (4 if outer == "cg" else 6) * 8 * n
+    assert list(r["prof"]) == ["spmv64"] and r["spmv"] == sides * r["steps"]
+    assert r["bytes"] == launches * per_launch + r["steps"] * 2 * sides * 8 * n
+    A.close()
