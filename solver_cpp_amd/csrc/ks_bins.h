@@ -59,7 +59,7 @@ __global__ __launch_bounds__(kBlock) void k_bin_count(int nblk, int64_t nseg, co
   const int64_t s = blockIdx.x;
   for (int b = threadIdx.x; b < nblk; b += kBlock) h[b] = 0;
   __syncthreads();
-  for (int32_t j = snz[s] + (int32_t)threadIdx.x; j < snz[s + 1]; j += kBlock) atomicAdd(h + col[j] / kBinCols, 1);
+  for (int64_t j = snz[s] + (int64_t)threadIdx.x; j < snz[s + 1]; j += kBlock) atomicAdd(h + col[j] / kBinCols, 1);
   __syncthreads();
   for (int b = threadIdx.x; b < nblk; b += kBlock) cnt[b * nseg + s] = h[b];
 }
@@ -106,7 +106,7 @@ __global__ __launch_bounds__(kBlock) void k_bin_fill(int nblk, int64_t nseg, con
     mask[s * kBinWords + k] = start[k];
     before[s * kBinWords + k] = (uint16_t)c;
   }
-  for (int32_t j = j0 + (int32_t)threadIdx.x; j < j1; j += kBlock) {
+  for (int64_t j = j0 + (int64_t)threadIdx.x; j < j1; j += kBlock) {
     const int32_t c = col[j], b = c / kBinCols;
     const int p = atomicAdd(at + b, 1);
     lcol[out[b] + p] = (uint16_t)(c - b * kBinCols);

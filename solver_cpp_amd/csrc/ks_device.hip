@@ -200,11 +200,11 @@ bool scattered_rows(int64_t n, const int32_t* hp, const int32_t* hc) {
 // or with several lanes a row (over 8 entries on average) the row's next one.
 bool gathers_runs(int64_t n, const int32_t* hp, const int32_t* hc) {
   const bool lanes = hp[n] > 8 * n;
-  auto near = [&](int32_t a, int32_t b) { return std::abs((int64_t)hc[a] - hc[b]) <= 8; };
+  auto near = [&](int64_t a, int64_t b) { return std::abs((int64_t)hc[a] - hc[b]) <= 8; };
   int64_t runs = 0, all = 0;
   for (int64_t r = 0; r + 1 < n; r += n / 1024 | 1)
-    for (int32_t j = hp[r], e = std::min(hp[r + 1], hp[r] + 64); j < e; ++j) {
-      const int32_t below = hp[r + 1] + (j - hp[r]);
+    for (int64_t j = hp[r], e = j + std::min(hp[r + 1] - hp[r], 64); j < e; ++j) {
+      const int64_t below = hp[r + 1] + (j - hp[r]);
       ++all;
       runs += (below < hp[r + 2] && near(j, below)) || (lanes && j + 1 < hp[r + 1] && near(j, j + 1));
     }
@@ -247,8 +247,8 @@ void build_bins(ks_mat* m, BinSet& bs, const int32_t* hp, const int32_t* ptr, co
   KS_HIPCK(hipMemcpyAsync(start.data(), dstart.p, sizeof(int32_t) * nblk, hipMemcpyDeviceToHost, s));
   KS_HIPCK(hipStreamSynchronize(s));
   for (int b = 0; b < nblk; ++b) {
-    const int64_t k = std::max<int64_t>(1, (start[b + 1] - start[b] + kBinUnit - 1) / kBinUnit);
     const int64_t a = start[b], len = start[b + 1] - a;
+    const int64_t k = std::max<int64_t>(1, (len + kBinUnit - 1) / kBinUnit);
     for (int64_t i = 0; i < k; ++i)
       if (len > 0) {
         unit.push_back(b);
