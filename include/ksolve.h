@@ -80,11 +80,18 @@ typedef enum ks_status {
                                  gathers x from slices of 16384 columns in LDS
                                  in a pass of its own) */
 #define KS_MAT_COL32    2048u /* keep int32 column indices in the SpMV.  Without
-                                 it, a matrix whose rows repeat at most 32
-                                 lists of column offsets col - row (stencils)
-                                 is read with a 16-bit pattern code per row
-                                 instead of indices and row pointers, and
-                                 otherwise one whose entries all lie within
+                                 it, a matrix whose rows repeat with their
+                                 values (at most 128 different rows of at most
+                                 8 entries, at least 4096 entries in all, not
+                                 KS_MAT_BORROW: stencils with coefficients
+                                 constant or constant in parts) is read as a
+                                 byte per row and a table (row classes),
+                                 until new values no longer repeat; one whose
+                                 rows repeat at most 32 lists of column offsets
+                                 col - row (stencils) is read with a 16-bit
+                                 pattern code per row instead of indices and
+                                 row pointers (row patterns); and otherwise
+                                 one whose entries all lie within
                                  32767 columns of their row (stencils, banded
                                  matrices) also gets int16 offsets col - row,
                                  which the workgroup-tile SpMV reads instead
@@ -219,12 +226,13 @@ ks_status ks_mat_info(const ks_mat* m, int64_t* n, int64_t* nnz,
 /* Bytes per column index in the entry format of A (trans = 0) or A^T
  * (trans = 1), in a precision (KS_F64 / KS_F32): 2 with int16 offsets or
  * delta-coded columns (see KS_MAT_COL32), else 4.  A side kept as row
- * patterns reports the entry format it would have without them.  No
+ * patterns or classes reports the entry format it would have without them.  No
  * reference counterpart (the reference always reads int32 columns,
  * cudaFunction.cu:127-156). */
 ks_status ks_mat_index_bytes(const ks_mat* m, int32_t trans, int32_t precision, int32_t* bytes);
 /* HBM bytes of one SpMV in the format its kernel reads: values, column
- * indices and row pointers (or row-pattern codes), x and y once.  No
+ * indices and row pointers (or the codes of row patterns or classes), x and y
+ * once.  No
  * reference counterpart; the bench uses it for the SpMV's byte count. */
 ks_status ks_mat_spmv_bytes(const ks_mat* m, int32_t trans, int32_t precision, double* bytes);
 

@@ -4,8 +4,10 @@
 // three dependent launches it takes 14 us: each launch costs 4 to 5 us
 // whatever it does.  Here one launch runs up to kCoopIters steps.  The
 // workgroups (one per CU at most, so all are resident together) own
-// contiguous rows, one or two per thread, whose matrix entries and vector
-// elements stay in registers between the steps.  Two things cross workgroups:
+// contiguous rows, up to four per thread (BiCG two), whose matrix entries and
+// vector elements stay in the thread's registers between the steps, and of the
+// most rows some in its scratch (FP64 CG with four 380 bytes, FP32 80; BiCG with
+// two 390 and 200).  Two things cross workgroups:
 //  * vectors that other rows' products gather: written with agent-scope
 //    stores, which go through to memory, and gathered with agent-scope loads
 //    (a workgroup's own part from LDS);
@@ -29,14 +31,14 @@
 
 namespace ks {
 
-// Threads of a workgroup and the most rows per thread: 512 threads were the
-// fastest at most sizes (CG, 256 x 256 / 512 x 512 / 700 x 700: 6.4 / 8.6 /
-// 13.2 us a step; 256 threads 6.7 / 9.8 / 41, 1024 threads 6.6 / 8.3 / 15.0),
-// and leave the 256 registers that four rows take.
+// Threads of a workgroup and the most rows per thread: of one build, 512 threads
+// were the fastest at most sizes (CG, 256 x 256 / 512 x 512 / 700 x 700: 6.4 / 8.6 /
+// 13.2 us a step; 256 threads 6.7 / 9.8 / 41, 1024 threads 6.6 / 8.3 / 15.0): they
+// leave 256 registers a thread.
 constexpr int kCoopThreads = 512;
 constexpr int kCoopRpt = 4;
 constexpr int kCoopMaxWg = 256;
-constexpr int kCoopRow = 8;       // entries of a row held in registers
+constexpr int kCoopRow = 8;       // entries of a row at most
 constexpr int kCoopVals = 64;     // values of one reduction
 constexpr int kCoopIters = 1024;  // steps per launch
 constexpr int kCoopSpin = 1 << 21;
@@ -394,8 +396,8 @@ __global__ __launch_bounds__(NT) void k_cg_coop(int64_t n, const int32_t* __rest
 // A^T p*), the reduction of
 // (p*, A p), the updates, and the reduction of (r*, r) and (r, r).  vec holds
 // r, r*, then p and p* of even and of odd steps.  Both matrices' entries are
-// kept, so a thread takes at most two rows (at two, 380 bytes of them in scratch
-// in FP64 and 190 in FP32; BicgLevel::kRpt).
+// kept, so a thread takes at most two rows (at two, 390 bytes of them in scratch
+// in FP64 and 200 in FP32; BicgLevel::kRpt).
 // Measured (7-point grids, us a step, on chip against five launches): FP64 16^3
 // 6.1 / 23.2, 32^3 8.0 / 23.6, 50^3 11.5 / 27.2, 64^3 20.7 / 28.4; FP32 inside
 // VPGMRES 16^3 7.8 / 24.9, 50^3 13.4 / 25.5, 64^3 18.1 / 25.5.

@@ -464,7 +464,7 @@ void klaunch_n(ks_ctx* c, int cls, void (*kernel)(P...), int G, A&&... args) {
 // Whether a solve with A runs on chip (ks_coop.h): rows of at most kCoopRow
 // entries, at most `rpt` per thread of one workgroup per CU.  Four rows per
 // thread of CG is about where a step stops being the faster one on chip (some of
-// their entries lie in scratch: 370 bytes in FP64, 80 in FP32).  CG, us a step, on
+// their entries lie in scratch: 380 bytes in FP64, 80 in FP32).  CG, us a step, on
 // chip against three launches: 5-point 256 x 256 6.0 / 14.5, 512 x 512 8.3 /
 // 16.6, 724 x 724 14.2 / 21.4; 7-point 32^3 6.2 / 15.4, 63^3 9.3 / 21.3, 80^3
 // 22.9 / 22.8, and in FP32 inside VPGMRES 13.3 / 20.6.  Rows that gather more

@@ -141,11 +141,11 @@ constexpr int kPanels = 10;
 // the GPU.  Measured, FP64 / FP32 / SDDMM in us, column blocks against the
 // layout before them (merge path, column panels from 2^21 rows): rows of up
 // to 4096 entries, n = 250000 115 / 80 / 139 against 103 / 93 / 166, 400000
-// 155 / 104 / 183 against 163 / 147 / 320, 10^6 405 / 208 / 421 against 530 /
-// 368 / 789, 4 10^6 1596 / 965 / 1645 against 1884 / 1604 / 3511; rows of up
+// 155 / 105 / 176 against 163 / 143 / 276, 10^6 408 / 213 / 433 against 528 /
+// 368 / 789, 4 10^6 1593 / 973 / 1657 against 1887 / 1612 / 3500; rows of up
 // to 300 entries, n = 500000 (6.6M entries) 97 / 61 / 109 against 67 / 58 /
-// 127, 10^6 (13M) 129 / 85 / 148 against 155 / 112 / 236, 4 10^6 488 / 254 /
-// 478 against 1275 / 748 / 998.  Sides of even row lengths (a random
+// 127, 10^6 (13M) 130 / 86 / 145 against 156 / 112 / 231, 4 10^6 491 / 253 /
+// 482 against 912 / 586 / 1005.  Sides of even row lengths (a random
 // matrix's A^T) keep tiles and panels, which are as fast in FP64 (4 10^6:
 // 1527 against 1418) and fuse the GMRES projection.
 constexpr int64_t kBinMinRows = 3 << 17, kBinMinEntries = 10 << 20;
@@ -450,17 +450,19 @@ void drop_rows(ks_mat* m, RowBuf& rows, int flag, const Plan& pl, PatBuf& pat, c
   rows.code = nullptr;
 }
 
-// The SpMV's 16-bit column indices of A and A^T, unless KS_MAT_COL32: row
-// patterns where they apply (not with KS_MAT_COL_DELTA), else int16 offsets
-// when every offset fits (hp, hc: A's host row pointers and columns; A^T's
-// offsets are A's negated, so both fit), delta-coded columns where those
-// apply, in the order KS_MAT_COL_DELTA asks for, and with the first two the
-// row classes, where those apply (what new values fall back to is built with them
-// or, of few classes, when that happens); int32 columns otherwise, and
-// for a side whose SpMV runs on column panels (which read int32 columns).
-// Row classes need rows of at most kRowLen entries, kRowMinNnz entries in all and
-// values that only ks_mat_update_values changes; both they and patterns workgroup
-// tiles, none of them one long row.
+// What the SpMV of A and of A^T reads instead of int32 columns, unless
+// KS_MAT_COL32 (hp, hc: A's host row pointers and columns):
+//  * row classes, where rows repeat with their values: rows of at most kRowLen
+//    entries, kRowMinNnz entries in all, values that only ks_mat_update_values
+//    changes;
+//  * else row patterns, where rows repeat their offsets;
+//  * else int16 offsets, when every offset fits (A^T's are A's negated), or
+//    delta-coded columns, when every row encodes.
+// Classes and patterns need workgroup tiles, none of them one long row, and no
+// KS_MAT_COL_DELTA, which also prefers delta codes to int16 offsets.  More than
+// kPatMax classes have the next format that applies beside them, for when new
+// values end them; fewer become patterns then (drop_rows).  A side on column
+// panels keeps int32 columns.
 void build_index16(ks_mat* m, const int32_t* hp, const int32_t* hc) {
   ks_ctx* c = m->ctx;
   hipStream_t s = c->stream;
@@ -926,7 +928,8 @@ double resid_norm(ks_ctx* c, ks_mat* m, bool trans, const double* b, const doubl
   else
     r.alloc(m->n);
   auto A = m->view<double>(trans && m->has_t);
-  launch_spmv<double, 1>(c, A, x, EpiResid<double, FinStore>{b, r.p, FinStore{c->hscal_dev + 1, 1}}, Gate{}, 8.0 * m->n);
+  launch_spmv<double, 1>(c, A, x, EpiResid<double, FinStore>{b, r.p, FinStore{c->hscal_dev + 1, 1}}, Gate{},
+                         8.0 * m->n);
   KS_HIPCK(hipStreamSynchronize(c->stream));
   return c->hscal[1];
 }
@@ -962,8 +965,8 @@ std::mutex& coop_mutex(int device) {
 }
 
 // Run a constructed solve level and fill the result.  Returns false when an
-// on-chip launch gave up waiting (x and res are then undefined).  prof_mask selects the
-// kernel classes timed with events; rbuf (optional, n doubles of device
+// on-chip launch gave up waiting (x and res are then undefined).  prof_mask
+// selects the kernel classes timed with events; rbuf (optional, n doubles of device
 // memory the solve no longer needs at the end) holds the residuals of the
 // true-residual checks.
 bool run_level(ks_ctx* c, ks_mat* m, Level& Lv, const ks_params* p, unsigned prof_mask, bool trans,

@@ -668,12 +668,12 @@ struct CgLevel : Level {
       const int64_t ld = pad64(n);
       const int iters = (int)std::min<int64_t>(kCoopIters, cfg.maxloop - u * kCoopIters);
       // a launch reads the CSR, x, r and p and writes x
-      const StatArgs st = stat(c, sizeof(T) == 8 ? KS_K_SPMV64 : KS_K_SPMV32, spmv_bytes<T>(n, A.nnz) + 2.0 * sizeof(T) * n);
+      const StatArgs st =
+          stat(c, sizeof(T) == 8 ? KS_K_SPMV64 : KS_K_SPMV32, spmv_bytes<T>(n, A.nnz) + 2.0 * sizeof(T) * n);
       auto go = [&](auto kernel) {
-        kernel<<<coop_grid(c, n), kCoopThreads, 0, c->stream>>>(n, A.ptr, A.col, A.val, src, x, r.p, ld,
-                                                             sizeof(T) == 8 ? nullptr : xout, ctl(), coop_args(c, outer_stop), mode,
-                                                             u + 1 == max_units(), iters,
-                                                             mode == 1 ? gouter() : gstep(), st);
+        kernel<<<coop_grid(c, n), kCoopThreads, 0, c->stream>>>(
+            n, A.ptr, A.col, A.val, src, x, r.p, ld, sizeof(T) == 8 ? nullptr : xout, ctl(), coop_args(c, outer_stop),
+            mode, u + 1 == max_units(), iters, mode == 1 ? gouter() : gstep(), st);
       };
       switch (coop_rows(c, n)) {
         case 1: go(k_cg_coop<T, kCoopThreads, 1>); break;
@@ -847,7 +847,8 @@ struct BicgLevel : Level {
       const int mode = u > 0 ? 0 : x0given ? 2 : 1;
       const int iters = (int)std::min<int64_t>(kCoopIters, cfg.maxloop - u * kCoopIters);
       // a launch reads both CSRs, x, r, r*, p and p* and writes x
-      const StatArgs st = stat(c, sizeof(T) == 8 ? KS_K_SPMV64 : KS_K_SPMV32, 2 * spmv_bytes<T>(n, A.nnz) + 2.0 * sizeof(T) * n);
+      const StatArgs st =
+          stat(c, sizeof(T) == 8 ? KS_K_SPMV64 : KS_K_SPMV32, 2 * spmv_bytes<T>(n, A.nnz) + 2.0 * sizeof(T) * n);
       auto go = [&](auto kernel) {
         kernel<<<coop_grid(c, n), kCoopThreads, 0, c->stream>>>(
             n, A.ptr, A.col, A.val, AT.ptr, AT.col, AT.val, src, x, vec.p, pad64(n), sizeof(T) == 8 ? nullptr : xout,

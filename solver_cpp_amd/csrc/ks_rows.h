@@ -83,7 +83,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
   // NK >= most entries gathered per row; places past a row's end hold offset 0
   auto sweep = [&](auto nk) {
     constexpr int NK = decltype(nk)::value;
-    auto at = [](const T* x, uint32_t byte) { return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(x) + byte); };
+    auto at = [](const T* x, uint32_t byte) {
+      return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(x) + byte);
+    };
     for (int slot = 0; t < end; t += B * step, slot += B) {
       T g0[B][NK], g1[B][NK];
       int32_t row[B], cls[B];
